@@ -248,9 +248,7 @@ int mcfd_batch_set_solution_column(mcfd_batch *b, int32_t c, const double *colum
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
     const auto &ref = b->cases[c];
-    const auto &g = *b->groups[ref.group];
-    Check(hipMemcpyAsync(g.u0.ptr + ref.first_cell * g.np * 5, column, ref.n_cells * g.np * 5 * sizeof(double),
-                         hipMemcpyHostToDevice, b->stream), "set solution");
+    b->groups[ref.group]->SetColumn(column, ref.first_cell, ref.n_cells, b->stream);
     Check(hipStreamSynchronize(b->stream), "sync");
   });
 }
@@ -260,9 +258,7 @@ int mcfd_batch_get_solution_column(mcfd_batch *b, int32_t c, double *column) {
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
     const auto &ref = b->cases[c];
-    const auto &g = *b->groups[ref.group];
-    Check(hipMemcpyAsync(column, g.u0.ptr + ref.first_cell * g.np * 5, ref.n_cells * g.np * 5 * sizeof(double),
-                         hipMemcpyDeviceToHost, b->stream), "get solution");
+    b->groups[ref.group]->GetColumn(column, ref.first_cell, ref.n_cells, b->stream);
     Check(hipStreamSynchronize(b->stream), "sync");
   });
 }

@@ -50,15 +50,66 @@ void FacePointLocal(int f, const double *x1d, int a, int b, double *s) {
   else { s[1] = x1d[a]; s[2] = x1d[b]; }
 }
 
+// The packed word of FrFace::gather: the neighbour's node behind in-face point
+// (a, b) of this cell, m nodes in from the face, is first + sa a + sb b + sm m.
+int32_t GatherWord(int q, int orient, int nf) {
+  auto node = [&](int a, int b, int m) {
+    int a2, b2;
+    ApplyOrient(orient, q, a, b, &a2, &b2);
+    return HexLineNode(q, nf, a2, b2, kHexFaceSide[nf] ? q - 1 - m : m);
+  };
+  const int first = node(0, 0, 0);
+  const int step[3] = { node(1, 0, 0) - first, node(0, 1, 0) - first, node(0, 0, 1) - first };
+  return (int32_t)((uint32_t)(uint8_t)first | (uint32_t)(uint8_t)step[0] << 8 | (uint32_t)(uint8_t)step[1] << 16 |
+                   (uint32_t)(uint8_t)step[2] << 24);
+}
+
+// Which of a face's two cells holds the left state (FrFace): +1 where its
+// stored normal (from the holder outwards) points left to right, else -1.
+bool HolderIsLeft(const HexFace &face, bool exact) {
+  const bool holder_upper = kHexFaceSide[face.holder_face] != 0;
+  if (exact) return true;
+  if (face.sharer >= 0 && (kHexFaceSide[face.sharer_face] != 0) == holder_upper) return true;
+  return holder_upper;
+}
+
 }  // namespace
+
+// The cells' face records; normal_of(face index, sign) is the index of the
+// face's normal times sign.
+template <class NormalOf>
+void FrHexGroup::BuildFaceRecords(NormalOf &&normal_of) {
+  h_faces.assign(6 * n_cells, FrFace{ INT32_MIN, 0, 0, -1 });
+  any_swap = false;
+  auto put = [&](int64_t cell, int local, int32_t nbr, int32_t gather, int32_t normal, bool left, int32_t bface) {
+    const bool swap = left != (kHexFaceSide[local] != 0);
+    any_swap = any_swap || swap;
+    h_faces[cell * 6 + local] = FrFace{ nbr, gather, normal << 1 | (swap ? 1 : 0), bface };
+  };
+  for (size_t f = 0; f < conn.faces.size(); ++f) {
+    const auto &face = conn.faces[f];
+    const bool left = HolderIsLeft(face, riemann == MCFD_RIEMANN_EXACT);
+    const int32_t normal = normal_of(f, left ? 1.0 : -1.0);
+    if (normal >= (1 << 24)) throw Failure{ MCFD_ENOTSUP, "too many distinct face normals" };
+    if (face.sharer >= 0) {
+      put(face.holder, face.holder_face, (int32_t)face.sharer, GatherWord(q, face.orient, face.sharer_face), normal,
+          left, -1);
+      put(face.sharer, face.sharer_face, (int32_t)face.holder,
+          GatherWord(q, InverseOrient(face.orient), face.holder_face), normal, !left, -1);
+    } else {
+      put(face.holder, face.holder_face, -(1 + face.tag), 0, normal, left, (int32_t)(f - conn.n_interior));
+    }
+  }
+  for (const auto &v : h_faces)
+    if (v.nbr == INT32_MIN) throw std::invalid_argument("cell face without a face record");
+}
 
 // Geometry of a mesh with trilinear cells (polynomial/hexahedron.hpp:172-239
 // keeps J* and det(J) per node; fr/general.hpp:103-205 the flux point's
 // J* column; the face integrator the frame of each face point):
-//   geo_node [cell][node]  J* (9), 1 / det(J) at the node;
-//   fscale [cell][face][a * Q + b]  +-|J*.col(normal dir)| at the flux point;
-//   frames [face][a * Q + b]  n, t of the face map at the point, indexed by the
-//     holder's in-face (a, b);
+//   col_node [cell][r][node]  J*.col(r) at the node; inv_det_node [cell][node];
+//   face_point [cell][face][a * Q + b]  the unit normal of the face map at the
+//     point, left to right, and |J*.col(normal dir)| of this cell there;
 //   geo [cell]  only the length cbrt(volume) / 2, volume = sum of w det(J).
 void FrHexGroup::BuildCurved(const mcfd_scheme_desc &) {
   const int64_t nc = n_cells;
@@ -66,8 +117,9 @@ void FrHexGroup::BuildCurved(const mcfd_scheme_desc &) {
   diag_metric = false;
   h_geo.assign(nc * kGeoStride, 0.0);
   h_geo_id.resize(nc);
-  h_geo_node.assign(nc * np * kNodeGeoStride, 0.0);
-  h_fscale.assign(nc * 6 * nfp, 0.0);
+  h_col_node.assign(nc * np * 9, 0.0);
+  h_inv_det.assign(nc * np, 0.0);
+  h_face_point.assign(nc * 6 * nfp * 4, 0.0);
   corner0.resize(nc);
   for (int64_t c = 0; c < nc; ++c) {
     const double *xv = conn.vertices[c].data();
@@ -76,15 +128,17 @@ void FrHexGroup::BuildCurved(const mcfd_scheme_desc &) {
       for (int jj = 0; jj < q; ++jj)
         for (int k = 0; k < q; ++k) {
           const double s[3] = { x1d[i], x1d[jj], x1d[k] };
-          double jac[9];
+          double jac[9], g[9];
           TrilinearJacobian(xv, s, jac);
-          double *g = h_geo_node.data() + (c * np + (i * q + jj) * q + k) * kNodeGeoStride;
+          const int node = (i * q + jj) * q + k;
           const double det = Adjugate(jac, g);
           if (!(det > 0)) throw std::invalid_argument("inverted trilinear hexahedron");
-          g[9] = 1.0 / det;
+          for (int r = 0; r < 3; ++r)
+            for (int e = 0; e < 3; ++e) h_col_node[((c * 3 + r) * np + node) * 3 + e] = g[3 * e + r];
+          h_inv_det[c * np + node] = 1.0 / det;
           volume += w1d[i] * w1d[jj] * w1d[k] * det;
         }
-    h_geo[c * kGeoStride + 16] = std::cbrt(volume) * 0.5;  // mesh/part.hpp:230
+    h_geo[c * kGeoStride + kGeoLength] = std::cbrt(volume) * 0.5;  // mesh/part.hpp:230
     h_geo_id[c] = (int32_t)c;
     for (int f = 0; f < 6; ++f) {
       const int dir = kHexFaceNormalDir[f];
@@ -95,42 +149,31 @@ void FrHexGroup::BuildCurved(const mcfd_scheme_desc &) {
           TrilinearJacobian(xv, s, jac);
           Adjugate(jac, g);
           const double n = std::sqrt(g[dir] * g[dir] + g[3 + dir] * g[3 + dir] + g[6 + dir] * g[6 + dir]);
-          h_fscale[(c * 6 + f) * nfp + a * q + b] = kHexFaceSide[f] ? n : -n;
+          h_face_point[((c * 6 + f) * nfp + a * q + b) * 4 + 3] = n;
         }
     }
     corner0[c] = { xv[0], xv[1], xv[2] };
   }
   if ((int64_t)conn.faces.size() >= (int64_t(1) << 24))
-    throw Failure{ MCFD_ENOTSUP, "too many faces for the per-point frames of a trilinear mesh" };
-  h_frames.assign(conn.faces.size() * nfp * kFrameStride, 0.0);
-  h_nbr.assign(6 * nc, INT32_MIN);
-  h_finfo.assign(6 * nc, 0);
-  for (size_t fi = 0; fi < conn.faces.size(); ++fi) {
+    throw Failure{ MCFD_ENOTSUP, "too many faces for the per-point normals of a trilinear mesh" };
+  BuildFaceRecords([&](size_t fi, double sign) {
     const auto &face = conn.faces[fi];
     for (int i = 0; i < q; ++i)
       for (int j = 0; j < q; ++j) {
         int a, b;
         ApplyOrient(face.quad_to_holder, q, i, j, &a, &b);
-        FaceFrameAt(face.corners, x1d[i], x1d[j], h_frames.data() + (fi * nfp + a * q + b) * kFrameStride);
+        double frame[6];
+        FaceFrameAt(face.corners, x1d[i], x1d[j], frame);
+        double *h = h_face_point.data() + ((face.holder * 6 + face.holder_face) * nfp + a * q + b) * 4;
+        for (int d = 0; d < 3; ++d) h[d] = sign * frame[d];
+        if (face.sharer < 0) continue;
+        int a2, b2;
+        ApplyOrient(face.orient, q, a, b, &a2, &b2);
+        double *s = h_face_point.data() + ((face.sharer * 6 + face.sharer_face) * nfp + a2 * q + b2) * 4;
+        for (int d = 0; d < 3; ++d) s[d] = sign * frame[d];
       }
-    const int32_t fid = (int32_t)fi;
-    const int64_t hs = face.holder * 6 + face.holder_face;
-    if (face.sharer >= 0) {
-      const int64_t ss = face.sharer * 6 + face.sharer_face;
-      h_nbr[hs] = (int32_t)face.sharer;
-      h_finfo[hs] = (fid << 7) | (1 << 6) | (face.orient << 3) | face.sharer_face;
-      h_nbr[ss] = (int32_t)face.holder;
-      h_finfo[ss] = (fid << 7) | (InverseOrient(face.orient) << 3) | face.holder_face;
-    } else {
-      h_nbr[hs] = -(1 + face.tag);
-      h_finfo[hs] = (fid << 7) | (1 << 6);
-    }
-  }
-  for (auto v : h_nbr)
-    if (v == INT32_MIN) throw std::invalid_argument("cell face without a face record");
-  h_bface_of.assign(6 * nc, -1);
-  for (size_t f = conn.n_interior; f < conn.faces.size(); ++f)
-    h_bface_of[conn.faces[f].holder * 6 + conn.faces[f].holder_face] = (int32_t)(f - conn.n_interior);
+    return 0;
+  });
 }
 
 void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &scheme,
@@ -158,18 +201,42 @@ void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &schem
   }
   conn = BuildHexConnectivity(mesh);
 
-  // line tables
+  // line tables; the points are symmetric about 0, and the kernels rely on the
+  // tables being so to the last bit
   x1d.resize(q);
   w1d.resize(q);
   GaussRule(scheme.nodes == MCFD_NODES_LOBATTO, q, x1d.data(), w1d.data());
   std::memset(&lt, 0, sizeof(lt));
-  for (int i = 0; i < q; ++i)
-    for (int m = 0; m < q; ++m) lt.d[i][m] = LagrangeDerivative(q, x1d.data(), m, x1d[i]);
+  double dg[kMaxQ][kMaxQ];
   for (int m = 0; m < q; ++m) {
-    lt.lend[0][m] = LagrangeValue(q, x1d.data(), m, -1.0);
-    lt.lend[1][m] = LagrangeValue(q, x1d.data(), m, +1.0);
+    lt.end[m] = LagrangeValue(q, x1d.data(), m, -1.0);
+    lt.lend[0][m] = (float)LagrangeValue(q, x1d.data(), m, -1.0);
+    lt.lend[1][m] = (float)LagrangeValue(q, x1d.data(), m, +1.0);
     lt.gp[0][m] = CorrectionLeftDerivative(degree, scheme.c_next, x1d[m]);
     lt.gp[1][m] = CorrectionRightDerivative(degree, scheme.c_next, x1d[m]);
+  }
+  for (int i = 0; i < q; ++i)
+    for (int m = 0; m < q; ++m) {
+      const double d = LagrangeDerivative(q, x1d.data(), m, x1d[i]);
+      lt.d[i][m] = (float)d;
+      dg[i][m] = d - lt.gp[0][i] * lt.end[m] - lt.gp[1][i] * lt.end[q - 1 - m];
+    }
+  for (int i = 0; i < q; ++i)
+    for (int m = 0; m < q; ++m) lt.dg[i][m] = 0.5 * (dg[i][m] - dg[q - 1 - i][q - 1 - m]);
+
+  h_ops.clear();
+  if (q == 4) {
+    CellOps o{};
+    for (int lane = 0; lane < 64; ++lane) {
+      const int h = lane >> 4, l = lane & 3;
+      o.dg[lane] = lt.dg[l][h];
+      const double end = (l & 1) ? lt.end[3 - h] : lt.end[h], gp = lt.gp[h & 1][l];
+      o.end01[lane] = l < 2 ? end : 0.0;
+      o.end23[lane] = l < 2 ? 0.0 : end;
+      o.gp01[lane] = h < 2 ? gp : 0.0;
+      o.gp23[lane] = h < 2 ? 0.0 : gp;
+    }
+    h_ops.push_back(o);
   }
 
   const int64_t nc = mesh.n_cells;
@@ -191,17 +258,15 @@ void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &schem
     const auto &j = conn.jac[c];
     double d = conn.det[c];
     // J* = det(J) J^{-1} is the adjugate of J
+    double js[9];
+    Adjugate(j.data(), js);
     std::array<double, kGeoStride> g{};
-    g[0] = j[4] * j[8] - j[5] * j[7]; g[1] = j[2] * j[7] - j[1] * j[8]; g[2] = j[1] * j[5] - j[2] * j[4];
-    g[3] = j[5] * j[6] - j[3] * j[8]; g[4] = j[0] * j[8] - j[2] * j[6]; g[5] = j[2] * j[3] - j[0] * j[5];
-    g[6] = j[3] * j[7] - j[4] * j[6]; g[7] = j[1] * j[6] - j[0] * j[7]; g[8] = j[0] * j[4] - j[1] * j[3];
-    g[9] = 1.0 / d;
-    for (int f = 0; f < 6; ++f) {
-      int dir = kHexFaceNormalDir[f];
-      double n = std::sqrt(g[dir] * g[dir] + g[3 + dir] * g[3 + dir] + g[6 + dir] * g[6 + dir]);
-      g[10 + f] = kHexFaceSide[f] ? n : -n;
+    for (int r = 0; r < 3; ++r) {
+      for (int e = 0; e < 3; ++e) g[4 * r + e] = js[3 * e + r];
+      g[4 * r + 3] = std::sqrt(js[r] * js[r] + js[3 + r] * js[3 + r] + js[6 + r] * js[6 + r]);
     }
-    g[16] = std::cbrt(8 * d) * 0.5;  // mesh/part.hpp:230, volume = 8 det(J)
+    g[kGeoInvDet] = 1.0 / d;
+    g[kGeoLength] = std::cbrt(8 * d) * 0.5;  // mesh/part.hpp:230, volume = 8 det(J)
     auto it = geo_ids.find(g);
     if (it == geo_ids.end()) {
       it = geo_ids.emplace(g, (int32_t)geo_ids.size()).first;
@@ -212,42 +277,24 @@ void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &schem
     corner0[c] = { mesh.coords[3 * n0], mesh.coords[3 * n0 + 1], mesh.coords[3 * n0 + 2] };
   }
   diag_metric = true;
-  for (size_t r = 0; r < h_geo.size(); r += kGeoStride)
-    for (int e = 0; e < 9; ++e)
-      if (e % 4 != 0 && h_geo[r + e] != 0.0) diag_metric = false;
+  for (size_t rec = 0; rec < h_geo.size(); rec += kGeoStride)
+    for (int r = 0; r < 3; ++r)
+      for (int e = 0; e < 3; ++e)
+        if (e != r && h_geo[rec + 4 * r + e] != 0.0) diag_metric = false;
 
-  // per-cell face records
-  std::map<std::array<double, kFrameStride>, int32_t> frame_ids;
-  h_frames.clear();
-  h_nbr.assign(6 * nc, INT32_MIN);
-  h_finfo.assign(6 * nc, 0);
-  for (const auto &face : conn.faces) {
-    std::array<double, kFrameStride> fr;
-    std::copy(face.frame, face.frame + 6, fr.begin());
-    auto it = frame_ids.find(fr);
-    if (it == frame_ids.end()) {
-      it = frame_ids.emplace(fr, (int32_t)frame_ids.size()).first;
-      h_frames.insert(h_frames.end(), fr.begin(), fr.end());
+  // per-cell face records, normals deduplicated bitwise
+  std::map<std::array<double, 3>, int32_t> normal_ids;
+  h_normals.clear();
+  BuildFaceRecords([&](size_t f, double sign) {
+    const double *fr = conn.faces[f].frame;
+    const std::array<double, 3> n{ sign * fr[0], sign * fr[1], sign * fr[2] };
+    auto it = normal_ids.find(n);
+    if (it == normal_ids.end()) {
+      it = normal_ids.emplace(n, (int32_t)normal_ids.size()).first;
+      h_normals.insert(h_normals.end(), { n[0], n[1], n[2], 0.0 });
     }
-    int32_t fid = it->second;
-    if (fid >= (1 << 24)) throw Failure{ MCFD_ENOTSUP, "too many distinct face frames" };
-    int64_t hs = face.holder * 6 + face.holder_face;
-    if (face.sharer >= 0) {
-      int64_t ss = face.sharer * 6 + face.sharer_face;
-      h_nbr[hs] = (int32_t)face.sharer;
-      h_finfo[hs] = (fid << 7) | (1 << 6) | (face.orient << 3) | face.sharer_face;
-      h_nbr[ss] = (int32_t)face.holder;
-      h_finfo[ss] = (fid << 7) | (InverseOrient(face.orient) << 3) | face.holder_face;
-    } else {
-      h_nbr[hs] = -(1 + face.tag);
-      h_finfo[hs] = (fid << 7) | (1 << 6);
-    }
-  }
-  for (auto v : h_nbr)
-    if (v == INT32_MIN) throw std::invalid_argument("cell face without a face record");
-  h_bface_of.assign(6 * nc, -1);
-  for (size_t f = conn.n_interior; f < conn.faces.size(); ++f)
-    h_bface_of[conn.faces[f].holder * 6 + conn.faces[f].holder_face] = (int32_t)(f - conn.n_interior);
+    return it->second;
+  });
 }
 
 void FrHexGroup::BoundaryPoints(std::vector<int32_t> *tags, std::vector<double> *xyz) const {
@@ -284,20 +331,20 @@ void FrHexGroup::Upload(hipStream_t stream) {
   size_t cs = ColumnSize();
   u0.Allocate(cs); u1.Allocate(cs); u2.Allocate(cs); res.Allocate(cs);
   Check(hipMemsetAsync(u0.ptr, 0, cs * sizeof(double), stream), "memset");
-  nbr.Upload(h_nbr, stream);
-  finfo.Upload(h_finfo, stream);
+  faces.Upload(h_faces, stream);
   geo_id.Upload(h_geo_id, stream);
   geo.Upload(h_geo, stream);
-  frames.Upload(h_frames, stream);
+  normals.Upload(h_normals, stream);
+  ops.Upload(h_ops, stream);
   if (curved) {
-    geo_node.Upload(h_geo_node, stream);
-    fscale.Upload(h_fscale, stream);
+    col_node.Upload(h_col_node, stream);
+    inv_det.Upload(h_inv_det, stream);
+    face_point.Upload(h_face_point, stream);
   }
   bc_kind.Upload(h_bc_kind, stream);
   bc_state.Upload(h_bc_state, stream);
   if (!h_cell_case.empty()) cell_case.Upload(h_cell_case, stream);
   if (!h_tile_order.empty()) tile_order.Upload(h_tile_order, stream);
-  bface_of.Upload(h_bface_of, stream);
   if (riemann == MCFD_RIEMANN_EXACT) {
     const size_t n_star = size_t(n_cells) * 6 * q * q;
     exact_star.Allocate(n_star);
@@ -342,11 +389,24 @@ void FrHexGroup::BuildTileOrder(int tile_cells) {
   for (int64_t t = 0; t < n_tiles; ++t) h_tile_order[t] = key[t].second;
 }
 
+void FrHexGroup::SetColumn(const double *column, int64_t first_cell, int64_t count, hipStream_t stream) {
+  const size_t at = size_t(first_cell) * np * 5, n = size_t(count) * np * 5;
+  Check(hipMemcpyAsync(res.ptr + at, column, n * sizeof(double), hipMemcpyHostToDevice, stream), "set solution");
+  Check(LaunchFrLayout(true, res.ptr + at, u0.ptr + at, np, count, stream), "set solution layout");
+}
+
+void FrHexGroup::GetColumn(double *column, int64_t first_cell, int64_t count, hipStream_t stream) {
+  const size_t at = size_t(first_cell) * np * 5, n = size_t(count) * np * 5;
+  Check(LaunchFrLayout(false, u0.ptr + at, res.ptr + at, np, count, stream), "get solution layout");
+  Check(hipMemcpyAsync(column, res.ptr + at, n * sizeof(double), hipMemcpyDeviceToHost, stream), "get solution");
+}
+
 FrHexArgs FrHexGroup::Args(int stage, double dt) const {
   FrHexArgs a;
   a.u0 = u0.ptr;
-  a.nbr = nbr.ptr; a.finfo = finfo.ptr; a.geo_id = geo_id.ptr;
-  a.geo = geo.ptr; a.frames = frames.ptr;
+  a.cell_ops = ops.ptr;
+  a.faces = faces.ptr; a.geo_id = geo_id.ptr;
+  a.geo = geo.ptr; a.normals = normals.ptr;
   a.bc_kind = bc_kind.ptr; a.bc_state = bc_state.ptr;
   a.cell_case = cell_case.ptr;
   a.case_dt = cell_case.ptr ? case_dt.ptr : nullptr;
@@ -358,12 +418,12 @@ FrHexArgs FrHexGroup::Args(int stage, double dt) const {
   a.dt_min_bits = nullptr;
   a.exact_star = exact_star.ptr;
   a.bc_point_state = nullptr;  // set by the caller when boundary functions are in use
-  a.bface_of = bface_of.ptr;
-  a.diag_metric = diag_metric ? 1 : 0;
+  a.any_swap = any_swap ? 1 : 0;
   a.mixed = mixed ? 1 : 0;
   a.curved = curved ? 1 : 0;
-  a.geo_node = geo_node.ptr;
-  a.fscale = fscale.ptr;
+  a.col_node = col_node.ptr;
+  a.inv_det_node = inv_det.ptr;
+  a.face_point = face_point.ptr;
   switch (stage) {
   case 0: a.us = u0.ptr; a.out = res.ptr; break;
   case 1: a.us = u0.ptr; a.out = u1.ptr; break;

@@ -20,33 +20,36 @@ namespace mcfd {
 
 struct FrHexGroup {
   int q = 0, np = 0, degree = 0, riemann = 0;
-  bool mixed = false, diag_metric = false, curved = false;
+  bool mixed = false, diag_metric = false, curved = false, any_swap = false;
   int64_t n_cells = 0;
   HexConnectivity conn;
   LineTables lt;
   std::vector<double> x1d, w1d;  // 1-D solution points and their quadrature weights
   std::vector<std::array<double, 3>> corner0;  // node 0 of each cell
   // host copies uploaded by Upload()
-  std::vector<int32_t> h_nbr, h_finfo, h_geo_id, h_bc_kind, h_cell_case, h_tile_order;
-  std::vector<double> h_geo, h_frames, h_bc_state;
-  // curved meshes: [cell][node][kNodeGeoStride] and [cell][6][Q * Q]
-  std::vector<double> h_geo_node, h_fscale;
-  DeviceArray<double> geo_node, fscale;
-  DeviceArray<double> u0, u1, u2, res;
-  DeviceArray<int32_t> nbr, finfo, geo_id, bc_kind, cell_case, tile_order;
-  DeviceArray<double> geo, frames, bc_state, case_dt;
+  std::vector<FrFace> h_faces;
+  std::vector<CellOps> h_ops;  // one entry at Q = 4
+  std::vector<int32_t> h_geo_id, h_bc_kind, h_cell_case, h_tile_order;
+  std::vector<double> h_geo, h_normals, h_bc_state;
+  // curved meshes: J* columns [cell][r][node][3], 1 / det(J) [cell][node], and
+  // flux-point normals and scales [cell][6][Q * Q][4]
+  std::vector<double> h_col_node, h_inv_det, h_face_point;
+  DeviceArray<double> col_node, inv_det, face_point;
+  DeviceArray<double> u0, u1, u2;  // states in planes (FrHexArgs)
+  DeviceArray<double> res;         // residual column, and staging of columns in and out
+  DeviceArray<FrFace> faces;
+  DeviceArray<CellOps> ops;
+  DeviceArray<int32_t> geo_id, bc_kind, cell_case, tile_order;
+  DeviceArray<double> geo, normals, bc_state, case_dt;
   // exact solver: per (cell, local face, flux point) state of its solver
   // object, the sign of the last star velocity (zero at creation)
   DeviceArray<uint8_t> exact_star;
-  // boundary face index of each boundary cell face, [cell][6] (-1 elsewhere),
-  // for the per-point boundary values of BoundaryTable
-  std::vector<int32_t> h_bface_of;
-  DeviceArray<int32_t> bface_of;
 
   // Host-side construction; bc_kind/bc_state index the mesh's boundary tags.
   void Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &scheme,
              const std::vector<int32_t> &bc_kinds, const std::vector<double> &bc_states);
   void BuildCurved(const mcfd_scheme_desc &scheme);
+  template <class NormalOf> void BuildFaceRecords(NormalOf &&normal_of);
   // Order in which the stage kernel sweeps its tiles of `tile_cells`
   // consecutive cells: Morton order of the tile centres, so that the tiles in
   // flight on one XCD are spatial neighbours and their face-trace gathers hit
@@ -56,6 +59,10 @@ struct FrHexGroup {
   void Upload(hipStream_t stream);
 
   size_t ColumnSize() const { return size_t(n_cells) * np * 5; }
+  // The solution u0 of `count` cells from or to a host column (staged in `res`;
+  // not synchronised).
+  void SetColumn(const double *column, int64_t first_cell, int64_t count, hipStream_t stream);
+  void GetColumn(double *column, int64_t first_cell, int64_t count, hipStream_t stream);
   // Kernel arguments of one pass: stage 0 residual, 1..3 SSP-RK3 stages.
   FrHexArgs Args(int stage, double dt) const;
   void SamplePoints(double *xyz) const;

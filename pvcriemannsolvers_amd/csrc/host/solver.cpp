@@ -67,8 +67,18 @@ struct mcfd_solver {
     }
     if (fuse_dt) dt_fresh = dt_pending = true;
   }
+  // The solution from or to a host column (not synchronised).
+  void SetColumn(const double *column) {
+    if (dg) Check(hipMemcpyAsync(modal.u0.ptr, column, ColumnSize() * sizeof(double), hipMemcpyHostToDevice, stream),
+                  "set solution");
+    else group.SetColumn(column, 0, group.n_cells, stream);
+  }
+  void GetColumn(double *column) {
+    if (dg) Check(hipMemcpyAsync(column, modal.u0.ptr, ColumnSize() * sizeof(double), hipMemcpyDeviceToHost, stream),
+                  "get solution");
+    else group.GetColumn(column, 0, group.n_cells, stream);
+  }
   size_t ColumnSize() const { return dg ? modal.ColumnSize() : group.ColumnSize(); }
-  double *Solution() { return dg ? modal.u0.ptr : group.u0.ptr; }
   double *Residual() { return dg ? modal.res.ptr : group.res.ptr; }
 };
 
@@ -163,8 +173,7 @@ int mcfd_set_solution_column(mcfd_solver *h, const double *column) {
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
     h->dt_fresh = false;
-    Check(hipMemcpyAsync(h->Solution(), column, h->ColumnSize() * sizeof(double),
-                         hipMemcpyHostToDevice, h->stream), "set solution");
+    h->SetColumn(column);
     if (h->dg) h->modal.SolutionChanged(h->stream);
     Check(hipStreamSynchronize(h->stream), "set solution sync");
   });
@@ -175,8 +184,7 @@ int mcfd_restore_solution_column(mcfd_solver *h, const double *column) {
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
     h->dt_fresh = false;
-    Check(hipMemcpyAsync(h->Solution(), column, h->ColumnSize() * sizeof(double),
-                         hipMemcpyHostToDevice, h->stream), "restore solution");
+    h->SetColumn(column);
     if (h->dg) h->modal.SolutionChanged(h->stream, /*limit=*/false);
     Check(hipStreamSynchronize(h->stream), "restore solution sync");
   });
@@ -186,8 +194,7 @@ int mcfd_get_solution_column(mcfd_solver *h, double *column) {
   MCFD_REQUIRE_DEVICE(h);
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
-    Check(hipMemcpyAsync(column, h->Solution(), h->ColumnSize() * sizeof(double),
-                         hipMemcpyDeviceToHost, h->stream), "get solution");
+    h->GetColumn(column);
     Check(hipStreamSynchronize(h->stream), "get solution sync");
   });
 }
@@ -268,8 +275,7 @@ int mcfd_evaluate(mcfd_solver *h, const double *column, int32_t n_local, const d
     std::vector<double> own;
     if (values && !column) {
       own.resize(h->ColumnSize());
-      Check(hipMemcpyAsync(own.data(), h->Solution(), own.size() * sizeof(double), hipMemcpyDeviceToHost,
-                           h->stream), "get solution");
+      h->GetColumn(own.data());
       Check(hipStreamSynchronize(h->stream), "get solution sync");
       column = own.data();
     }

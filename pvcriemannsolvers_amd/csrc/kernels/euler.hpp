@@ -1,7 +1,7 @@
 // Device-only Euler helpers of the stage kernels (FP64), on top of the
-// portable physics of mini/riemann/euler_core.hpp: the reciprocal-refined
-// primitive recovery and Roe flux of the FR kernels, and the face flux as the
-// FR kernels evaluate it.
+// portable physics of mini/riemann/euler_core.hpp: refined reciprocals and
+// square roots, and the face fluxes in vector form as the FR kernels evaluate
+// them.
 #ifndef MINICFD_KERNELS_EULER_HPP_
 #define MINICFD_KERNELS_EULER_HPP_
 
@@ -24,96 +24,223 @@ __device__ __forceinline__ double FastRcp(double x) {
   return __fma_rn(r, e, r);
 }
 
-// Conservative -> primitive with the reference's zeroing rule
-// (types.hpp:195-202,289-301) via one reciprocal of rho.  The plain
-// arithmetic is done first; the rule only selects among its results, so
-// a wavefront where no lane needs the rule (rho > 0, E >= 0, p >= 0 on every
-// lane) skips the selects and gets bitwise the same values as one that
-// applies them.  *inv_rho receives FastRcp of the returned density.
-__device__ __forceinline__ State FastPrimitive(State const &c, double *inv_rho) {
-  const double rho = c.v[0];
-  const double inv = FastRcp(rho);
-  State p;
-  p.v[0] = rho;
-  p.v[1] = c.v[1] * inv;
-  p.v[2] = c.v[2] * inv;
-  p.v[3] = c.v[3] * inv;
-  const double ke = 0.5 * (p.v[1] * p.v[1] + p.v[2] * p.v[2] + p.v[3] * p.v[3]);
-  p.v[4] = (c.v[4] - rho * ke) * kGm1;
-  *inv_rho = inv;
-  if (__all(rho > 0 && c.v[4] >= 0 && p.v[4] >= 0)) return p;
-  // rho < 0 or E < 0: all zero; rho == 0: momenta and E kept as they are;
-  // otherwise p < 0: all zero
+// sqrt by v_rsq_f64 and two fused corrections: within 1 ulp for normal x,
+// 0 for 0, NaN for x < 0.  The compiler's correctly rounded sqrt adds range
+// scaling and class checks, about twice the instructions.
+__device__ __forceinline__ double FastSqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __fma_rn(-h, g, 0.5);
+  g = __fma_rn(g, r, g);
+  h = __fma_rn(h, r, h);
+  g = __fma_rn(__fma_rn(-g, g, x), h, g);
+  return x == 0 ? 0.0 : g;
+}
+
+// x / 3, correctly rounded: the quotient by the rounded reciprocal is at most
+// one unit off, and the fused remainder puts it right (Markstein's division
+// for a constant divisor), in 3 instructions instead of the divide's 10.
+__device__ __forceinline__ double ThirdOf(double x) {
+  const double q = x * (1.0 / 3.0);
+  return __fma_rn(__fma_rn(-3.0, q, x), 1.0 / 3.0, q);
+}
+
+// One trace of a face with what the fluxes need of it: density and its
+// reciprocal, velocity, pressure, total energy, and the velocity along the
+// unit normal.  The reference rotates both traces into the face
+// frame, solves there and rotates the flux back (rotated/euler.hpp:117-159);
+// the solvers only need the normal velocity, so the fluxes below keep the
+// vectors in global coordinates: no tangents, two dot products instead of
+// three rotations.
+struct FaceTrace { double rho, inv, v[3], p, e, un; };
+
+// The trace's plain arithmetic (types.hpp:289-301, one reciprocal); *plain is
+// cleared where the zeroing rule (ApplyZeroRule) changes the result.
+__device__ __forceinline__ FaceTrace PlainTrace(State const &c, const double *n, bool *plain) {
+  FaceTrace t;
+  t.rho = c.v[0];
+  t.inv = FastRcp(t.rho);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) t.v[d] = c.v[1 + d] * t.inv;
+  t.e = c.v[4];
+  const double rk = c.v[1] * t.v[0] + c.v[2] * t.v[1] + c.v[3] * t.v[2];  // 2 rho k
+  t.p = (t.e - 0.5 * rk) * kGm1;
+  t.un = t.v[0] * n[0] + t.v[1] * n[1] + t.v[2] * n[2];
+  *plain = *plain && t.rho > 0 && t.e >= 0 && t.p >= 0;
+  return t;
+}
+// types.hpp:195-202: all zero where rho < 0, E < 0 or p < 0; momenta and E kept
+// as velocity and pressure where rho == 0.
+__device__ __forceinline__ void ApplyZeroRule(State const &c, const double *n, FaceTrace *t) {
   const bool bad = c.v[0] < 0 || c.v[4] < 0;
   const bool vacuum = !bad && c.v[0] == 0;
-  const bool zero = bad || (!vacuum && p.v[4] < 0);
+  const bool zero = bad || (!vacuum && t->p < 0);
 #pragma unroll
-  for (int k = 1; k < 5; ++k) p.v[k] = zero ? 0.0 : (vacuum ? c.v[k] : p.v[k]);
-  p.v[0] = zero ? 0.0 : rho;  // a vacuum keeps its signed zero
-  if (zero || vacuum) *inv_rho = FastRcp(p.v[0]);
-  return p;
+  for (int d = 0; d < 3; ++d) t->v[d] = zero ? 0.0 : (vacuum ? c.v[1 + d] : t->v[d]);
+  t->p = zero ? 0.0 : (vacuum ? c.v[4] : t->p);
+  t->e = zero ? 0.0 : (vacuum ? c.v[4] * (1 / kGm1) : t->e);
+  t->rho = zero ? 0.0 : t->rho;
+  if (zero || vacuum) t->inv = FastRcp(t->rho);
+  t->un = t->v[0] * n[0] + t->v[1] * n[1] + t->v[2] * n[2];
 }
-__device__ __forceinline__ State FastPrimitive(State const &c) {
-  double inv;
-  return FastPrimitive(c, &inv);
-}
-
-// Roe flux of normal-frame primitives (same waves as RoeFlux) with
-// reciprocals instead of divisions; inv_l, inv_r = FastRcp of the densities.
-__device__ __forceinline__ State FastRoeFlux(State const &l, State const &r, double inv_l, double inv_r) {
-  constexpr double kGoGm1 = kGamma / kGm1;
-  double kel = 0.5 * (l.v[1] * l.v[1] + l.v[2] * l.v[2] + l.v[3] * l.v[3]);
-  double ker = 0.5 * (r.v[1] * r.v[1] + r.v[2] * r.v[2] + r.v[3] * r.v[3]);
-  double el = l.v[4] * (1 / kGm1) + l.v[0] * kel;  // total energy per volume
-  double er = r.v[4] * (1 / kGm1) + r.v[0] * ker;
-  State flux;
-  flux.v[0] = 0.5 * (l.v[0] * l.v[1] + r.v[0] * r.v[1]);
-  flux.v[1] = 0.5 * ((l.v[0] * l.v[1]) * l.v[1] + l.v[4] + (r.v[0] * r.v[1]) * r.v[1] + r.v[4]);
-  flux.v[2] = 0.5 * ((l.v[0] * l.v[2]) * l.v[1] + (r.v[0] * r.v[2]) * r.v[1]);
-  flux.v[3] = 0.5 * ((l.v[0] * l.v[3]) * l.v[1] + (r.v[0] * r.v[3]) * r.v[1]);
-  flux.v[4] = 0.5 * ((el + l.v[4]) * l.v[1] + (er + r.v[4]) * r.v[1]);
-  double sl = sqrt(l.v[0]), sr = sqrt(r.v[0]);
-  double inv = FastRcp(sl + sr);
-  double h0l = l.v[4] * inv_l * kGoGm1 + kel;
-  double h0r = r.v[4] * inv_r * kGoGm1 + ker;
-  double rho = sl * sr;
-  double u = (sl * l.v[1] + sr * r.v[1]) * inv;
-  double v = (sl * l.v[2] + sr * r.v[2]) * inv;
-  double w = (sl * l.v[3] + sr * r.v[3]) * inv;
-  double h = (sl * h0l + sr * h0r) * inv;
-  double ke = (u * u + v * v + w * w) * 0.5;
-  double aa = kGm1 * (h - ke);
-  double a = sqrt(aa), ua = u * a, inv_aa = FastRcp(aa);
-  double dp = r.v[4] - l.v[4], du = r.v[1] - l.v[1];
-  double s1 = 0.25 * (dp - rho * a * du) * inv_aa * fabs(u - a);
-  double s2 = 0.5 * ((r.v[0] - l.v[0]) - dp * inv_aa) * fabs(u);
-  double s3 = 0.5 * (rho * (r.v[2] - l.v[2])) * fabs(u);
-  double s4 = 0.5 * (rho * (r.v[3] - l.v[3])) * fabs(u);
-  double s5 = 0.25 * (dp + rho * a * du) * inv_aa * fabs(u + a);
-  flux.v[0] -= s1 + s2 + s5;
-  flux.v[1] -= s1 * (u - a) + s2 * u + s5 * (u + a);
-  flux.v[2] -= (s1 + s2 + s5) * v + s3;
-  flux.v[3] -= (s1 + s2 + s5) * w + s4;
-  flux.v[4] -= s1 * (h - ua) + s2 * ke + s3 * v + s4 * w + s5 * (h + ua);
-  return flux;
+__device__ __forceinline__ FaceTrace TraceOf(State const &c, const double *n) {
+  bool plain = true;
+  FaceTrace t = PlainTrace(c, n, &plain);
+  if (!__all(plain)) ApplyZeroRule(c, n, &t);
+  return t;
 }
 
-// The upwind flux as the FR stage kernels evaluate it: Roe on primitives
-// recovered with one reciprocal of rho per side (FastPrimitive, FastRoeFlux),
-// the other solvers as UpwindFlux.
-template <int kRiemann>
-__device__ __forceinline__ State FaceFlux(FaceFrame const &f, State const &cl, State const &cr, bool &star) {
-  if constexpr (kRiemann == kRoe) {
-    double inv_l, inv_r;
-    State l = FastPrimitive(cl, &inv_l), r = FastPrimitive(cr, &inv_r);
-    GlobalToNormal(f, &l);
-    GlobalToNormal(f, &r);
-    State flux = FastRoeFlux(l, r, inv_l, inv_r);
-    NormalToGlobal(f, &flux);
-    return flux;
-  } else {
-    return UpwindFlux<kRiemann>(f, cl, cr, star);
+// types.hpp:313-321: physical flux of one trace through the unit normal n.
+__device__ __forceinline__ State TraceFlux(FaceTrace const &t, const double *n) {
+  State f;
+  f.v[0] = t.rho * t.un;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) f.v[1 + d] = f.v[0] * t.v[d] + t.p * n[d];
+  f.v[4] = (t.e + t.p) * t.un;
+  return f;
+}
+
+// Roe flux (the waves of RoeFlux in euler_core.hpp): sqrt(rho_r / rho_l) gives
+// both the averaging weight and the mean density, one reciprocal square root
+// the sound speed and its inverse square.
+__device__ __forceinline__ State FastRoe(FaceTrace const &l, FaceTrace const &r, const double *n) {
+  const double hl = (l.e + l.p), hr = (r.e + r.p);  // rho times total enthalpy
+  const double ratio = FastSqrt(r.rho * l.inv);
+  const double wr = ratio * FastRcp(1.0 + ratio);
+  const double rho = l.rho * ratio;
+  double dv[3], v[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    dv[d] = r.v[d] - l.v[d];
+    v[d] = l.v[d] + wr * dv[d];
   }
+  const double dun = r.un - l.un, un = l.un + wr * dun, dp = r.p - l.p;
+  const double h0l = hl * l.inv, h = h0l + wr * (hr * r.inv - h0l);
+  const double ke = 0.5 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+  const double aa = kGm1 * (h - ke);
+  const double a = FastSqrt(aa), inv_aa = FastRcp(aa);
+  const double rad = rho * a * dun;
+  const double s1 = 0.25 * (dp - rad) * inv_aa * fabs(un - a);
+  const double s5 = 0.25 * (dp + rad) * inv_aa * fabs(un + a);
+  const double s2 = 0.5 * ((r.rho - l.rho) - dp * inv_aa) * fabs(un);
+  const double t = 0.5 * rho * fabs(un);           // both shear waves
+  const double s = s1 + s2 + s5, b = (s5 - s1) * a, bn = b - t * dun;
+  State f;
+  const double ml = 0.5 * (l.rho * l.un), mr = 0.5 * (r.rho * r.un);
+  f.v[0] = ml + mr - s;
+  const double pm = 0.5 * (l.p + r.p) - bn;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) f.v[1 + d] = ml * l.v[d] + mr * r.v[d] + pm * n[d] - s * v[d] - t * dv[d];
+  const double vdv = v[0] * dv[0] + v[1] * dv[1] + v[2] * dv[2];
+  f.v[4] = 0.5 * (hl * l.un + hr * r.un) - ((s1 + s5) * h + s2 * ke + un * bn + t * vdv);
+  return f;
+}
+
+// HLLC flux (hllc.hpp:30-109): wave speeds u -+ a q from one square root each
+// (a q = sqrt(a^2 + c (p* - p) / rho) needs no division by p), the star state
+// formed once, for the side the contact selects.
+__device__ __forceinline__ State FastHllc(FaceTrace const &l, FaceTrace const &r, const double *n) {
+  const double al = l.rho > 0 && l.p > 0 ? FastSqrt(kGamma * l.p * l.inv) : 0.0;
+  const double ar = r.rho > 0 && r.p > 0 ? FastSqrt(kGamma * r.p * r.inv) : 0.0;
+  const double p_est = fmax(0.0, 0.5 * (l.p + r.p - (r.un - l.un) * (0.25 * (l.rho + r.rho) * (al + ar))));
+  const double aql = p_est > l.p ? FastSqrt((kGamma * l.p + (kGp1 / 2) * (p_est - l.p)) * l.inv) : al;
+  const double aqr = p_est > r.p ? FastSqrt((kGamma * r.p + (kGp1 / 2) * (p_est - r.p)) * r.inv) : ar;
+  const double wl = l.un - aql, wr = r.un + aqr;
+  const double ml = l.rho * (wl - l.un), mr = r.rho * (wr - r.un);
+  const double ws = (r.p - l.p + ml * l.un - mr * r.un) * FastRcp(ml - mr);
+  const bool super_l = 0.0 <= wl, super_r = !super_l && wr <= 0.0;
+  const bool left = super_l || (!super_r && 0.0 <= ws);
+  FaceTrace k;
+  k.rho = left ? l.rho : r.rho;
+  k.inv = left ? l.inv : r.inv;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) k.v[d] = left ? l.v[d] : r.v[d];
+  k.p = left ? l.p : r.p;
+  k.e = left ? l.e : r.e;
+  k.un = left ? l.un : r.un;
+  const double wk = left ? wl : wr, mk = left ? ml : mr;
+  State f = TraceFlux(k, n);
+  if (super_l || super_r) return f;
+  const double inv_ws = FastRcp(wk - ws), temp = mk * inv_ws, du = ws - k.un;
+  f.v[0] += wk * (temp - k.rho);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) f.v[1 + d] += wk * (temp * (k.v[d] + du * n[d]) - k.rho * k.v[d]);
+  f.v[4] += wk * (temp * (k.e * k.inv) + du * (temp * ws + k.p * inv_ws) - k.e);
+  return f;
+}
+
+// Exact flux (ExactFlux in euler_core.hpp) with the passive tangential velocity
+// as a vector: that of the side the contact moves away from.
+__device__ __forceinline__ State VectorExact(FaceTrace const &l, FaceTrace const &r, const double *n, bool &star) {
+  const State pl = { { l.rho, l.un, 0.0, 0.0, l.p } }, pr = { { r.rho, r.un, 0.0, 0.0, r.p } };
+  const State s = ExactState(pl, pr, star);
+  FaceTrace t;
+  t.rho = s.v[0];
+  t.un = s.v[1];
+  t.p = s.v[4];
+  const double du = t.un - (star ? l.un : r.un);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) t.v[d] = (star ? l.v[d] : r.v[d]) + du * n[d];
+  t.e = t.p * (1 / kGm1) + t.rho * (0.5 * (t.v[0] * t.v[0] + t.v[1] * t.v[1] + t.v[2] * t.v[2]));
+  return TraceFlux(t, n);
+}
+
+template <int kRiemann>
+__device__ __forceinline__ State TraceUpwind(FaceTrace const &l, FaceTrace const &r, const double *n, bool &star) {
+  if constexpr (kRiemann == kExact) return VectorExact(l, r, n, star);
+  else if constexpr (kRiemann == kHllc) return FastHllc(l, r, n);
+  else return FastRoe(l, r, n);
+}
+// The upwind flux through the unit normal n (from left to right) as the FR
+// stage kernels evaluate it.  `star` is the exact solver's per-point state.
+template <int kRiemann>
+__device__ __forceinline__ State FaceFlux(const double *n, State const &cl, State const &cr, bool &star) {
+  bool plain = true;
+  FaceTrace l = PlainTrace(cl, n, &plain), r = PlainTrace(cr, n, &plain);
+  if (!__all(plain)) {
+    ApplyZeroRule(cl, n, &l);
+    ApplyZeroRule(cr, n, &r);
+  }
+  return TraceUpwind<kRiemann>(l, r, n, star);
+}
+
+// Flux of a boundary point whose condition is not a Riemann problem
+// (rotated/euler.hpp:144-174,181-280; the rotated forms are in
+// euler_core.hpp), through the unit normal n, which points out of the cell
+// (outward) or into it: the physical flux of a boundary state, (0, p n, 0) at
+// a wall.  pow(x, gamma / (gamma - 1)) of the subsonic inlet is x^3 sqrt(x).
+__device__ __forceinline__ State BoundaryFlux(int kind, bool outward, const double *n, State const &own,
+                                              State const &given) {
+  const bool inlet = kind == kBcSupersonicInlet;
+  State c;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) c.v[k] = inlet ? given.v[k] : own.v[k];
+  FaceTrace t = TraceOf(c, n);
+  if (kind == kBcInviscidWall) t.un = 0.0;
+  if (kind == kBcSubsonicInlet || kind == kBcSubsonicOutlet) {
+    if (kind == kBcSubsonicOutlet) {  // the interior's p / rho and velocity at the given pressure
+      t.rho = given.v[4] / (t.p / t.rho);
+      t.p = given.v[4];
+    } else {
+      const double c_in = t.rho > 0 && t.p > 0 ? sqrt(kGamma * t.p / t.rho) : 0.0;
+      const double r_in = (outward ? -t.un : t.un) - c_in * (2 / kGm1);
+      const double cos_n = n[0] * given.v[1] + n[1] * given.v[2] + n[2] * given.v[3], a2 = cos_n * cos_n;
+      const double gamma_r = kGamma * kGasR, t_total = given.v[4];
+      // larger root of qa x^2 + 2 r_in x + qc = 0
+      const double qa = a2 + 2 / kGm1, qc = (kGm1 / 2) * (r_in * r_in) - a2 * gamma_r * t_total;
+      const double c_b = (sqrt(r_in * r_in - qa * qc) - r_in) / qa;
+      const double t_b = c_b * c_b / gamma_r;
+      const double mach = sqrt((t_total / t_b - 1) / (kGm1 / 2));
+      const double x = 1 + (kGm1 / 2) * mach * mach;
+      t.p = given.v[0] / (x * x * x * sqrt(x));
+      t.rho = t.p / kGasR / t_b;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) t.v[d] = given.v[1 + d] * (mach * c_b);
+      t.un = t.v[0] * n[0] + t.v[1] * n[1] + t.v[2] * n[2];
+    }
+    t.e = t.p * (1 / kGm1) + t.rho * (0.5 * (t.v[0] * t.v[0] + t.v[1] * t.v[1] + t.v[2] * t.v[2]));
+  }
+  return TraceFlux(t, n);
 }
 
 }  // namespace mcfd

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(64) void FaceFluxPointsKernel(int kind, int64_t n, 
   } else if (kind == kFluxSubsonicOutlet) {
     out = SubsonicOutletFlux(f, l, r);
   } else if constexpr (kForm == 0) {
-    out = FaceFlux<kRiemann>(f, l, r, star);
+    out = FaceFlux<kRiemann>(f.n, l, r, star);
   } else {
     out = UpwindFlux<kRiemann>(f, l, r, star);
   }

@@ -1,30 +1,41 @@
-// Nodal flux reconstruction on affine hexahedra for CDNA4 (gfx950).
+// Nodal flux reconstruction on hexahedra for CDNA4 (gfx950).
 //
 // One pass = residual of spatial/fr/general.hpp (volume term :271-288, face
 // correction :296-315,409-434, boundary corrections :435-640, det(J) scaling
 // :249-268) fused with one SSP-RK3 stage of temporal/rk.hpp:31-49.
 //
-// Work decomposition: a 256-thread workgroup owns C consecutive cells.  Each
-// pass
-//   0. loads the cells' states (one thread per solution point) and keeps a
-//      skewed structure-of-arrays copy in LDS;
-//   1. the three columns of F~ = F J* go through LDS (Q >= 3: all three in
-//      one round behind one barrier, while the first face task's neighbour
-//      line is already in flight; Q = 2: one column per round), every
-//      solution point accumulates its sum-factorised Q-point derivatives
-//      and every flux point extrapolates its direction's column to the face;
-//   2. per flux point of the cells' 6 faces: own trace (LDS), neighbour trace
-//      (the neighbour's line of Q points, gathered through L2), upwind flux
-//      and flux gap.  Each interior face is solved by both of its cells with
-//      bit-identical inputs, so the scheme stays conservative without
-//      atomics or a separate face pass;
-//   3. per solution point: lifted gaps, 1/det(J), RK stage in the
-//      reference's operation order, store.
-// The same body serves the single-mesh launch and the persistent batched
-// launch that walks a work list spanning several polynomial degrees.
+// Two kernels.  FP64 at Q = 4 points: one wavefront per cell or per two cells
+// on v_mfma_f64_4x4x4 (below).  All else: lanes that own a line of solution
+// points.  A workgroup owns C cells (16, 7, 4, 3, 1 for Q = 2..6), and each lane
+//   1. gathers, for the flux points at its line's ends, the neighbours' lines
+//      behind them (through L1 and L2); the cells' own states go to LDS once;
+//   2. extrapolates both traces of each end and solves the upwind flux there;
+//   3. forms F~_r = F J*.col(r) at its nodes and contracts it in registers with
+//      the tables in scalar registers, the ends' own fluxes lifted out of the
+//      derivative table, and lifts the upwind fluxes;
+//   4. writes the line's part of the divergence to LDS.
+// Then the threads, one per value, sum the three directions' parts and do the
+// RK stage in the reference's operation order.  Each interior face is solved by
+// both of its cells with bit-identical inputs, so the scheme stays conservative
+// without atomics or a separate face pass.  The line body serves the
+// single-mesh launch and the persistent batched launch that walks a work list
+// spanning several polynomial degrees.
+//
+// What bounds both: a pass must move U, U0 and the new U, 120 B per node (HBM at
+// about half its copy rate), and issues its FP64 instructions in about half the
+// pass's cycles; the vector memory unit, four lanes per clock whatever the width,
+// takes a third to a half.  No one unit is full, so the number of wavefronts
+// in flight decides, and with it the registers: hence lines taken one end at a
+// time and contracted node by node, and states in planes, where a line gather
+// costs four lanes one cache line.  Per pass, against one thread per node with
+// tasks per flux point, columns and a derivative through LDS: 64^3 p3 900 -> 595
+// us, 30 x 28 x 26 curved p3 113 -> 73, 35 x 37 x 33 p4 322 -> 246, 47 x 41 x 43
+// p2 180 -> 121, 36^3 p4 mixed 368 -> 297, 64^3 p1 147 -> 116, 24 x 25 x 23 p5
+// 185 -> 157, 8^3 p3 10.6 -> 9.0 (Roe, p2 HLLC).
 #include "fr_hex.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 #include "euler.hpp"
 #include "fr_common.hpp"
@@ -33,499 +44,760 @@ namespace mcfd {
 
 namespace {
 
-using fr::Extrapolate;
-using fr::FaceLineIndex;
-using fr::LineIndex;
-using fr::LocalFluxColumn;
 using fr::LogicalBlock;
-using fr::SkewedLineIndex;
 
-template <int Q, int Cells = 256 / (Q * Q * Q), int Threads = 256, bool OneRound = false>
+template <int Q>
 struct Shape {
   static constexpr int kPoints = Q * Q * Q;        // solution points per cell
-  static constexpr int kFacePoints = Q * Q;        // flux points per face
-  static constexpr int kFaceTasks = 6 * Q * Q;     // flux points per cell
-  static constexpr int kCells = Cells;             // cells per workgroup
-  static constexpr int kThreads = Threads;         // workgroup size
-  static_assert(Cells * Q * Q * Q <= Threads, "one thread per solution point");
-  static_assert(Threads % 64 == 0 && Threads <= 1024, "whole wavefronts");
-  // Skewed LDS position of solution point (i, j, k): i * kSI + j * kSJ + k.
-  // With kSJ = Q + 1 and kSI = Q (Q + 1) the Q x Q points of any line family
-  // read by one wavefront fall in distinct LDS banks (Q = 4: 20 i + 5 j + k).
-  static constexpr int kSJ = Q + 1;
-  static constexpr int kSI = Q * (Q + 1);
-  static constexpr int kSpan = (Q - 1) * (kSI + kSJ + 1) + 1;
-  static constexpr int kPad = kSpan | 1;           // odd row stride per component
-  static constexpr int kFacePad = kFaceTasks + 1;
-  // per cell: the F~ column(s) in flight (one direction, or all three with
-  // OneRound), later the flux gaps
-  static constexpr int kColumns = (OneRound ? 15 : 5) * kPad;
-  static constexpr int kScratch = kColumns > 5 * kFacePad ? kColumns : 5 * kFacePad;
-  static constexpr int kTasks = (kCells * kFaceTasks + Threads - 1) / Threads;  // per thread
-  static_assert(kCells >= 1, "at most one workgroup of solution points per cell");
-  // states, F~ columns / flux gaps, mixed reference values, face area scales
-  static constexpr int kLdsDoubles = kCells * 5 * kPad + kCells * kScratch + kCells * 15 + kCells * 6;
+  static constexpr int kLines = Q * Q;             // lines per cell and direction
+  static constexpr int kCells = Q == 6 ? 1 : (Q == 5 ? 3 : 64 / kLines);  // cells per workgroup
+  // Q = 6: two lanes per line, each with one end and the half of the nodes next
+  // to it; a whole line's registers cost a wavefront per SIMD there
+  static constexpr bool kSplit = Q == 6;
+  static constexpr int kRows = kSplit ? Q / 2 : Q, kEnds = kSplit ? 1 : 2;  // per lane
+  // lanes per direction: one wavefront for Q <= 4; two cells of Q = 5 or one of
+  // Q = 6 would leave 22 % and 44 % of its lanes idle, so there the directions
+  // follow each other (88 % and 84 % in use)
+  static constexpr int kDirLanes = Q <= 4 ? 64 : kCells * kLines * (kSplit ? 2 : 1);
+  static constexpr int kThreads = (3 * kDirLanes + 63) / 64 * 64;
+  // LDS position of solution point (i, j, k): i * kSI + j * kSJ + k.  The Q x Q
+  // points at one depth of any line family must fall in distinct LDS banks: for
+  // odd Q they do in the states' own order, for even Q with kSJ = Q + 1 and
+  // kSI = Q (Q + 1) (Q = 4: 20 i + 5 j + k).
+  static constexpr bool kSkew = Q % 2 == 0;
+  static constexpr int kSJ = kSkew ? Q + 1 : Q;
+  static constexpr int kSI = Q * kSJ;
+  static constexpr int kPad = kSkew ? ((Q - 1) * (kSI + kSJ + 1) + 1) | 1 : Q * Q * Q;  // of a component
+  // the cells' states, later the z direction's part of the divergence; the x
+  // direction's; and the y direction's, or (kAddY) no third share, which would
+  // cost resident workgroups: there y adds to x's part, behind one more barrier
+  static constexpr int kShare = kCells * 5 * kPad;
+  static constexpr bool kAddY = Q == 4;
+  static constexpr int kCellData = (kAddY ? 2 : 3) * kShare;  // per cell: 1 / det(J), time step
+  static constexpr int kFlux = kCellData + 2 * kCells;  // kSplit: the fluxes, for the line's other lane
+  static constexpr int kLdsDoubles = kFlux + (kSplit ? 3 * kDirLanes * 5 : 0);
+  static constexpr int kValues = kCells * 5 * kPoints, kLoads = (kValues + kThreads - 1) / kThreads;
+  // LDS position of value e of the workgroup's planes [cell][5][node]
+  __device__ static int At(int e) {
+    if (!kSkew) return e;
+    const int plane = e / kPoints, node = e - plane * kPoints;
+    return plane * kPad + node / (Q * Q) * kSI + node / Q % Q * kSJ + node % Q;
+  }
 };
 
-// kMixed: the F~ columns cross LDS as FP32 deviations from the cell's first
-// solution point and are contracted with FP32 FMAs (each row of the
-// derivative matrix sums to zero, so the FP64 reference value drops out of
-// the divergence); each direction's FP32 partial is accumulated in FP64.
-// States, pressure recovery, traces, the Riemann solve, the flux gaps and
-// the RK combination stay FP64.
-//
-// kOneRound: all three F~ columns cross LDS in one round (three times the
-// column space; one barrier instead of six, two in the mixed form); the
-// arithmetic and its order are those of the three-round form, so both give
-// bitwise the same results.  kPrefetch (with kOneRound): the neighbour lines
-// of that many face-task slots are loaded before the passes.
+// dg[i][m] and g_R'(x_i) through the symmetry of the points about 0: half of
+// the table suffices, and the other half's sign is free in the FMA.
+template <int Q>
+__device__ __forceinline__ double DerivativeEntry(const LineTables &lt, int i, int m) {
+  const bool low = i < Q - 1 - i || (i == Q - 1 - i && m < Q - 1 - m);
+  return low ? lt.dg[i][m] : -lt.dg[Q - 1 - i][Q - 1 - m];
+}
+
+// Makes the compiler form v here: left to itself it sinks the flux below to its
+// use, past the other end's solve, and both ends' traces stay in registers.
+template <class T>
+__device__ __forceinline__ void Pin(T *v) {
+#pragma unroll
+  for (int k = 0; k < 5; ++k) asm volatile("" : "+v"(v[k]));
+}
+
+// kMixed: the F~ lines are contracted as FP32 deviations from the value at the
+// cell's first solution point, with FP32 FMAs (each row of the derivative
+// matrix sums to zero, so the FP64 reference value drops out of the
+// divergence); each line's FP32 partial is accumulated in FP64.  States,
+// pressure recovery, traces, the Riemann solve, the flux gaps and the RK
+// combination stay FP64.
 //
 // kCurved (trilinear cells): J* and 1/det(J) are read per solution point, the
-// flux-point scale per cell flux point and the frame per face flux point (in
-// the holder's in-face order) instead of per cell and per face.
-template <int Q, int Cells, int Threads, int kRiemann, bool kDiag, bool kMixed, bool kOneRound = false,
-          int kPrefetch = 0, bool kCurved = false>
-__device__ __forceinline__ void FrHexStageBody(const FrHexArgs &a, const LineTables &lt, int64_t block,
-                                               double *lds) {
-  using S = Shape<Q, Cells, Threads, kOneRound>;
-  constexpr int NP = S::kPoints, NFP = S::kFacePoints, C = S::kCells;
-  constexpr int PAD = S::kPad, FPAD = S::kFacePad, T = S::kTasks;
-  double *s_u = lds;                          // states, SoA per cell
-  double *s_x = lds + C * 5 * PAD;            // F~ column per pass, then flux gaps
-  double *s_ref = s_x + C * S::kScratch;      // mixed: FP64 column values at node 0, [d][cell][5]
-  double *s_scale = s_ref + C * 15;           // signed face area scales of each cell
-  float *s_x32 = reinterpret_cast<float *>(s_x);
-
-  const int tid = threadIdx.x;
+// normal and the scale per cell flux point instead of per cell and per face.
+template <int Q, int kRiemann, bool kMixed, bool kCurved>
+__device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables &lt, int64_t block, double *lds) {
+  using S = Shape<Q>;
+  constexpr int NP = S::kPoints, NL = S::kLines, C = S::kCells, PAD = S::kPad, DL = S::kDirLanes;
   const int64_t c0 = block * C;
   if (c0 >= a.n_cells) return;
-  const int nc = (int)min<int64_t>(C, a.n_cells - c0);
-  const int64_t base = c0 * NP * 5;
+  const int64_t left_over = a.n_cells - c0;
+  const int nc = left_over < C ? (int)left_over : C;
 
-  // ---- node phase: load, primitive, SoA copy of the state
-  const bool node_active = tid < nc * NP;
-  const int ncell = tid / NP, node = tid - (tid / NP) * NP;
-  const int ni = node / (Q * Q), nj = (node / Q) % Q, nk = node % Q;
-  const int spos = ni * S::kSI + nj * S::kSJ + nk;  // skewed LDS position
-  State cu, pu;
-  double u0v[5] = { 0, 0, 0, 0, 0 };
-  const double *js = nullptr;
-  double inv_det = 0;
-  if (node_active) {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) cu.v[k] = a.us[base + tid * 5 + k];
-    pu = FastPrimitive(cu);
-    if (a.stage >= 2) {  // U0 of the RK combination, fetched early
-#pragma unroll
-      for (int k = 0; k < 5; ++k) u0v[k] = a.u0[base + tid * 5 + k];
-    }
-    if constexpr (kCurved) {
-      js = a.geo_node + ((c0 + ncell) * NP + node) * kNodeGeoStride;
-    } else {
-      js = a.geo + (int64_t)a.geo_id[c0 + ncell] * kGeoStride;
-      if (node < 6) s_scale[ncell * 6 + node] = js[10 + node];
-    }
-    inv_det = js[9];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) s_u[(ncell * 5 + k) * PAD + spos] = cu.v[k];
-  }
-
-  // ---- face task bookkeeping (flux points of the workgroup's cells)
-  // Tasks are numbered direction-major: w = ((d * C + cell) * 2 + side) * Q^2
-  // + a * Q + b covers the two faces normal to reference direction d.  A
-  // wavefront then holds flux points of one direction (of at most two where
-  // C * 2 Q^2 is not a multiple of 64), so the extrapolation of pass d runs
-  // only in the wavefronts that own direction d instead of in all of them.
-  constexpr int PER_DIR = C * 2 * NFP;
-  int t_cell[T], t_f[T], t_a[T], t_b[T];
-  bool t_on[T];
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const int w = tid + Threads * t;
-    const int d = w / PER_DIR, rd = w - d * PER_DIR;
-    const int cell = rd / (2 * NFP), rc = rd - cell * (2 * NFP);
-    const int side = rc / NFP, fp = rc - side * NFP;
-    t_on[t] = d < 3 && cell < nc;
-    t_cell[t] = cell;
-    // local face of (direction, side): x {4, 2}, y {1, 3}, z {0, 5}
-    t_f[t] = d == 0 ? (side ? 2 : 4) : (d == 1 ? (side ? 3 : 1) : (side ? 5 : 0));
-    t_a[t] = fp / Q;
-    t_b[t] = fp - (fp / Q) * Q;
-  }
-  // neighbour and face-info words of the face tasks, fetched before the
-  // volume passes so that the face phase starts its gathers at once
-  int32_t t_nb[T], t_info[T];
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-    t_nb[t] = t_on[t] ? a.nbr[(c0 + t_cell[t]) * 6 + t_f[t]] : 0;
-    t_info[t] = t_on[t] ? a.finfo[(c0 + t_cell[t]) * 6 + t_f[t]] : 0;
-  }
-  double fn[T][5];
-
-  // mixed: node 0 of each cell publishes its three F~ columns, the FP64
-  // references of the FP32 deviations; the first pass's barrier orders them
-  if constexpr (kMixed) {
-    if (node_active && node == 0) {
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        double col[5];
-        LocalFluxColumn<kDiag>(cu, pu, js, d, col);
-#pragma unroll
-        for (int k = 0; k < 5; ++k) s_ref[(d * C + ncell) * 5 + k] = col[k];
-      }
-    }
-  }
-
-  // neighbour line of face task t (Q nodes of the neighbour cell along the
-  // face normal, in the orientation of this cell's flux point)
-  auto gather = [&](int t, double (*raw)[5]) {
-    const int32_t nb = t_nb[t], info = t_info[t];
-    const int ia = t_a[t], ib = t_b[t];
-    const int nf = info & 7, orient = (info >> 3) & 7;
-    const int s = (orient & 1) ? ib : ia, tt = (orient & 1) ? ia : ib;
-    const int na = (orient & 2) ? Q - 1 - s : s;
-    const int nbb = (orient & 4) ? Q - 1 - tt : tt;
-    const LineIndex ln = FaceLineIndex(Q, nf);
-    const double *src = a.us + ((int64_t)nb * NP + na * ln.a_mul + nbb * ln.b_mul) * 5;
-#pragma unroll
-    for (int m = 0; m < Q; ++m)
-#pragma unroll
-      for (int k = 0; k < 5; ++k) raw[m][k] = src[m * ln.stride * 5 + k];
+  const int tid = threadIdx.x;
+  const int dir = DL == 64 ? __builtin_amdgcn_readfirstlane(tid >> 6) : min(tid / DL, 2);
+  const int half = S::kSplit ? (tid - dir * DL) / (C * NL) : 0;  // of a split line: its end
+  const int lane = tid - dir * DL - half * (C * NL);
+  const int cell = lane / NL, line = lane - (lane / NL) * NL;
+  const int la = line / Q, lb = line - (line / Q) * Q;  // in-face indices of the line's two ends
+  const bool active = half < 2 && cell < nc;
+  const int64_t c = c0 + (active ? cell : 0);
+  const int stride = dir == 0 ? Q * Q : (dir == 1 ? Q : 1);
+  const int node0 = la * (dir == 0 ? Q : Q * Q) + lb * (dir == 2 ? Q : 1);
+  // local faces at the line's lower and upper end: x {4, 2}, y {1, 3}, z {0, 5}
+  const int f_lo = dir == 0 ? 4 : (dir == 1 ? 1 : 0), f_hi = dir == 0 ? 2 : (dir == 1 ? 3 : 5);
+  // Loads are waited for in the order of their issue: what is needed first, or
+  // needed to form an address, goes first.
+  const int f_first = half == 1 ? f_hi : f_lo;
+  const FrFace lower = a.faces[c * 6 + f_first], upper = S::kSplit ? lower : a.faces[c * 6 + f_hi];
+  const int geo_id = kCurved ? 0 : a.geo_id[c];
+  double v[S::kLoads];  // the cells' states, one load per value for all three directions
+  const int values = nc * 5 * NP;
+  auto value = [&](int it) {  // threads past the end repeat the last value
+    const int e = tid + it * S::kThreads;
+    return e < values ? e : values - 1;
   };
-  constexpr int PF = kPrefetch < T ? kPrefetch : T;
-  double pre[PF > 0 ? PF : 1][Q][5];
-
-  // ---- three passes: one column of F~ at a time through LDS (or all three
-  // written at once with kOneRound)
-  double div[5] = { 0, 0, 0, 0, 0 };
-  if constexpr (kOneRound) {
-    if constexpr (kMixed) __syncthreads();  // the FP64 references of the deviations
-    if (node_active) {
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        double col[5];
-        LocalFluxColumn<kDiag>(cu, pu, js, d, col);
-        if constexpr (kMixed) {
+  for (int it = 0; it < S::kLoads; ++it) v[it] = a.us[c0 * (5 * NP) + value(it)];
+  // unit normal (left to right) and face scale of end s
+  double n[3], scale = 0;
+  auto geometry = [&](FrFace const &face, int s) {
+    if constexpr (kCurved) {
+      const double *fp = a.face_point + ((c * 6 + (s ? f_hi : f_first)) * NL + line) * 4;
 #pragma unroll
-          for (int k = 0; k < 5; ++k)
-            s_x32[ncell * S::kScratch + (5 * d + k) * PAD + spos] = (float)(col[k] - s_ref[(d * C + ncell) * 5 + k]);
-        } else {
+      for (int d = 0; d < 3; ++d) n[d] = fp[d];
+      scale = fp[3];
+    } else {
+      const double *fp = a.normals + (int64_t)(face.normal >> 1) * kNormalStride;
 #pragma unroll
-          for (int k = 0; k < 5; ++k) s_x[ncell * S::kScratch + (5 * d + k) * PAD + spos] = col[k];
-        }
-      }
+      for (int d = 0; d < 3; ++d) n[d] = fp[d];
     }
-    __syncthreads();
-    // the first face tasks' neighbour lines, in flight during the passes
-#pragma unroll
-    for (int t = 0; t < PF; ++t)
-      if (t_on[t] && t_nb[t] >= 0) gather(t, pre[t]);
-  }
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int cb = kOneRound ? 5 * d * PAD : 0;  // column d within the cell's scratch
-    if constexpr (!kOneRound) {
-      __syncthreads();
-      double col[5];
-      if (node_active) {
-        LocalFluxColumn<kDiag>(cu, pu, js, d, col);
-        if constexpr (kMixed) {
-#pragma unroll
-          for (int k = 0; k < 5; ++k)
-            s_x32[ncell * S::kScratch + k * PAD + spos] = (float)(col[k] - s_ref[(d * C + ncell) * 5 + k]);
-        } else {
-#pragma unroll
-          for (int k = 0; k < 5; ++k) s_x[ncell * S::kScratch + k * PAD + spos] = col[k];
-        }
-      }
-      __syncthreads();
-    }
-    if (node_active) {
-      const int id = d == 0 ? ni : (d == 1 ? nj : nk);
-      const int stride = d == 0 ? S::kSI : (d == 1 ? S::kSJ : 1);
-      const int line0 = spos - id * stride;
-      if constexpr (kMixed) {
-        const float *sx = s_x32 + ncell * S::kScratch + cb;
-#pragma unroll
-        for (int k = 0; k < 5; ++k) {
-          float acc = 0.0f;
-#pragma unroll
-          for (int m = 0; m < Q; ++m) acc = __fmaf_rn((float)lt.d[id][m], sx[k * PAD + line0 + m * stride], acc);
-          div[k] += (double)acc;
-        }
-      } else {
-        const double *sx = s_x + ncell * S::kScratch + cb;
-#pragma unroll
-        for (int k = 0; k < 5; ++k) {
-          double acc = div[k];
-#pragma unroll
-          for (int m = 0; m < Q; ++m) acc = __fma_rn(lt.d[id][m], sx[k * PAD + line0 + m * stride], acc);
-          div[k] = acc;
-        }
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      const LineIndex li = SkewedLineIndex<Q>(t_f[t]);
-      if (t_on[t] && li.dir == d) {
-        const int l0 = t_a[t] * li.a_mul + t_b[t] * li.b_mul;
-        const double *lw = lt.lend[li.side];
-        if constexpr (kMixed) {
-          const float *sx = s_x32 + t_cell[t] * S::kScratch + cb;
-#pragma unroll
-          for (int k = 0; k < 5; ++k) {
-            float acc = (float)lw[0] * sx[k * PAD + l0];
-#pragma unroll
-            for (int m = 1; m < Q; ++m) acc = __fmaf_rn((float)lw[m], sx[k * PAD + l0 + m * li.stride], acc);
-            fn[t][k] = s_ref[(d * C + t_cell[t]) * 5 + k] + (double)acc;
-          }
-        } else {
-          const double *sx = s_x + t_cell[t] * S::kScratch + cb;
-#pragma unroll
-          for (int k = 0; k < 5; ++k) {
-            double vals[Q];
-#pragma unroll
-            for (int m = 0; m < Q; ++m) vals[m] = sx[k * PAD + l0 + m * li.stride];
-            fn[t][k] = Extrapolate<Q>(lw, vals);
-          }
-        }
-      }
-    }
-  }
-
-  // ---- flux points: traces, upwind flux, flux gap
-  double gap[T][5];
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-    if (!t_on[t]) continue;
-    const int f = t_f[t], ia = t_a[t], ib = t_b[t];
-    const LineIndex li = SkewedLineIndex<Q>(f);
-    const double *lw = lt.lend[li.side];
-    State own;
-    {
-      const int l0 = ia * li.a_mul + ib * li.b_mul;
-      const double *su = s_u + t_cell[t] * 5 * PAD;
+  };
+  // the neighbour's line behind end s, from its lower end upwards
+  struct Line { double v[Q][5]; };
+  auto gather = [&](FrFace const &face) {
+    Line nb;  // left undefined without a neighbour
+    if (!active || face.nbr < 0) return nb;
+    const int g = face.gather, step = g >> 24;
+    const int first = (g & 255) + (int)(int8_t)(g >> 8) * la + (int)(int8_t)(g >> 16) * lb + (step < 0 ? (Q - 1) * step : 0);
+    const int up = step < 0 ? -step : step;
+    const double *src = a.us + (int64_t)face.nbr * (5 * NP) + first;
+    if (__all(up == 1)) {  // along consecutive nodes
+      typedef double Two __attribute__((ext_vector_type(2), aligned(8)));
 #pragma unroll
       for (int k = 0; k < 5; ++k) {
-        double vals[Q];
 #pragma unroll
-        for (int m = 0; m < Q; ++m) vals[m] = su[k * PAD + l0 + m * li.stride];
-        own.v[k] = Extrapolate<Q>(lw, vals);
+        for (int q = 0; q + 1 < Q; q += 2) {
+          const Two w = *reinterpret_cast<const Two *>(src + k * NP + q);
+          nb.v[q][k] = w.x;
+          nb.v[q + 1][k] = w.y;
+        }
+        if (Q & 1) nb.v[Q - 1][k] = src[k * NP + Q - 1];
       }
-    }
-    const int32_t nb = t_nb[t];
-    const int32_t info = t_info[t];
-    const double *fr;
-    double scale;
-    if constexpr (kCurved) {
-      // the face point in the holder's in-face order: this cell's own (a, b),
-      // or the neighbour's where the neighbour holds the face
-      int cp = ia * Q + ib;
-      if (!((info >> 6) & 1)) {
-        const int orient = (info >> 3) & 7;
-        const int s = (orient & 1) ? ib : ia, tt = (orient & 1) ? ia : ib;
-        cp = ((orient & 2) ? Q - 1 - s : s) * Q + ((orient & 4) ? Q - 1 - tt : tt);
-      }
-      fr = a.frames + ((int64_t)(info >> 7) * NFP + cp) * kFrameStride;
-      scale = a.fscale[((c0 + t_cell[t]) * 6 + f) * NFP + ia * Q + ib];
+      asm volatile("; 16-byte loads" ::: "memory");  // keeps the compiler from merging the two branches' loads
     } else {
-      fr = a.frames + (int64_t)(info >> 7) * kFrameStride;
-      scale = s_scale[t_cell[t] * 6 + f];
-    }
-    FaceFrame frame;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) { frame.n[d] = fr[d]; frame.t[d] = fr[3 + d]; }
-    frame.b[0] = frame.n[1] * frame.t[2] - frame.n[2] * frame.t[1];
-    frame.b[1] = frame.n[2] * frame.t[0] - frame.n[0] * frame.t[2];
-    frame.b[2] = frame.n[0] * frame.t[1] - frame.n[1] * frame.t[0];
-    State fu;
-    double sgn = 1.0;
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int k = 0; k < 5; ++k) nb.v[q][k] = src[k * NP + q * up];
+    }
+    return nb;
+  };
+  geometry(lower, 0);
+  if (tid < nc) {
+    lds[S::kCellData + tid] = kCurved ? 0.0 : a.geo[(int64_t)a.geo_id[c0 + tid] * kGeoStride + kGeoInvDet];
+    lds[S::kCellData + C + tid] = a.case_dt ? a.case_dt[a.cell_case[c0 + tid]] : a.dt;
+  }
+  double dir_col[3] = { 0, 0, 0 };
+  if constexpr (!kCurved) {
+    const double *src = a.geo + (int64_t)geo_id * kGeoStride + 4 * dir;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) dir_col[e] = src[e];
+    scale = src[3];
+  }
+  Line nb = gather(lower);
+#pragma unroll
+  for (int it = 0; it < S::kLoads; ++it) lds[S::At(value(it))] = v[it];
+  __syncthreads();
+
+  const int pos0 = cell * 5 * PAD + la * (dir == 0 ? S::kSJ : S::kSI) + lb * (dir == 2 ? S::kSJ : 1);
+  const int pos_step = dir == 0 ? S::kSI : (dir == 1 ? S::kSJ : 1);
+  double flux[S::kEnds][5];  // upwind fluxes at the line's ends times the face scale, along +r
+  if (active) {
+#pragma unroll
+    for (int s = 0; s < S::kEnds; ++s) {
+      const bool at_upper = S::kSplit ? half == 1 : s == 1;
+      const FrFace face = s ? upper : lower;
+      const int64_t point = (c * 6 + (s ? f_hi : f_first)) * NL + line;  // this cell's flux point
+      const bool swap = (kRiemann == kExact || a.any_swap) ? (face.normal & 1) != 0 : false;
+      State other;
+      int kind = kBcSmart;
+      if (face.nbr >= 0) {
+        // the neighbour's trace at the end it has here, in that same order
+        const bool lower_end = (face.gather >> 24) > 0;
+        double end[Q];
+#pragma unroll
+        for (int m = 0; m < Q; ++m) end[m] = lower_end ? lt.end[m] : lt.end[Q - 1 - m];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+          double acc = end[0] * nb.v[0][k];
+#pragma unroll
+          for (int m = 1; m < Q; ++m) acc = __fma_rn(end[m], nb.v[m][k], acc);
+          other.v[k] = acc;
+        }
+      } else {
+        const int tag = -face.nbr - 1;
+        kind = a.bc_kind[tag];
+        // the tag's constant state, or this point's value of the tag's
+        // boundary function at the stage time
+        const double *gs = a.bc_point_state ? a.bc_point_state + ((int64_t)face.bface * NL + line) * 5
+                                            : a.bc_state + tag * 5;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) other.v[k] = gs[k];
+      }
+      Pin(other.v);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      // the own trace: a fused chain from the line's lower node upwards, the
+      // order in which the cell behind the face forms it too
+      State own;
+      double own_end[Q];
+#pragma unroll
+      for (int m = 0; m < Q; ++m) own_end[m] = at_upper ? lt.end[Q - 1 - m] : lt.end[m];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        double acc = own_end[0] * lds[pos0 + k * PAD];
+#pragma unroll
+        for (int m = 1; m < Q; ++m) acc = __fma_rn(own_end[m], lds[pos0 + k * PAD + m * pos_step], acc);
+        own.v[k] = acc;
+      }
+      Pin(own.v);
+      // the exact solver's state of this flux point, one copy per side: both
+      // sides solve the same problem with the same inputs every pass, so the
+      // two copies stay equal
+      bool star = kRiemann == kExact ? a.exact_star[point] != 0 : false;
+      State l, r;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        l.v[k] = at_upper ? own.v[k] : other.v[k];
+        r.v[k] = at_upper ? other.v[k] : own.v[k];
+      }
+      if (kRiemann == kExact || a.any_swap) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+          const double x = l.v[k], y = r.v[k];
+          l.v[k] = swap ? y : x;
+          r.v[k] = swap ? x : y;
+        }
+      }
+      State fu;
+      if (kind == kBcSmart) {
+        fu = FaceFlux<kRiemann>(n, l, r, star);
+      } else {  // the flux through the left-to-right normal, as the upwind one
+        const bool left = at_upper != swap;
+        fu = BoundaryFlux(kind, left, n, left ? l : r, left ? r : l);
+      }
+      if constexpr (kRiemann == kExact) a.exact_star[point] = star ? 1 : 0;
+      // left-to-right is the +r direction of this cell unless the roles are swapped
+      const double along = swap ? -scale : scale;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) flux[s][k] = fu.v[k] * along;
+      Pin(flux[s]);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + 1 < S::kEnds) {  // not in flight during the solve: that would cost a wavefront per SIMD
+        geometry(upper, 1);
+        nb = gather(upper);
+      }
+    }
+  }
+
+  double *const my_flux = lds + S::kFlux + 5 * tid, *const far_flux = my_flux + (half ? -5 : 5) * (C * NL);
+  if (S::kSplit && active) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) my_flux[k] = flux[0][k];
+  }
+
+  // ---- each thread's values of U, and U0, for the RK stage
+  double u0[S::kLoads];
+  if (a.stage >= 2) {
+#pragma unroll
+    for (int it = 0; it < S::kLoads; ++it) u0[it] = __builtin_nontemporal_load(a.u0 + c0 * (5 * NP) + value(it));
+  }
+#pragma unroll
+  for (int it = 0; it < S::kLoads; ++it) v[it] = lds[S::At(value(it))];
+
+  // ---- F~_r along the line, contracted node by node, so that only the Q x 5
+  // sums stay in registers; then the fluxes lifted
+  typedef typename std::conditional<kMixed, float, double>::type Sum;
+  Sum d[S::kRows][5];
+  Sum gap_end[2][5];  // mixed: F~_r's deviation at the line's ends
+  // Nodes are taken upwards, and inwards from the lane's end of a split line:
+  // the tables' symmetry leaves the sums there with the opposite sign.  FP32
+  // sums keep one order for all rows, and the upper lane its own table rows.
+  const bool inwards = S::kSplit && !kMixed && half == 1;
+  const bool mirror = S::kSplit && half == 1;
+  const int first_pos = pos0 + (inwards ? (Q - 1) * pos_step : 0), node_step = inwards ? -pos_step : pos_step;
+  double ref[5];      // mixed: F~_r of the cell's first solution point, formed by every line alike
+  if (active) {
+    const double *col_src = kCurved ? a.col_node + ((c * 3 + dir) * NP + node0 + (inwards ? (Q - 1) * stride : 0)) * 3 : nullptr;
+    const int col_step = inwards ? -3 * stride : 3 * stride;
+    double col[3], next[3] = { dir_col[0], dir_col[1], dir_col[2] };
+    if constexpr (kCurved) {
+#pragma unroll
+      for (int e = 0; e < 3; ++e) next[e] = col_src[e];
+    }
+    if constexpr (kMixed) {
+      State first;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) first.v[k] = lds[cell * 5 * PAD + k * PAD];
+      const FaceTrace t = TraceOf(first, dir_col);
+      ref[0] = first.v[1] * dir_col[0] + first.v[2] * dir_col[1] + first.v[3] * dir_col[2];
+#pragma unroll
+      for (int e = 0; e < 3; ++e) ref[1 + e] = first.v[1 + e] * t.un + t.p * dir_col[e];
+      ref[4] = (first.v[4] + t.p) * t.un;
+    }
+#pragma unroll
+    for (int m = 0; m < Q; ++m) {
+      double w[5];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) w[k] = lds[first_pos + k * PAD + m * node_step];
+#pragma unroll
+      for (int e = 0; e < 3; ++e) col[e] = next[e];
+      if (kCurved && m + 1 < Q) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) next[e] = col_src[(m + 1) * col_step + e];
+      }
+      // contravariant momentum and velocity, and pressure; the zeroing rule of
+      // types.hpp:195-202,289-301 only where some lane of the wavefront needs it
+      const double inv = FastRcp(w[0]);
+      const double mom = w[1] * col[0] + w[2] * col[1] + w[3] * col[2];
+      double vel = mom * inv;
+      double p = (w[4] - 0.5 * (w[1] * w[1] + w[2] * w[2] + w[3] * w[3]) * inv) * kGm1;
+      if (!__all(w[0] > 0 && w[4] >= 0 && p >= 0)) {
+        const bool bad = w[0] < 0 || w[4] < 0;
+        const bool vacuum = !bad && w[0] == 0;
+        const bool zero = bad || (!vacuum && p < 0);
+        vel = zero ? 0.0 : (vacuum ? mom : vel);
+        p = zero ? 0.0 : (vacuum ? w[4] : p);
+      }
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        const double f = k == 0 ? mom : (k == 4 ? (w[4] + p) * vel : w[k] * vel + p * col[k == 0 ? 0 : k - 1]);
+        if constexpr (kMixed) {
+          const float dev = (float)(f - ref[k]);
+#pragma unroll
+          for (int i = 0; i < S::kRows; ++i)
+            d[i][k] = __fmaf_rn(mirror ? lt.d[Q - 1 - i][m] : lt.d[i][m], dev, m ? d[i][k] : 0.0f);
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+            gap_end[s][k] = m ? __fmaf_rn(lt.lend[s][m], dev, gap_end[s][k]) : lt.lend[s][0] * dev;
+        } else {
+#pragma unroll
+          for (int i = 0; i < S::kRows; ++i)
+            d[i][k] = m ? __fma_rn(DerivativeEntry<Q>(lt, i, m), f, d[i][k]) : DerivativeEntry<Q>(lt, i, 0) * f;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < S::kRows; ++i) Pin(d[i]);  // else the sums are put off and all nodes' fluxes stay in registers
+      if constexpr (kMixed) {
+        Pin(gap_end[0]);
+        Pin(gap_end[1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __syncthreads();  // from here on the z lines' parts replace the states
+  double *const part = lds + (dir == 2 ? 0 : (dir == 1 && !S::kAddY ? 2 : 1) * S::kShare) + pos0;
+  auto lift = [&](bool add) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      // the lower and the upper end's gap; of a split line the near and the far end's
+      double gap[2] = { flux[0][k], S::kSplit ? far_flux[k] : flux[S::kEnds - 1][k] };
+      if constexpr (kMixed) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)  // less F~_r at the ends
+          gap[s] -= ref[k] + (double)(mirror ? gap_end[1 - s][k] : gap_end[s][k]);
+      }
+#pragma unroll
+      for (int i = 0; i < S::kRows; ++i) {
+        double sum = (double)d[i][k];
+        if (kMixed && mirror) sum = -sum;
+        sum = __fma_rn(lt.gp[0][i], gap[0], sum);
+        sum = __fma_rn(-lt.gp[0][Q - 1 - i], gap[1], sum);
+        if (mirror) sum = -sum;
+        const int at = k * PAD + (mirror ? Q - 1 - i : i) * pos_step;
+        if (add) sum = part[at] + sum;
+        part[at] = sum;
+      }
+    }
+  };
+  if (active && !(S::kAddY && dir == 1)) lift(false);
+  __syncthreads();
+  if constexpr (S::kAddY) {
+    if (active && dir == 1) lift(true);
+    __syncthreads();
+  }
+
+  // ---- per value: the three directions' sum, 1/det(J), RK stage, store
+#pragma unroll
+  for (int it = 0; it < S::kLoads; ++it) {
+    const int e = tid + it * S::kThreads;
+    if (e >= values) continue;
+    const int at = S::At(e), cl = C == 1 ? 0 : e / (5 * NP), k = (e - cl * (5 * NP)) / NP, node = e - (cl * 5 + k) * NP;
+    const double inv_det = kCurved ? a.inv_det_node[(c0 + cl) * NP + node] : lds[S::kCellData + cl];
+    double sum = lds[S::kShare + at];
+    if constexpr (!S::kAddY) sum += lds[2 * S::kShare + at];
+    sum += lds[at];
+    const double out = fr::RkOutput(a.stage, -sum * inv_det, v[it], u0[it], lds[S::kCellData + C + cl]);
+    // the residual is handed out as a column, states stay in planes; streamed,
+    // so that the states which neighbours still gather keep the L2
+    __builtin_nontemporal_store(out, a.out + (a.stage == 0 ? ((c0 + cl) * NP + node) * 5 + k : c0 * (5 * NP) + e));
+    if (a.dt_min_bits) lds[at] = out;
+  }
+  if (a.dt_min_bits) {
+    // fem.hpp:412-435 on the state just written, as FrHexTimeStepKernel: min
+    // over cells of length / max(1e-5, max over nodes of |u| + c), which is the
+    // min over nodes of length / max(1e-5, |u| + c); the bits of positive
+    // doubles order as the doubles do
+    __syncthreads();
+    double local = 1e300;
+    for (int w = tid; w < nc * NP; w += S::kThreads) {
+      const int cl = w / NP, at = S::At(cl * 5 * NP + w - cl * NP);
+      State out;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) out.v[k] = lds[at + k * PAD];
+      local = fmin(local, a.geo[(int64_t)(kCurved ? c0 + cl : a.geo_id[c0 + cl]) * kGeoStride + kGeoLength] /
+                              fmax(1e-5, MaxSpeed(out)));
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o /= 2) local = fmin(local, __shfl_xor(local, o));
+    if ((tid & 63) == 0) atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(local));
+  }
+}
+
+// Wavefronts per SIMD to leave room for: what the registers allow without
+// spills (whose traffic has cost more than a wavefront every time).  Q = 4 mixed
+// with 4 and 76 B of spills: 48^3 428 us instead of 322.
+template <int Q, int kRiemann>
+constexpr int LineWaves() {
+  return kRiemann == kExact ? 2 : ((Q <= 3 || Q == 6 ? 4 : 3));
+}
+
+template <int Q, int kRiemann, bool kMixed, bool kCurved>
+__global__ __launch_bounds__(Shape<Q>::kThreads) __attribute__((amdgpu_waves_per_eu(LineWaves<Q, kRiemann>())))
+void FrHexStageKernel(FrHexArgs a, LineTables lt) {
+  __shared__ double lds[Shape<Q>::kLdsDoubles];
+  int64_t block = LogicalBlock(a.xcd_remap);
+  if (a.tile_order) block = a.tile_order[block];
+  FrLineBody<Q, kRiemann, kMixed, kCurved>(a, lt, block, lds);
+}
+
+// ------------------------------------------------------------ Q = 4, FP64
+// One wavefront per cell: its 64 lanes are the cell's 4^3 nodes, and the 4 x 4
+// line operators are v_mfma_f64_4x4x4 (four independent 4 x 4 products): with
+// lane = 16 h + 4 m + l,
+//   D(h, m, l) = C(h, m, l) + sum_k A(k, m, h) B(k, m, l),
+// a fused chain over k = 0..3, where X(k, m, l) is X's value in lane
+// 16 k + 4 m + l.  A field F given with the contracted index in h is
+// multiplied by a table T as mfma(T^, F), T^(k, m, r) = T[r][k].
+__device__ __forceinline__ double Mfma(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+
+// LDS of the kernel below, in doubles: the cells' states (skewed as Shape<4>)
+// and the records of the flux points to come.
+template <int kCells>
+struct CellShape {
+  static constexpr int kState = 5 * 79, kLater = kCells * kState + (kCells & 1);
+  static constexpr int kLdsDoubles = kLater + kCells * 2 * 64;
+};
+
+// kCells = 1 or 2 cells, c0 and c0 + 1, on one wavefront.  The 32 z flux points
+// of a cell fill half a wavefront: two cells share one pass over theirs.
+// Against one line per lane at the same size (64^3, Roe): 862 -> 638 us with one
+// cell per wavefront.  4 wavefronts per SIMD; 5 gave nothing.
+template <int kCells, int kRiemann, bool kCurved>
+__device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables &lt, int64_t c0, double *lds) {
+  using S = CellShape<kCells>;
+  constexpr int NP = 64, Z = kCells;  // slots 0 .. Z - 1: the cells' x and y faces; slot Z: the z faces
+  const int lane = threadIdx.x & 63;
+  const int h = lane >> 4, m = (lane >> 2) & 3, l = lane & 3;
+  // This lane's flux points.  Slots below Z: x-, x+, y-, y+ in h = 0..3 at in-face
+  // (m, l).  Slot Z: z-, z+ of the first cell in h = 0, 1 and of the second in
+  // h = 2, 3 (or of the first again), at (l, m).
+  const int f_xy = (0x3124 >> (4 * h)) & 7, f_z = (h & 1) ? 5 : 0;
+  const int64_t c1 = kCells == 2 && c0 + 1 < a.n_cells ? c0 + 1 : c0;  // an odd last cell is done twice
+  // Loads are waited for in the order of their issue: what is needed first, or
+  // needed to form an address, goes first.  The cells' geometry is uniform and
+  // comes through scalar loads, as long as no store precedes them.
+  double geo[kCells][14], dt[kCells];
+#pragma unroll
+  for (int g = 0; g < kCells; ++g) {
+    const int64_t c = g ? c1 : c0;
+    const double *src = a.geo + (int64_t)a.geo_id[c] * kGeoStride;
+#pragma unroll
+    for (int e = 0; e < 14; ++e) geo[g][e] = src[e];
+    dt[g] = a.case_dt ? a.case_dt[a.cell_case[c]] : a.dt;
+  }
+  auto cell_at = [&](int s) -> int64_t { return s == Z ? (h < 2 ? c0 : c1) : (s ? c1 : c0); };
+  FrFace face = a.faces[cell_at(Z) * 6 + f_z];
+  double u[kCells][5];
+  FrFace *const later = reinterpret_cast<FrFace *>(lds + S::kLater);  // the later slots' records wait in LDS
+#pragma unroll
+  for (int s = 0; s < Z; ++s) later[s * 64 + lane] = a.faces[cell_at(s) * 6 + f_xy];
+#pragma unroll
+  for (int g = 0; g < kCells; ++g)
+#pragma unroll
+    for (int k = 0; k < 5; ++k) u[g][k] = a.us[(g ? c1 : c0) * (5 * NP) + k * NP + lane];
+  const CellOps *ops = a.cell_ops;
+
+  // the neighbour's line behind flux point s, from its lower end upwards
+  struct Line { double v[4][5]; };
+  auto gather = [&](int s) {
+    Line nb;  // left undefined without a neighbour
+    if (face.nbr < 0) return nb;
+    const int g = face.gather, step = g >> 24;
+    const int first = (g & 255) + (int)(int8_t)(g >> 8) * m + (int)(int8_t)(g >> 16) * l + (step < 0 ? 3 * step : 0);
+    const int up = step < 0 ? -step : step;
+    const double *src = a.us + (int64_t)face.nbr * (5 * NP) + first;
+    if (s == Z && __all(up == 1)) {
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        const double2 lo = *reinterpret_cast<const double2 *>(src + k * NP);
+        const double2 hi = *reinterpret_cast<const double2 *>(src + k * NP + 2);
+        nb.v[0][k] = lo.x;
+        nb.v[1][k] = lo.y;
+        nb.v[2][k] = hi.x;
+        nb.v[3][k] = hi.y;
+      }
+      asm volatile("; 16-byte loads" ::: "memory");  // keeps the compiler from merging the two branches' loads
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int k = 0; k < 5; ++k) nb.v[q][k] = src[k * NP + q * up];
+    }
+    return nb;
+  };
+  // unit normal (left to right) and face scale of flux point s
+  double n[3], scale;
+  auto point_of = [&](int s) { return (cell_at(s) * 6 + (s == Z ? f_z : f_xy)) * 16 + (s == Z ? l * 4 + m : m * 4 + l); };
+  auto geometry = [&](int s) {
+    if constexpr (kCurved) {
+      const double *fp = a.face_point + point_of(s) * 4;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) n[d] = fp[d];
+      scale = fp[3];
+    } else {
+      const double *fp = a.normals + (int64_t)(face.normal >> 1) * kNormalStride;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) n[d] = fp[d];
+      scale = s == Z ? (h < 2 ? geo[0][11] : geo[kCells - 1][11]) : (h < 2 ? geo[s % kCells][3] : geo[s % kCells][7]);
+    }
+  };
+  geometry(Z);
+  Line nb = gather(Z);
+  // states with j, and with k, in h: (i, k) and (j, i) in (m, l)
+  const int at_x = h * 20 + m * 5 + l, at_y = m * 20 + h * 5 + l, at_z = l * 20 + m * 5 + h;
+#pragma unroll
+  for (int g = 0; g < kCells; ++g)
+#pragma unroll
+    for (int k = 0; k < 5; ++k) lds[g * S::kState + k * 79 + at_x] = u[g][k];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  double end01 = ops->end01[lane], end23 = ops->end23[lane];
+  // the cell's own traces at its ends
+  auto own_trace = [&](int s) {
+    State own;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const double *const su = lds + (s == Z ? 0 : s) * S::kState + k * 79;
+      if (s < Z) own.v[k] = Mfma(end23, su[at_y], Mfma(end01, su[at_x], 0.0));
+      else if (kCells == 1) own.v[k] = Mfma(end01 + end23, su[at_z], 0.0);
+      else own.v[k] = Mfma(end23, su[S::kState + at_z], Mfma(end01, su[at_z], 0.0));
+    }
+    return own;
+  };
+  double flux_z[5];
+#pragma unroll
+  for (int turn = 0; turn <= Z; ++turn) {
+    const int s = turn == 0 ? Z : turn - 1;
+    State own = own_trace(s);
+    Pin(own.v);
+    double flux[5];
+
+    // ---- flux points
+    const bool upper = (h & 1) != 0;
+    const bool swap = (face.normal & 1) != 0, left = upper != swap;
+    State other;
+    int kind = kBcSmart;
+    if (face.nbr >= 0) {
+      // the neighbour's trace at the end it has here, in its own order
+      const bool lower_end = (face.gather >> 24) > 0;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        double acc = (lower_end ? lt.end[0] : lt.end[3]) * nb.v[0][k];
+#pragma unroll
+        for (int q = 1; q < 4; ++q) acc = __fma_rn(lower_end ? lt.end[q] : lt.end[3 - q], nb.v[q][k], acc);
+        other.v[k] = acc;
+      }
+    } else {
+      const int tag = -face.nbr - 1;
+      kind = a.bc_kind[tag];
+      // the tag's constant state, or this point's value of the tag's boundary
+      // function at the stage time
+      const double *gs = a.bc_point_state
+          ? a.bc_point_state + ((int64_t)face.bface * 16 + m * 4 + l) * 5 : a.bc_state + tag * 5;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) other.v[k] = gs[k];
+    }
+    if (s == Z) {  // gathered at (m, l), where four lanes share a cache line; wanted at (l, m)
+      kind = __shfl(kind, 16 * h + 4 * l + m);
+#pragma unroll
+      for (int k = 0; k < 5; ++k) other.v[k] = __shfl(other.v[k], 16 * h + 4 * l + m);
+    }
+    Pin(other.v);
+    asm volatile("" ::: "memory");
+    const double along = swap ? -scale : scale;
+    __builtin_amdgcn_sched_barrier(0);
     // the exact solver's state of this flux point, one copy per side: both
     // sides solve the same problem with the same inputs every pass, so the
     // two copies stay equal
-    const int64_t star_slot = ((c0 + t_cell[t]) * 6 + f) * NFP + ia * Q + ib;
-    bool star = kRiemann == kExact ? a.exact_star[star_slot] != 0 : false;
-    if (nb >= 0) {
-      const bool holder = (info >> 6) & 1;
-      const double *nw = lt.lend[FaceLineIndex(Q, info & 7).side];
-      double raw[Q][5];
-      if (kOneRound && t < PF) {
-#pragma unroll
-        for (int m = 0; m < Q; ++m)
-#pragma unroll
-          for (int k = 0; k < 5; ++k) raw[m][k] = pre[t < PF ? t : 0][m][k];
-      } else {
-        gather(t, raw);
-      }
-      State other;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) {
-        double vals[Q];
-#pragma unroll
-        for (int m = 0; m < Q; ++m) vals[m] = raw[m][k];
-        other.v[k] = Extrapolate<Q>(nw, vals);
-      }
-      fu = FaceFlux<kRiemann>(frame, holder ? own : other, holder ? other : own, star);
-      sgn = holder ? 1.0 : -1.0;
-    } else {
-      const int tag = -nb - 1;
-      const int kind = a.bc_kind[tag];
-      // the tag's constant state, or this point's value of the tag's
-      // boundary function at the stage time
-      const double *gs = a.bc_point_state
-          ? a.bc_point_state + ((int64_t)a.bface_of[(c0 + t_cell[t]) * 6 + f] * NFP + ia * Q + ib) * 5
-          : a.bc_state + tag * 5;
-      State given;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) given.v[k] = gs[k];
-      if (kind == kBcInviscidWall) {
-        fu = WallFlux(frame, own);
-      } else if (kind == kBcSupersonicOutlet) {
-        fu = StateFlux(frame, own);
-      } else if (kind == kBcSupersonicInlet) {
-        fu = StateFlux(frame, given);
-      } else if (kind == kBcSubsonicInlet) {
-        fu = SubsonicInletFlux(frame, own, given);
-      } else if (kind == kBcSubsonicOutlet) {
-        fu = SubsonicOutletFlux(frame, own, given);
-      } else {
-        fu = FaceFlux<kRiemann>(frame, own, given, star);
-      }
-    }
-    if constexpr (kRiemann == kExact) a.exact_star[star_slot] = star ? 1 : 0;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) gap[t][k] = fu.v[k] * (sgn * scale) - fn[t][k];
-  }
-  __syncthreads();  // every read of the F~ columns is done
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-    if (!t_on[t]) continue;
-    const int r = t_f[t] * NFP + t_a[t] * Q + t_b[t];  // face-major gap slot of the node phase
-#pragma unroll
-    for (int k = 0; k < 5; ++k) s_x[t_cell[t] * S::kScratch + k * FPAD + r] = gap[t][k];
-  }
-  __syncthreads();
-
-  // ---- node phase: lifted gaps, 1/det(J), RK stage, store
-  double speed = 0.0;  // |u| + c of the new state, for a fused time step
-  if (node_active) {
-    const double *sg = s_x + ncell * S::kScratch;
-    const double *su = s_u + ncell * 5 * PAD;
-    const double dt = a.case_dt ? a.case_dt[a.cell_case[c0 + ncell]] : a.dt;
-    double outv[5];
+    bool star = kRiemann == kExact ? a.exact_star[point_of(s)] != 0 : false;
+    State ls, rs;
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-      const double *g = sg + k * FPAD;
-      const double corr = fr::LiftedGaps<Q>(g, lt, ni, nj, nk);
-      const double res = (-div[k] - corr) * inv_det;
-      outv[k] = fr::RkOutput(a.stage, res, su[k * PAD + spos], u0v[k], dt);
+      ls.v[k] = left ? own.v[k] : other.v[k];
+      rs.v[k] = left ? other.v[k] : own.v[k];
     }
-    // one basic block of stores: merged into 16-byte stores of the node record
+    State fu;
+    if (kind == kBcSmart) fu = FaceFlux<kRiemann>(n, ls, rs, star);
+    else fu = BoundaryFlux(kind, left, n, left ? ls : rs, left ? rs : ls);
+    if constexpr (kRiemann == kExact) a.exact_star[point_of(s)] = star ? 1 : 0;
+    // left-to-right is the +r direction of this cell unless the roles are swapped
 #pragma unroll
-    for (int k = 0; k < 5; ++k) a.out[base + tid * 5 + k] = outv[k];
+    for (int k = 0; k < 5; ++k) flux[k] = fu.v[k] * along;
+    Pin(flux);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    if (s == Z) {
+#pragma unroll
+      for (int k = 0; k < 5; ++k) flux_z[k] = flux[k];
+      face = later[lane];
+      geometry(0);
+      nb = gather(0);
+      continue;
+    }
+
+  // ---- F~_r = F J*.col(r) at the nodes, contracted: x and z into div in the
+  // node order, y into divy with j in h; and the fluxes lifted
+    const double dg = ops->dg[lane], gp01 = ops->gp01[lane], gp23 = ops->gp23[lane];
+    const int g = s;
+    const int64_t c = g ? c1 : c0;
+    double *const su = lds + g * S::kState;
+    double u0[5] = { 0, 0, 0, 0, 0 };
+    const double inv_det = kCurved ? a.inv_det_node[c * NP + lane] : geo[g][kGeoInvDet];
+    if (a.stage >= 2) {
+#pragma unroll
+      for (int k = 0; k < 5; ++k) u0[k] = __builtin_nontemporal_load(a.u0 + c * (5 * NP) + k * NP + lane);
+    }
+    double col[3][3];
+    if constexpr (kCurved) {
+      const int node[3] = { lane, 16 * m + 4 * h + l, 16 * l + 4 * m + h };
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int e = 0; e < 3; ++e) col[r][e] = a.col_node[((c * 3 + r) * NP + node[r]) * 3 + e];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int e = 0; e < 3; ++e) col[r][e] = geo[g][4 * r + e];
+    }
+    double div[5], divy[5];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      double v[5];
+#pragma unroll
+      for (int k = 0; k < 5; ++k) v[k] = su[k * 79 + (r == 0 ? at_x : (r == 1 ? at_y : at_z))];
+      // contravariant momentum and velocity, and pressure
+      const double inv = FastRcp(v[0]);
+      const double mom = v[1] * col[r][0] + v[2] * col[r][1] + v[3] * col[r][2];
+      double vel = mom * inv;
+      double p = (v[4] - 0.5 * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]) * inv) * kGm1;
+      if (!__all(v[0] > 0 && v[4] >= 0 && p >= 0)) {  // the zeroing rule of types.hpp:195-202,289-301
+        const bool bad = v[0] < 0 || v[4] < 0;
+        const bool vacuum = !bad && v[0] == 0;
+        const bool zero = bad || (!vacuum && p < 0);
+        vel = zero ? 0.0 : (vacuum ? mom : vel);
+        p = zero ? 0.0 : (vacuum ? v[4] : p);
+      }
+#pragma unroll
+      for (int k = 0; k < 5; ++k) {
+        const double fk = k == 0 ? mom : (k == 4 ? (v[4] + p) * vel : v[k] * vel + p * col[r][k == 0 ? 0 : k - 1]);
+        if (r == 0) div[k] = Mfma(gp01, flux[k], Mfma(dg, fk, 0.0));
+        else if (r == 1) divy[k] = Mfma(gp23, flux[k], Mfma(dg, fk, 0.0));
+        else div[k] = Mfma(flux_z[k], g ? gp23 : gp01, Mfma(fk, dg, div[k]));
+      }
+    }
+
+    double uc[5];
+    // y's part to the node order; 1/det(J), RK stage, store
+#pragma unroll
+    for (int k = 0; k < 5; ++k) uc[k] = su[k * 79 + at_x];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int k = 0; k < 5; ++k) su[k * 79 + at_y] = divy[k];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    State out;
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const double sum = div[k] + su[k * 79 + at_x];
+      out.v[k] = fr::RkOutput(a.stage, -sum * inv_det, uc[k], u0[k], dt[g]);
+    }
+    if (g == 0 || c1 != c0) {
+      // the residual is handed out as a column, states stay in planes; streamed,
+      // so that the states which neighbours still gather keep the L2
+      const int64_t to = a.stage == 0 ? (c * NP + lane) * 5 : c * (5 * NP) + lane;
+      const int step = a.stage == 0 ? 1 : NP;
+#pragma unroll
+      for (int k = 0; k < 5; ++k) __builtin_nontemporal_store(out.v[k], a.out + to + k * step);
+    }
     if (a.dt_min_bits) {
-      State nw;
+      // fem.hpp:412-435 on the state just written, as FrHexTimeStepKernel: min
+      // over cells of length / max(1e-5, max over nodes of |u| + c); the bits of
+      // positive doubles order as the doubles do
+      double v = fmax(1e-5, MaxSpeed(out));
 #pragma unroll
-      for (int k = 0; k < 5; ++k) nw.v[k] = outv[k];
-      speed = MaxSpeed(nw);
+      for (int o = 32; o >= 1; o /= 2) v = fmax(v, __shfl_xor(v, o));
+      if (lane == 0)
+        atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(geo[g][kGeoLength] / v));
     }
-  }
-  if (a.dt_min_bits) {
-    // fem.hpp:412-435 on the state just written, as FrHexTimeStepKernel:
-    // min over cells of length / max(1e-5, max over nodes of |u| + c)
-    __syncthreads();  // every read of the LDS states and gaps is done
-    double *s_speed = s_u, *s_cell = s_x;
-    if (node_active) s_speed[tid] = speed;
-    __syncthreads();
-    if (tid < nc) {
-      double vmax = 1e-5;
-      for (int p = 0; p < NP; ++p) vmax = fmax(vmax, s_speed[tid * NP + p]);
-      s_cell[tid] = a.geo[(int64_t)a.geo_id[c0 + tid] * kGeoStride + 16] / vmax;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      double local = 1e300;
-      for (int c = 0; c < nc; ++c) local = fmin(local, s_cell[c]);
-      atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(local));
+    if (turn < Z) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      face = later[(s + 1) * 64 + lane];
+      geometry(s + 1);
+      nb = gather(s + 1);
     }
   }
 }
 
-template <int Q, int Cells, int Threads, int kRiemann, bool kDiag, bool kMixed, bool kOneRound, int kPrefetch,
-          bool kCurved = false>
-__global__ __launch_bounds__(Threads) void FrHexStageKernel(FrHexArgs a, LineTables lt) {
-  __shared__ double lds[Shape<Q, Cells, Threads, kOneRound>::kLdsDoubles];
-  // The line tables are indexed by lane-varying node indices: read from the
-  // kernel arguments they would be vector loads on the critical path of every
-  // pass, so they are staged in LDS once (the body's first barrier orders it).
-  __shared__ LineTables s_lt;
-  constexpr int kTableDoubles = sizeof(LineTables) / sizeof(double);
-  if (threadIdx.x < kTableDoubles)
-    reinterpret_cast<double *>(&s_lt)[threadIdx.x] = reinterpret_cast<const double *>(&lt)[threadIdx.x];
-  int64_t block = LogicalBlock(a.xcd_remap);
-  if (a.tile_order) block = a.tile_order[block];
-  FrHexStageBody<Q, Cells, Threads, kRiemann, kDiag, kMixed, kOneRound, kPrefetch, kCurved>(a, s_lt, block, lds);
+template <int kCells, int kRiemann, bool kCurved>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kRiemann == kExact ? 2 : 4)))
+void FrHexCellKernel(FrHexArgs a, LineTables lt) {
+  __shared__ __attribute__((aligned(16))) double lds[CellShape<kCells>::kLdsDoubles];
+  constexpr int kPerTile = Shape<4>::kCells / kCells;
+  const int64_t block = LogicalBlock(a.xcd_remap);
+  const int64_t tile = a.tile_order ? a.tile_order[block / kPerTile] : block / kPerTile;
+  const int64_t c = tile * Shape<4>::kCells + block % kPerTile * kCells;
+  if (c >= a.n_cells) return;
+  FrCellBody<kCells, kRiemann, kCurved>(a, lt, c, lds);
 }
 
-// Single-mesh launch shape per Q: one thread per solution point.  Q = 4 and
-// 5 run on 128-thread workgroups (2 cells and 1 cell): the same 3 waves per
-// SIMD as 256-thread ones, with each barrier waiting on two wavefronts
-// instead of four (Q = 4: 0.93 against 0.96 ms per stage at 64^3; Q = 3 as
-// 4 cells on 128 threads leaves 20 threads idle and measured no better).  At Q = 4
-// the face tasks (96 per cell) fill two slots in half of the wavefronts; 96
-// threads per cell (one task each) measured slower on MI355X, since the extra
-// wavefronts idle through the volume passes and occupy wave slots that other
-// workgroups would fill.
-template <int Q> struct StageTile {
-  static constexpr int kCells = Q == 4 ? 2 : (Q == 5 ? 1 : Shape<Q>::kCells);
-  static constexpr int kThreads = (Q == 4 || Q == 5) ? 128 : 256;
-  static constexpr bool kOneRound = Q >= 3;  // at Q = 2 the column space would cost a workgroup per CU
-  // face tasks whose neighbour lines are issued before the passes: one, as
-  // the registers of the three-waves-per-SIMD budget allow
-  static constexpr int kPrefetch = 1;
-};
+// Tile variants of the persistent batched launch: a work item is 1, 2 or 4
+// consecutive blocks of Shape<Q>::kCells cells.
+constexpr int TileBlocks(int tile) { return 1 << tile; }
 
-// Tile variants per Q (cells per workgroup) that the batched launch and its
-// autotuner choose from.
-template <int Q, int V> struct TileOf;
-template <> struct TileOf<2, 0> { static constexpr int kCells = 32; };
-template <> struct TileOf<2, 1> { static constexpr int kCells = 16; };
-template <> struct TileOf<2, 2> { static constexpr int kCells = 8; };
-template <> struct TileOf<3, 0> { static constexpr int kCells = 9; };
-template <> struct TileOf<3, 1> { static constexpr int kCells = 4; };
-template <> struct TileOf<3, 2> { static constexpr int kCells = 2; };
-template <> struct TileOf<4, 0> { static constexpr int kCells = 4; };
-template <> struct TileOf<4, 1> { static constexpr int kCells = 2; };
-template <> struct TileOf<4, 2> { static constexpr int kCells = 1; };
-
-template <int Q, int V>
-constexpr int TileLds() { return Shape<Q, TileOf<Q, V>::kCells, 256, (Q >= 3)>::kLdsDoubles; }
-
-// One out-of-line body per (Q, tile): each is register-allocated on its own
-// within the kernel's 3-waves-per-SIMD budget, where nine inlined bodies
-// would share one allocation and spill.  Q >= 3 bodies pass all three F~
-// columns through LDS in one round, as the single-mesh launch does.
-template <int Q, int V, int kRiemann, bool kMixed>
-__device__ __noinline__ void BatchBody(const FrHexBatchGroup *g, int64_t block, double *lds) {
-  FrHexStageBody<Q, TileOf<Q, V>::kCells, 256, kRiemann, true, kMixed, (Q >= 3), 1>(g->args, g->lt, block, lds);
-}
-
+// One out-of-line body per Q: each is register-allocated on its own within the
+// kernel's budget, where the inlined bodies would share one allocation.
 template <int Q, int kRiemann, bool kMixed>
-__device__ __forceinline__ void BatchItem(const FrHexBatchGroup &g, int64_t block, double *lds) {
-  switch (g.tile) {
-  case 0: BatchBody<Q, 0, kRiemann, kMixed>(&g, block, lds); break;
-  case 1: BatchBody<Q, 1, kRiemann, kMixed>(&g, block, lds); break;
-  default: BatchBody<Q, 2, kRiemann, kMixed>(&g, block, lds); break;
-  }
+__device__ __noinline__ void BatchBody(const FrHexBatchGroup *g, int64_t block, double *lds) {
+  FrLineBody<Q, kRiemann, kMixed, false>(g->args, g->lt, block, lds);
 }
 
 // Persistent batched pass: workgroup w processes the contiguous item range
 // [w * n_items / W, (w + 1) * n_items / W) of the work list (blocks of all
 // degree groups in order), so consecutive blocks -- and their neighbour
-// cells -- stay in one XCD's L2.  LDS is sized at launch for the largest tile
+// cells -- stay in one XCD's L2.  LDS is sized at launch for the largest block
 // in use.
 template <int kRiemann, bool kMixed>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void FrHexBatchKernel(FrHexBatchArgs b) {
+__global__ __launch_bounds__(Shape<4>::kThreads) __attribute__((amdgpu_waves_per_eu(kRiemann == kExact ? 2 : 3))) void FrHexBatchKernel(FrHexBatchArgs b) {
   extern __shared__ double lds[];
   const int64_t w = blockIdx.x, nw = gridDim.x;
   const int64_t begin = w * b.n_items / nw, end = (w + 1) * b.n_items / nw;
@@ -535,14 +807,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void F
     // field is fetched with scalar loads
     while (gi + 1 < b.n_groups && item >= b.group[gi + 1].first_item) ++gi;
     const FrHexBatchGroup &g = b.group[gi];
-    const int64_t block = item - g.first_item;
-    switch (g.q) {
-    case 2: BatchItem<2, kRiemann, kMixed>(g, block, lds); break;
-    case 3: BatchItem<3, kRiemann, kMixed>(g, block, lds); break;
-    default: BatchItem<4, kRiemann, kMixed>(g, block, lds); break;
+    const int blocks = TileBlocks(g.tile);
+    for (int v = 0; v < blocks; ++v) {
+      const int64_t block = (item - g.first_item) * blocks + v;
+      switch (g.q) {
+      case 2: BatchBody<2, kRiemann, kMixed>(&g, block, lds); break;
+      case 3: BatchBody<3, kRiemann, kMixed>(&g, block, lds); break;
+      default: BatchBody<4, kRiemann, kMixed>(&g, block, lds); break;
+      }
+      __syncthreads();  // the next block reuses the LDS buffers
     }
-    __syncthreads();  // the next item reuses the LDS buffers
   }
+}
+
+// Column layout [cell][node][5] <-> the kernels' planes [cell][5][node], one
+// thread per value of the planes.
+template <bool kToPlanes>
+__global__ __launch_bounds__(256) void FrLayoutKernel(const double *in, double *out, int np, int64_t n) {
+  const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (w >= n) return;
+  const int64_t c = w / (5 * np);
+  const int r = (int)(w - c * (5 * np)), k = r / np, node = r - k * np;
+  const int64_t col = (c * np + node) * 5 + k;
+  if constexpr (kToPlanes) out[w] = in[col];
+  else out[col] = in[w];
 }
 
 __global__ void ResetTimeStepBitsKernel(unsigned long long *bits) {
@@ -561,10 +849,10 @@ __global__ __launch_bounds__(256) void FrHexTimeStepKernel(const double *u, cons
     for (int p = 0; p < NP; ++p) {
       State s;
 #pragma unroll
-      for (int k = 0; k < 5; ++k) s.v[k] = uc[p * 5 + k];
+      for (int k = 0; k < 5; ++k) s.v[k] = uc[k * NP + p];
       vmax = fmax(vmax, MaxSpeed(s));
     }
-    local = fmin(local, geo[(int64_t)geo_id[c] * kGeoStride + 16] / vmax);
+    local = fmin(local, geo[(int64_t)geo_id[c] * kGeoStride + kGeoLength] / vmax);
   }
   s_min[threadIdx.x] = local;
   __syncthreads();
@@ -575,31 +863,42 @@ __global__ __launch_bounds__(256) void FrHexTimeStepKernel(const double *u, cons
   if (threadIdx.x == 0) atomicMin(dt_min_bits, (unsigned long long)__double_as_longlong(s_min[0]));
 }
 
+// Q = 4: two cells per wavefront save a quarter of the flux points' lanes but
+// halve the wavefronts, so a mesh that does not fill the chip with one cell per
+// wavefront (256 CUs, 16 wavefronts each) is better served that way.  Measured,
+// one against two cells, us per pass: 12^3 11.1 / 12.6, 16^3 16.4 / 16.7, 18^3
+// 21.5 / 21.0, 20^3 26.9 / 25.5, 32^3 90.5 / 84.5, 64^3 638 / 595.  The exact
+// solver keeps one: two spill (24^3 250 us against 218).
+constexpr int64_t kPairCells = 4096;
+
 template <int Q, int R>
 hipError_t Launch(const FrHexArgs &args, const LineTables &lt, hipStream_t stream) {
-  constexpr int C = StageTile<Q>::kCells, W = StageTile<Q>::kThreads;
-  constexpr bool O = StageTile<Q>::kOneRound;
-  constexpr int PF = StageTile<Q>::kPrefetch;
-  int64_t blocks = (args.n_cells + C - 1) / C;
-  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)blocks), block(W);
-  if (args.curved) {
-    if (args.mixed || args.diag_metric) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((FrHexStageKernel<Q, C, W, R, false, false, O, PF, true>), grid, block, 0, stream, args, lt);
-    return hipGetLastError();
+  constexpr int C = Shape<Q>::kCells;
+  const int64_t blocks = (args.n_cells + C - 1) / C;
+  if (blocks > 0x7fffffff || (args.curved && args.mixed)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)blocks), block(Shape<Q>::kThreads);
+  if constexpr (Q == 4) {
+    if (!args.mixed) {
+      if (blocks * C > 0x7fffffff || !args.cell_ops) return hipErrorInvalidValue;
+      const bool pair = R != kExact && args.n_cells > kPairCells;
+      const dim3 cells((unsigned)(blocks * (pair ? C / 2 : C))), wave(64);
+      if constexpr (R != kExact) {
+        if (pair && args.curved) hipLaunchKernelGGL((FrHexCellKernel<2, R, true>), cells, wave, 0, stream, args, lt);
+        else if (pair) hipLaunchKernelGGL((FrHexCellKernel<2, R, false>), cells, wave, 0, stream, args, lt);
+      }
+      if (!pair) {
+        if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<1, R, true>), cells, wave, 0, stream, args, lt);
+        else hipLaunchKernelGGL((FrHexCellKernel<1, R, false>), cells, wave, 0, stream, args, lt);
+      }
+      return hipGetLastError();
+    }
   }
-  if (args.mixed) {
-    if (args.diag_metric) {
-      hipLaunchKernelGGL((FrHexStageKernel<Q, C, W, R, true, true, O, PF>), grid, block, 0, stream, args, lt);
-    } else {
-      hipLaunchKernelGGL((FrHexStageKernel<Q, C, W, R, false, true, O, PF>), grid, block, 0, stream, args, lt);
-    }
+  if (args.curved) {
+    hipLaunchKernelGGL((FrHexStageKernel<Q, R, false, true>), grid, block, 0, stream, args, lt);
+  } else if (args.mixed) {
+    hipLaunchKernelGGL((FrHexStageKernel<Q, R, true, false>), grid, block, 0, stream, args, lt);
   } else {
-    if (args.diag_metric) {
-      hipLaunchKernelGGL((FrHexStageKernel<Q, C, W, R, true, false, O, PF>), grid, block, 0, stream, args, lt);
-    } else {
-      hipLaunchKernelGGL((FrHexStageKernel<Q, C, W, R, false, false, O, PF>), grid, block, 0, stream, args, lt);
-    }
+    hipLaunchKernelGGL((FrHexStageKernel<Q, R, false, false>), grid, block, 0, stream, args, lt);
   }
   return hipGetLastError();
 }
@@ -628,35 +927,31 @@ hipError_t LaunchFrHexStage(int q, int riemann, const FrHexArgs &args, const Lin
   }
 }
 
-int FrHexTileLdsBytes(int q, int tile) {
-  static const int lds[3][3] = { { TileLds<2, 0>(), TileLds<2, 1>(), TileLds<2, 2>() },
-                                 { TileLds<3, 0>(), TileLds<3, 1>(), TileLds<3, 2>() },
-                                 { TileLds<4, 0>(), TileLds<4, 1>(), TileLds<4, 2>() } };
-  if (q < 2 || q > 4 || tile < 0 || tile > 2) return 0;
-  return lds[q - 2][tile] * (int)sizeof(double);
-}
-
 int FrHexStageTileCells(int q) {
   switch (q) {
-  case 2: return StageTile<2>::kCells;
-  case 3: return StageTile<3>::kCells;
-  case 4: return StageTile<4>::kCells;
-  case 5: return StageTile<5>::kCells;
-  case 6: return StageTile<6>::kCells;
+  case 2: return Shape<2>::kCells;
+  case 3: return Shape<3>::kCells;
+  case 4: return Shape<4>::kCells;
+  case 5: return Shape<5>::kCells;
+  case 6: return Shape<6>::kCells;
   default: return 0;
   }
 }
 
-int FrHexTileCells(int q, int tile) {
-  static const int cells[3][3] = { { 32, 16, 8 }, { 9, 4, 2 }, { 4, 2, 1 } };
+int FrHexTileLdsBytes(int q, int tile) {
   if (q < 2 || q > 4 || tile < 0 || tile > 2) return 0;
-  return cells[q - 2][tile];
+  return (int)sizeof(double) * (q == 2 ? Shape<2>::kLdsDoubles : (q == 3 ? Shape<3>::kLdsDoubles : Shape<4>::kLdsDoubles));
+}
+
+int FrHexTileCells(int q, int tile) {
+  if (q < 2 || q > 4 || tile < 0 || tile > 2) return 0;
+  return FrHexStageTileCells(q) * TileBlocks(tile);
 }
 
 hipError_t LaunchFrHexBatch(int riemann, bool mixed, const FrHexBatchArgs &args, int n_workgroups,
                             hipStream_t stream) {
   if (args.n_groups < 1 || args.n_groups > kMaxBatchGroups || n_workgroups < 1) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)n_workgroups), block(256);
+  const dim3 grid((unsigned)n_workgroups), block(Shape<4>::kThreads);
   const size_t lds = (size_t)args.max_tile_lds;
   switch (riemann) {
 #define MCFD_BATCH_CASE(R)                                                                        \
@@ -676,7 +971,7 @@ int FrHexBatchResidentWorkgroups(int riemann, bool mixed, int lds_bytes) {
   hipError_t e = hipErrorInvalidValue;
   switch (riemann * 2 + (mixed ? 1 : 0)) {
 #define MCFD_OCC(R, M) \
-  case R * 2 + M: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<R, M>, 256, lds_bytes); break;
+  case R * 2 + M: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<R, M>, Shape<4>::kThreads, lds_bytes); break;
   MCFD_OCC(kExact, 0) MCFD_OCC(kExact, 1) MCFD_OCC(kHllc, 0) MCFD_OCC(kHllc, 1) MCFD_OCC(kRoe, 0) MCFD_OCC(kRoe, 1)
 #undef MCFD_OCC
   default: break;
@@ -686,6 +981,18 @@ int FrHexBatchResidentWorkgroups(int riemann, bool mixed, int lds_bytes) {
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return 0;
   return std::max(1, per_cu) * cus;
+}
+
+hipError_t LaunchFrLayout(bool to_planes, const double *in, double *out, int np, int64_t n_cells, hipStream_t stream) {
+  const int64_t n = n_cells * np * 5, blocks = (n + 255) / 256;
+  if (blocks < 1) return hipSuccess;
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
+  if (to_planes) {
+    hipLaunchKernelGGL(FrLayoutKernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream, in, out, np, n);
+  } else {
+    hipLaunchKernelGGL(FrLayoutKernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, in, out, np, n);
+  }
+  return hipGetLastError();
 }
 
 hipError_t LaunchResetTimeStepBits(unsigned long long *bits, hipStream_t stream) {

@@ -12,54 +12,86 @@ constexpr int kMaxQ = 6;
 constexpr int kMaxBatchGroups = 4;
 
 // 1-D tables of the solution-point line (Q points):
-//   d[i][m]   = l_m'(x_i)          (Lagrange derivative matrix)
-//   lend[e][m] = l_m(-1), l_m(+1)   (extrapolation to the line ends)
-//   gp[e][m]  = g_L'(x_m), g_R'(x_m) (Vincent correction derivatives)
+//   dg[i][m]  = l_m'(x_i) - g_L'(x_i) l_m(-1) - g_R'(x_i) l_m(+1): the derivative
+//               of the line's flux with the line ends' own flux values already
+//               lifted out, so that only the upwind fluxes are left to lift
+//   end[m]    = l_m(-1), the extrapolation to a line end from the node next to it
+//               inwards (the points are symmetric: l_{Q-1-m}(+1) = l_m(-1))
+//   gp[e][i]  = g_L'(x_i), g_R'(x_i) (Vincent correction derivatives)
+// and for the mixed form, which contracts deviations in FP32,
+//   d[i][m]   = l_m'(x_i), lend[e][m] = l_m(-1), l_m(+1).
 struct LineTables {
-  double d[kMaxQ][kMaxQ];
-  double lend[2][kMaxQ];
+  double dg[kMaxQ][kMaxQ];
+  double end[kMaxQ];
   double gp[2][kMaxQ];
+  float d[kMaxQ][kMaxQ];
+  float lend[2][kMaxQ];
 };
 
-// Per-cell affine geometry record (20 doubles):
-//   [0..8]  J* = det(J) J^{-1} (row-major, F~ = F J*)
-//   [9]     1 / det(J)
-//   [10..15] signed face scale +-|J*.col(normal dir)| of local faces 0..5
-//   [16]    length = cbrt(volume) / 2
-constexpr int kGeoStride = 20;
-constexpr int kFrameStride = 6;  // n, t
-// Per-node record of a trilinear cell: J* (9, as above), 1 / det(J).
-constexpr int kNodeGeoStride = 10;
+// Per-cell affine geometry record (16 doubles):
+//   [4 r + e]  e = 0..2: J*.col(r), J* = det(J) J^{-1} (F~_r = sum_e F_e [4 r + e]);
+//              e = 3: its length, the face scale of the two faces normal to r
+//   [12]       1 / det(J)
+//   [13]       length = cbrt(volume) / 2
+constexpr int kGeoStride = 16;
+constexpr int kGeoInvDet = 12, kGeoLength = 13;
+constexpr int kNormalStride = 4;  // unit normal, pad
 
+// Per cell face: the neighbour (or -(1 + boundary tag)); the neighbour's node
+// behind in-face point (a, b), m nodes in from the face, as
+// first + sa a + sb b + sm m, packed first | sa << 8 | sb << 16 | sm << 24
+// (bytes, the strides signed); the unit normal's index, pointing from the
+// pair's left to its right state, << 1 | swap; the boundary face index (-1
+// for interior faces).  The left state is that of the cell whose upper (+1)
+// end the face is; where the two cells do not agree on that (neighbours turned
+// against each other), and always for the exact solver, whose state has a
+// sign, it is the holder's, and `swap` marks the cell whose place that changes.
+struct alignas(16) FrFace {
+  int32_t nbr, gather, normal, bface;
+};
+
+// Lane operators of the one-wavefront-per-cell kernel (Q = 4), lane = 16 h + 4 m + l:
+struct CellOps {
+  double dg[64];     // dg[l][h]
+  double end01[64];  // extrapolation to the lower (l = 0) and upper (l = 1) line end from node h, 0 for l = 2, 3
+  double end23[64];  // the same for l = 2, 3
+  double gp01[64];   // g_L'(x_l) (h = 0) and g_R'(x_l) (h = 1), 0 for h = 2, 3
+  double gp23[64];   // the same for h = 2, 3
+};
+
+// States live in planes, [cell][5][node]: a wavefront's lines are then read
+// 8 bytes per lane from consecutive addresses, where the column layout
+// [cell][node][5] of the interface spreads them over 40 (LaunchFrLayout
+// converts).  The residual is written as a column.
 struct FrHexArgs {
+  const CellOps *cell_ops;  // lane operators of the one-wavefront-per-cell kernel (Q = 4)
   const double *us;      // state of this stage, also read for neighbour traces
   const double *u0;      // U0 for RK stages 2 and 3
-  double *out;           // residual (stage 0) or next state
-  const int32_t *nbr;    // [cell][6]: neighbour cell, or -(1 + boundary tag)
-  const int32_t *finfo;  // [cell][6]: frame id << 7 | holder << 6 | orient << 3 | neighbour face
+  double *out;           // residual (stage 0, a column) or next state
+  const FrFace *faces;   // [cell][6]
   const int32_t *geo_id; // [cell]
-  const double *geo;     // [geo][kGeoStride]
-  const double *frames;  // [frame][kFrameStride]; curved: [face][a * Q + b][kFrameStride]
-  // curved (trilinear) meshes: [cell][node][kNodeGeoStride] and the signed
-  // flux-point scales [cell][local face][a * Q + b]; null otherwise
-  const double *geo_node;
-  const double *fscale;
+  const double *geo;     // [geo][kGeoStride]; curved: [cell], the length only
+  const double *normals; // [normal][kNormalStride] (affine cells)
+  // curved (trilinear) meshes: J*.col(r) of every node [cell][r][node][3],
+  // 1 / det(J) [cell][node], and per cell flux point its unit normal (left to
+  // right) and face scale [cell][local face][a * Q + b][4]; null otherwise
+  const double *col_node;
+  const double *inv_det_node;
+  const double *face_point;
   const int32_t *bc_kind;   // [tag]: BcKind (euler.hpp)
   const double *bc_state;   // [tag][5] given state (conservative, or the subsonic parameters)
   // If set, the given state of every boundary flux point instead:
-  // [boundary face][a * Q + b][5], with bface_of [cell][6] the boundary face
-  // index of each boundary cell face (the tag's boundary function at the stage time)
+  // [boundary face][a * Q + b][5] (the tag's boundary function at the stage time)
   const double *bc_point_state;
-  const int32_t *bface_of;
   const int32_t *cell_case; // [cell] case index, or null (one time step for all cells)
   const double *case_dt;    // [case] time step when cell_case is set
   int64_t n_cells;
   double dt;
   int32_t stage;         // 0 residual, 1..3 SSP-RK3 stage
   int32_t xcd_remap;     // remap block ids so each XCD sweeps a contiguous range
-  int32_t diag_metric;   // every J* is diagonal (axis-aligned cells)
+  int32_t any_swap;      // some FrFace has its swap bit set
   int32_t mixed;         // FP32 flux-column contractions (mixed-precision form)
-  int32_t curved;        // per-node metrics and per-point scales and frames
+  int32_t curved;        // per-node metrics and per-point normals and scales
   const int32_t *tile_order;  // [tile]: tile swept by logical block b (spatial locality), or null
   // If set, the time-step reduction of LaunchFrHexTimeStep over the state this
   // pass writes is folded into *dt_min_bits (same arithmetic, no extra pass).
@@ -104,6 +136,8 @@ hipError_t LaunchFrHexBatch(int riemann, bool mixed, const FrHexBatchArgs &args,
 // given dynamic LDS (0 on failure).
 int FrHexBatchResidentWorkgroups(int riemann, bool mixed, int lds_bytes);
 
+// Column layout [cell][node][5] -> planes [cell][5][node] (to_planes), or back.
+hipError_t LaunchFrLayout(bool to_planes, const double *in, double *out, int np, int64_t n_cells, hipStream_t stream);
 // Per-cell minimum of length / max wave speed over the solution points
 // (spatial/fem.hpp:417-435), reduced to one double in *dt_min (device).
 // *bits = the ordered bits of 1e300, the start of a time-step reduction.

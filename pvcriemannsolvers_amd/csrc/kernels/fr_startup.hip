@@ -20,15 +20,15 @@ __global__ __launch_bounds__(256) void FrAverageKernel(double *u, const double *
   if (t >= n_cells * 5) return;
   const int64_t cell = t / 5;
   const int k = (int)(t - cell * 5);
-  double *uc = u + cell * np * 5;
+  double *uc = u + (cell * 5 + k) * np;
   double sum = 0, volume = 0;
   for (int q = 0; q < np; ++q) {
     const double w = MulRn(w_local[q], det[cell * np + q]);
-    sum = AddRn(sum, MulRn(uc[q * 5 + k], w));
+    sum = AddRn(sum, MulRn(uc[q], w));
     volume = AddRn(volume, w);
   }
   const double average = sum / volume;
-  for (int q = 0; q < np; ++q) uc[q * 5 + k] = average;
+  for (int q = 0; q < np; ++q) uc[q] = average;
 }
 
 __global__ __launch_bounds__(256) void FrMajorityKernel(const double *u, double *value, int32_t *failed,
@@ -37,13 +37,13 @@ __global__ __launch_bounds__(256) void FrMajorityKernel(const double *u, double 
   if (t >= n_cells * 5) return;
   const int64_t cell = t / 5;
   const int k = (int)(t - cell * 5);
-  const double *uc = u + cell * np * 5;
+  const double *uc = u + (cell * 5 + k) * np;
   bool found = false;
   double v = 0;
   for (int q = 0; q < np && !found; ++q) {
-    const double x = uc[q * 5 + k];
+    const double x = uc[q];
     int count = 0;
-    for (int r = 0; r <= q; ++r) count += uc[r * 5 + k] == x;
+    for (int r = 0; r <= q; ++r) count += uc[r] == x;
     if (count * 2 > np) {
       found = true;
       v = x;
@@ -56,9 +56,7 @@ __global__ __launch_bounds__(256) void FrMajorityKernel(const double *u, double 
 __global__ __launch_bounds__(256) void FrSetNodesKernel(double *u, const double *value, int64_t n_cells, int np) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= n_cells * np * 5) return;
-  const int64_t cell = t / (np * 5);
-  const int k = (int)(t % 5);
-  u[t] = value[cell * 5 + k];
+  u[t] = value[t / np];
 }
 
 dim3 Blocks(int64_t n) { return dim3((unsigned)((n + 255) / 256)); }

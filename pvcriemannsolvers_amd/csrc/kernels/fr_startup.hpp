@@ -9,7 +9,7 @@
 
 namespace mcfd {
 
-// u [cell][np][5] in place: every node takes the cell average with the
+// u [cell][5][np] in place: every node takes the cell average with the
 // global weights w_local[q] * det[cell * np + q] (det(J) at each node).
 hipError_t LaunchFrAverage(double *u, const double *w_local, const double *det, int64_t n_cells, int np,
                            hipStream_t stream);
@@ -17,7 +17,7 @@ hipError_t LaunchFrAverage(double *u, const double *w_local, const double *det, 
 // a component has none (value then 0).
 hipError_t LaunchFrMajority(const double *u, double *value, int32_t *failed, int64_t n_cells, int np,
                             hipStream_t stream);
-// u [cell][np][5] = value [cell][5] at every node.
+// u [cell][5][np] = value [cell][5] at every node.
 hipError_t LaunchFrSetNodes(double *u, const double *value, int64_t n_cells, int np, hipStream_t stream);
 
 }  // namespace mcfd

@@ -1,0 +1,65 @@
+"""FR kernels at the edges of their tiles: cells that do not fill a workgroup
+(16, 7, 4, 3, 1 cells for degrees 1..5), single cells, the last cell of a mesh
+whose cells go two to a wavefront (degree 3, more than 4096 cells), and
+neighbours turned against each other, whose lines are gathered in every
+direction.  Tolerances as in tests/test_fr_gpu.py: the same FP64 formulas summed
+in another order, 1e-12 relative (Roe, HLLC), 1e-7 for the exact solver's
+stopping rule; the mixed form's residual 1e-5 of its max norm.
+"""
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+from pvcriemannsolvers_amd import meshgen, spatial
+from test_boundary_cpu import rotate_cells
+from test_fr_gpu import RIEMANN, TOL, conservative, density_wave, make_pair, rel
+
+pytestmark = pytest.mark.gpu
+
+LEFT, RIGHT = conservative(1.0, (0.1, 0, 0), 1.0), conservative(0.125, (0, 0, 0), 0.1)
+BCS = [("smart", LEFT), ("smart", RIGHT)] + [("inviscid_wall", None)] * 4
+EDGES = [(1, 1), (1, 15), (1, 16), (1, 17), (2, 6), (2, 7), (2, 8), (3, 1), (3, 3), (3, 5),
+         (4, 2), (4, 3), (4, 4), (5, 1), (5, 3)]
+
+
+@pytest.mark.parametrize("degree,cells", EDGES)
+@pytest.mark.parametrize("riemann", ["roe", "hllc", "exact"])
+def test_tile_edges_turned_cells(degree, cells, riemann):
+    mesh = rotate_cells(meshgen.box_hex(cells, 1, 1, hi=(1.0, 0.1, 0.1), shuffle_seed=cells), degree)
+    o, g = make_pair(mesh, degree, riemann, BCS)
+    u = density_wave(o.node_coords(), seed=cells)
+    g.set_solution_column(u.reshape(-1))
+    assert rel(g.get_residual_column(), o.residual(u).reshape(-1)) < TOL[riemann]
+    np.testing.assert_array_equal(g.get_solution_column(), u.reshape(-1))
+    g.close()
+
+
+@pytest.mark.parametrize("degree", [1, 2, 3, 4, 5])
+def test_mixed_turned_cells(degree):
+    mesh = rotate_cells(meshgen.box_hex(5, 3, 3, periodic=(True,) * 3, shuffle_seed=3), 17)
+    o = ol.FrOracle(mesh, q=degree + 1, riemann=RIEMANN["roe"])
+    g = spatial.FiniteElement(mesh, degree=degree, riemann="roe", precision="mixed")
+    u = density_wave(o.node_coords(), seed=7)
+    g.set_solution_column(u.reshape(-1))
+    assert rel(g.get_residual_column(), o.residual(u).reshape(-1)) < 1e-5
+    g.close()
+
+
+@pytest.mark.parametrize("riemann,jitter", [("roe", 0.0), ("hllc", 0.0), ("roe", 0.2), ("exact", 0.0)])
+def test_two_cells_per_wavefront(riemann, jitter):
+    """4335 cells: the last wavefront has one; a step and the time step folded into it.
+    (Spacing 1/16, so that cell sizes carry no rounding of the coordinates: with
+    1/17 that alone moves this residual by 3e-12.)"""
+    mesh = rotate_cells(meshgen.box_hex(17, 17, 15, hi=(17 / 16, 17 / 16, 15 / 16), periodic=(True,) * 3,
+                                        jitter=jitter, seed=4, shuffle_seed=5), 6)
+    o, g = make_pair(mesh, 3, riemann)
+    u = density_wave(o.node_coords(), seed=8)
+    g.set_solution_column(u.reshape(-1))
+    assert rel(g.get_residual_column(), o.residual(u).reshape(-1)) < TOL[riemann]
+    dt = g.get_time_step(0.1)
+    ref = o.rk3(u.reshape(-1), dt, n_steps=1)
+    g.rk3_update(0.0, dt)
+    assert rel(g.get_solution_column(), ref) < TOL[riemann]
+    expect = o.time_step(ref, 0.1)
+    assert abs(g.get_time_step(0.1) - expect) <= (1e-12 if riemann != "exact" else 1e-7) * expect
+    g.close()
