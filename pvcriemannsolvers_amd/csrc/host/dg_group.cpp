@@ -394,14 +394,16 @@ void DgGroup::Upload(hipStream_t stream) {
   basis.Upload(h_basis, stream);
   geo.Upload(h_geo, stream);
   face_rec.Upload(h_faces, stream);
-  face_cells.Upload(h_face_cells, stream);
-  fhat.Allocate(faces.size() * nfp * 5);
   if (riemann == MCFD_RIEMANN_EXACT) {
+    face_cells.Upload(h_face_cells, stream);
+    fhat.Allocate(faces.size() * nfp * 5);
     exact_star.Allocate(faces.size() * nfp);
     Check(hipMemsetAsync(exact_star.ptr, 0, faces.size() * nfp, stream), "memset");
   }
   bc_state.Upload(h_bc_state, stream);
-  finfo.Upload(h_finfo, stream);
+  h_face_info.resize(h_finfo.size());
+  for (size_t i = 0; i < h_finfo.size(); ++i) h_face_info[i] = int2{ h_finfo[i], h_nbr[i] };
+  finfo.Upload(h_face_info, stream);
   bc_kind.Upload(h_bc_kind, stream);
   h_tables.assign(1, tables);
   tables_d.Upload(h_tables, stream);

@@ -1,31 +1,40 @@
 // Modal DG stage kernels for affine hexahedra and tetrahedra (gfx950).
 //
-// One stage pass is two launches.
+// One stage pass is one launch of DgModalStageKernel (for the exact solver two):
+// a workgroup of 256 threads owns G cells; each cell has T = NQ + NF * NFP point
+// tasks (its volume quadrature points and the quadrature points of its faces),
+// one thread per task, volume tasks of all G cells first.
+//   phase 0  the cells' Taylor coefficients, geometry and Gram-Schmidt factors
+//            are staged in LDS; a face task meanwhile evaluates the neighbour's
+//            trace from the neighbour's Taylor coefficients in global memory;
+//   phase 1  volume task: state u = Ct T(y) at the point, flux matrix times the
+//            global weight -> LDS;  face task: own trace, upwind or boundary
+//            flux, -/+ w Fhat and the point's offset Y -> LDS;
+//   phase 2  one wavefront: the Taylor moments Rt, R = Rt S^T, the SSP-RK3
+//            combination (temporal/rk.hpp:31-49 operation order), the new state's
+//            Taylor coefficients for the next pass (and, with a limiter, the
+//            WENO detector's record of the new state), and (optional) the
+//            time-step reduction of the new state.
+// Both cells of a face solve it, from the same two traces formed by the same
+// operations, so the scheme stays conservative without atomics.  That costs the
+// flux twice, and saves writing it once and reading it twice (1.4 KB of a P = 2
+// tetrahedron's 3.4 KB per pass) and a launch.  The exact solver, an iteration
+// of many times an approximate flux, is evaluated once per face point instead, by
+// DgFaceFluxKernel into fhat [face][point][5].
 //
-// DgFaceFluxKernel, one thread per face quadrature point: the holder's and
-// the sharer's traces from their Taylor coefficients, the Riemann or boundary
-// flux, times the weight -> fhat [face][point][5].  Each face is evaluated
-// once, so its two cells read the same flux and the scheme stays
-// conservative without atomics.
-//
-// DgModalStageKernel, a workgroup of 256 threads owning G cells; each cell
-// has T = NQ + NF * NFP point tasks (its volume quadrature points and the
-// quadrature points of its faces), one thread per task, volume tasks of all
-// G cells first.
-//   phase 0  the cells' Taylor coefficients and geometry are staged in LDS;
-//            the Gram-Schmidt factors and the state / U0 of phase 3 are
-//            loaded at the same time, so one round trip serves the pass;
-//   phase 1  volume task: state u = Ct T(y) at the point, flux matrix times
-//            the global weight -> LDS;  face task: -/+ w Fhat read from fhat
-//            and the point's offset Y -> LDS;
-//   phase 2  the Taylor moments Rt: a group of lanes per (cell, component),
-//            each lane over a subset of the cell's tasks, summed by DPP;
-//   phase 3  one thread per (cell, basis function, component): R = Rt S^T,
-//            the SSP-RK3 combination (temporal/rk.hpp:31-49 operation order)
-//            and the store;
-//   phase 4  the new state's Taylor coefficients for the next pass (and,
-//            with a limiter, the WENO detector's record of the new state);
-//   phase 5  (optional) the time-step reduction of the new state.
+// What bounds it: no unit is full (P = 2 tetrahedra: FP64 issue 45 %, vector memory
+// 59 %, LDS 37 %, HBM at 56 % of its copy rate); each workgroup passes through three
+// dependent phases, and 4 to 5 of them fit in a CU's LDS.  Moments by one
+// wavefront with 60 lanes in use take 600 instructions where eight lanes per
+// (cell, component) in all four took 4 x 430.  us per pass, against one launch
+// for the faces and one for the cells with the moments in all wavefronts:
+// 146k P = 2 tetrahedra (Roe) 256 -> 195, the four-quadrant problem's 221k (HLLC,
+// with the limiter) 507 -> 417, 750 tetrahedra 15.5 -> 10.2, 64k P = 2 hexahedra
+// 208 -> 157, 83k P = 1 tetrahedra 83 -> 68; the same cell pass after a face
+// pass: 227, 467, 13.6, 179 and 78.  Measured and no better: the neighbours'
+// coefficients loaded once per face and handed round through LDS (a third of the
+// vector memory work, 200), 5 wavefronts per SIMD (200), moments on two
+// wavefronts (212), 3 cells per workgroup (215).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -39,8 +48,8 @@ namespace {
 // LDS record of one volume task: the weighted flux matrix as F[d][k] (15),
 // a pad, then the point's offset y (3) from kSlotY.  A face task: the
 // weighted flux (5), then y (3).
-constexpr int kSlot = 20;
-constexpr int kSlotY = 16;
+constexpr int kSlot = 19;
+constexpr int kSlotY = 15;
 constexpr int kFaceSlot = 9;
 
 template <bool kHex, int P>
@@ -82,6 +91,41 @@ __device__ __forceinline__ State EvalTaylor(const double *ct, const double *y) {
   return u;
 }
 
+// EvalTaylor in two halves, so that not all 50 coefficients of P = 2 are in
+// registers at once, which costs a wavefront per SIMD, and in 16-byte loads.
+template <int P>
+__device__ __forceinline__ State TraceAt(const double *ct, const double *y) {
+  double c[30];
+  auto load = [&](const double *from, int n) {
+#pragma unroll
+    for (int i = 0; i < n; i += 2) {
+      const double2 v = *reinterpret_cast<const double2 *>(from + i);
+      c[i] = v.x;
+      c[i + 1] = v.y;
+    }
+  };
+  load(ct, 20);
+  State u;
+#pragma unroll
+  for (int k = 0; k < 5; ++k)
+    u.v[k] = __fma_rn(c[15 + k], y[2], __fma_rn(c[10 + k], y[1], __fma_rn(c[5 + k], y[0], c[k])));
+  if constexpr (P >= 2) {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) asm volatile("" : "+v"(u.v[k])::"memory");
+    load(ct + 20, 30);
+    const double t[6] = { MulRn(y[0], y[0]), MulRn(y[0], y[1]), MulRn(y[0], y[2]),
+                          MulRn(y[1], y[1]), MulRn(y[1], y[2]), MulRn(y[2], y[2]) };
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+#pragma unroll
+      for (int i = 0; i < 6; ++i) u.v[k] = __fma_rn(c[5 * i + k], t[i], u.v[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 5; ++k) asm volatile("" : "+v"(u.v[k])::"memory");
+  return u;
+}
+
 // The detector record's share of Taylor item (j, k) of a cell: the rho (k =
 // 0) and E (k = 4) coefficients, and with j = 0 the averages u[0][k] *
 // S[0][0] (polynomial().average() of limiter/weno.hpp:232-245).
@@ -89,16 +133,6 @@ __device__ __forceinline__ void FlagRecordItem(double *rec, int j, int k, double
   if (k == 0) rec[j] = taylor;
   if (k == 4) rec[10 + j] = taylor;
   if (j == 0 && (k == 0 || k == 4)) rec[kDgFlagAverage + (k == 4)] = u0k * s00;
-}
-
-// Lanes per (cell, component) in the moment phase of a 256-thread
-// workgroup of G cells: the largest power of two up to 16 (one DPP row)
-// with G * 5 * NPART <= 256.
-template <int G>
-constexpr int DgMomentParts() {
-  int p = 16;
-  while (p > 1 && G * 5 * p > 256) p /= 2;
-  return p;
 }
 
 // v from the lane given by a DPP control (within a row of 16 lanes).
@@ -124,257 +158,308 @@ __device__ __forceinline__ double GroupSum(double v) {
   return v;
 }
 
-// The face fluxes w Fhat were computed once per face point by
-// DgFaceFluxKernel into a.fhat; the face tasks read them.  Tetrahedra run at
-// 5 waves per SIMD (the LDS of 5 workgroups fits in a CU): the few bytes the
-// register bound spills cost less than the fifth wave gains.
-template <bool kHex, int P>
-__global__ __launch_bounds__(256, kHex ? 4 : 5) void DgModalStageKernel(DgModalArgs a) {
+template <bool kHex, int P, int kRiemann>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void DgModalStageKernel(DgModalArgs a) {
   using S = DgShape<kHex, P>;
   constexpr int N = S::kN, NQ = S::kNQ, NF = S::kNF, NFP = S::kNFP, T = S::kT, G = S::kG, PK = S::kPacked;
-  constexpr int GS = kDgGeoStride;
-  __shared__ double s_own[G * 5 * N + G * GS];  // own Taylor coefficients and geometry; then S
-  __shared__ double s_rt[G * 5 * N];       // Taylor moments Rt
-  __shared__ double s_vol[G * NQ * kSlot]; // volume tasks: flux x weight, pad, y
-  __shared__ double s_face[G * NF * NFP * kFaceSlot];  // face tasks: -/+ w Fhat (5), y; then the new state
-  static_assert(G * 5 * N <= G * NF * NFP * kFaceSlot, "LDS aliasing");
-  static_assert(G * PK <= G * 5 * N + G * GS, "LDS aliasing");
-  static_assert(G * N + G <= G * NQ * kSlot, "LDS aliasing");
-  double *s_ct = s_own, *s_geo = s_own + G * 5 * N;
-  double *s_s = s_own;  // Gram-Schmidt factors, from phase 2 on
-  double *s_new = s_face;
-  constexpr int kSIter = (G * PK + 255) / 256, kItems = (G * 5 * N + 255) / 256;
+  constexpr int GS = kDgGeoStride, CT = 5 * N;
+  __shared__ __attribute__((aligned(16))) double s_ct[G * CT];     // own Taylor coefficients; then the new state
+  __shared__ __attribute__((aligned(16))) double s_geo[G * GS];
+  __shared__ __attribute__((aligned(16))) double s_s[G * PK];      // Gram-Schmidt factors
+  __shared__ double s_vol[G * NQ * kSlot];             // volume tasks: flux x weight, y
+  __shared__ double s_face[G * NF * NFP * kFaceSlot];  // face tasks: -/+ w Fhat (5), y
 
   const int tid = threadIdx.x;
   const int64_t c0 = (int64_t)blockIdx.x * G;
-  if (c0 >= a.n_cells) return;
-  const int nc = (int)min<int64_t>(G, a.n_cells - c0);
+  const int64_t left_over = a.n_cells - c0;
+  const int nc = left_over < G ? (int)left_over : G;
 
-  // ---- this thread's point task and its global inputs: issued before the
-  // staging loads so that their latency overlaps them.  Tasks are numbered
+  // ---- this thread's point task and its global inputs.  Tasks are numbered
   // volume points of all G cells first, then face points, so that at most one
   // wavefront holds both kinds and runs both branches.
   const bool is_face = tid >= G * NQ;
-  const int tf = tid - G * NQ;
+  const int tf = is_face ? tid - G * NQ : 0;
   const int g = is_face ? tf / (NF * NFP) : tid / NQ;
-  const int r = is_face ? NQ + (tf - g * (NF * NFP)) : tid - g * NQ;
+  const int r = is_face ? tf - g * (NF * NFP) : tid - g * NQ;
   const bool active = g < nc && tid < G * T;
-  const int lf = is_face ? (r - NQ) / NFP : 0, q = is_face ? (r - NQ) - ((r - NQ) / NFP) * NFP : r;
+  const int lf = r / NFP, q = r - lf * NFP;  // of a face task
   const DgTables *tb = a.tables;
-  int32_t info = 0;
-  double eta[3] = { 0, 0, 0 }, wl = 0;
-  double fw[5] = { 0, 0, 0, 0, 0 };  // face task: w Fhat of this face point
+  int2 info = { 0, 0 };
+  if (active && is_face) info = a.finfo[(c0 + g) * 6 + lf];
+
+  // ---- phase 0: stage the cells' data in LDS, 16 bytes per load
+  auto stage = [&](const double *from, double *to, int doubles) {
+    typedef double Two __attribute__((ext_vector_type(2), aligned(8)));  // an odd number of cells' factors before
+    for (int w = 2 * tid; w < doubles; w += 2 * 256) {
+      if (w + 1 < doubles) *reinterpret_cast<Two *>(to + w) = *reinterpret_cast<const Two *>(from + w);
+      else to[w] = from[w];
+    }
+  };
+  stage(a.ct + c0 * CT, s_ct, nc * CT);
+  stage(a.basis + c0 * PK, s_s, nc * PK);
+  stage(a.geo + c0 * GS, s_geo, nc * GS);
+
+  double eta[3] = { 0, 0, 0 }, wl = 0, n[3] = { 0, 0, 0 }, area = 0;
+  double fw[5] = { 0, 0, 0, 0, 0 };  // face task: the other trace, then w Fhat
+  const bool holder = (info.x >> 7) & 1;
   if (active) {
     if (!is_face) {
 #pragma unroll
       for (int d = 0; d < 3; ++d) eta[d] = tb->vol_eta[r][d];
       wl = tb->vol_w[r];
     } else {
-      info = a.finfo[(c0 + g) * 6 + lf];
-      const bool holder = (info >> 7) & 1;
-      const int orient = (info >> 3) & 15;
+      const int orient = (info.x >> 3) & 15;
 #pragma unroll
       for (int d = 0; d < 3; ++d) eta[d] = tb->face_eta[lf][holder ? 0 : orient][q][d];
-      const double *src = a.fhat + ((int64_t)(info >> 8) * NFP + q) * 5;
+      if constexpr (kRiemann == kExact) {
+        const double *src = a.fhat + ((int64_t)(info.x >> 8) * NFP + q) * 5;
 #pragma unroll
-      for (int k = 0; k < 5; ++k) fw[k] = src[k];
+        for (int k = 0; k < 5; ++k) fw[k] = src[k];
+      } else {
+        const double *fc = a.faces + (int64_t)(info.x >> 8) * kDgFaceStride;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) n[d] = fc[d];
+        area = fc[6];
+        wl = tb->face_w[q];
+        if (info.y >= 0) {
+          const double *eta_n = tb->face_eta[info.x & 7][holder ? orient : 0][q];
+          const double *jn = a.geo + (int64_t)info.y * GS;
+          double j[10], y[3];
+#pragma unroll
+          for (int i = 0; i < 10; i += 2) {
+            const double2 v = *reinterpret_cast<const double2 *>(jn + i);
+            j[i] = v.x;
+            j[i + 1] = v.y;
+          }
+          Offset(j, eta_n, y);
+          const State other = TraceAt<P>(a.ct + (int64_t)info.y * CT, y);
+#pragma unroll
+          for (int k = 0; k < 5; ++k) fw[k] = other.v[k];
+        }
+      }
     }
   }
-
-  // the Gram-Schmidt factors S and the state and U0 of the phase-3 items,
-  // issued with the staging loads so that one round trip serves all of them
-  double s_pf[kSIter];
-#pragma unroll
-  for (int it = 0; it < kSIter; ++it) {
-    const int w = tid + 256 * it;
-    s_pf[it] = w < nc * PK ? a.basis[c0 * PK + w] : 0.0;
-  }
-  double us_pf[kItems], u0_pf[kItems];
-#pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const int w = tid + 256 * it;
-    const bool on = w < nc * 5 * N;
-    us_pf[it] = on && a.stage >= 1 ? a.us[c0 * 5 * N + w] : 0.0;
-    u0_pf[it] = on && a.stage >= 2 ? a.u0[c0 * 5 * N + w] : 0.0;
-  }
-
-  // ---- phase 0: stage the cells' data in LDS
-  for (int w = tid; w < nc * 5 * N; w += 256) s_ct[w] = a.ct[c0 * 5 * N + w];
-  for (int w = tid; w < nc * GS; w += 256) s_geo[w] = a.geo[c0 * GS + w];
   __syncthreads();
 
   // ---- phase 1: point tasks
   if (active) {
     const double *geo = s_geo + g * GS;
-    const double *own_ct = s_ct + g * 5 * N;
-    if (!is_face) {
-      double *slot = s_vol + (g * NQ + r) * kSlot;
-      double y[3];
-      Offset(geo, eta, y);
-      const State u = EvalTaylor<P>(own_ct, y);
-      double f[5][3];
-      FluxMatrix(u, f);
-      const double w = MulRn(wl, geo[9]);
+    double y[3];
+    Offset(geo, eta, y);
+    if (!is_face || kRiemann != kExact) {
+      const State own = TraceAt<P>(s_ct + g * CT, y);
+      if (!is_face) {
+        double *slot = s_vol + (g * NQ + r) * kSlot;
+        // the flux matrix (types.hpp:322-333), times the global weight
+        const double zero[3] = { 0, 0, 0 };
+        const FaceTrace t = TraceOf(own, zero);
+        const double w = MulRn(wl, geo[9]);
+        const double wp = t.p * w;
 #pragma unroll
-      for (int k = 0; k < 5; ++k)
+        for (int d = 0; d < 3; ++d) {
+          const double wv = t.v[d] * w;
+          slot[5 * d] = own.v[1 + d] * w;
 #pragma unroll
-        for (int d = 0; d < 3; ++d) slot[5 * d + k] = f[k][d] * w;
+          for (int e = 0; e < 3; ++e) slot[5 * d + 1 + e] = e == d ? __fma_rn(own.v[1 + e], wv, wp) : own.v[1 + e] * wv;
+          slot[5 * d + 4] = (own.v[4] + t.p) * wv;
+          slot[kSlotY + d] = y[d];
+        }
+      } else {
+        State flux;
+        bool star = false;
+        int kind = kBcSmart;
+        if (info.y < 0) {
+          const int tag = -info.y - 1;
+          kind = a.bc_kind[tag];
+          // the tag's constant state, or this point's value of the tag's
+          // boundary function at the stage time
+          const double *gs = a.bc_point_state
+              ? a.bc_point_state + (((int64_t)(info.x >> 8) - a.n_interior) * NFP + q) * 5 : a.bc_state + tag * 5;
 #pragma unroll
-      for (int d = 0; d < 3; ++d) slot[kSlotY + d] = y[d];
-    } else {
+          for (int k = 0; k < 5; ++k) fw[k] = gs[k];
+        }
+        if (kind == kBcSmart) {
+          State l, r;
+#pragma unroll
+          for (int k = 0; k < 5; ++k) {
+            l.v[k] = holder ? own.v[k] : fw[k];
+            r.v[k] = holder ? fw[k] : own.v[k];
+          }
+          flux = FaceFlux<kRiemann>(n, l, r, star);
+        } else {
+          State given;
+#pragma unroll
+          for (int k = 0; k < 5; ++k) given.v[k] = fw[k];
+          flux = BoundaryFlux(kind, true, n, own, given);
+        }
+        const double wq = MulRn(wl, area);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) fw[k] = flux.v[k] * wq;
+      }
+    }
+    if (is_face) {
       // dg/general.hpp:80-88: -w Fhat into the holder, +w Fhat into the sharer
-      double *slot = s_face + (g * NF * NFP + (r - NQ)) * kFaceSlot;
-      const bool holder = (info >> 7) & 1;
-      double y[3];
-      Offset(geo, eta, y);
+      double *slot = s_face + (g * NF * NFP + r) * kFaceSlot;
 #pragma unroll
       for (int k = 0; k < 5; ++k) slot[k] = holder ? -fw[k] : fw[k];
 #pragma unroll
       for (int d = 0; d < 3; ++d) slot[5 + d] = y[d];
     }
   }
-  __syncthreads();
-
-  // ---- phase 2: Taylor moments; S goes to the freed LDS of the own data
-  // at the end
-  // Taylor moments Rt[k][j].  Lane (cell, component, part) accumulates all N
-  // moments of its component over the points part, part + NPART, ... of the
-  // cell (volume points first, then face points), with the per-point FMA
-  // chains of the monomial table (basis/taylor.hpp:204-208):
+  // ---- phase 2, one wavefront: lane (cell, component, part) accumulates all N
+  // Taylor moments of its component over the points part, part + NPART, ... of
+  // the cell, with the per-point FMA chains of the monomial table
+  // (basis/taylor.hpp:204-208):
   //   volume: grad(Y_a Y_b) . F = F_a Y_b + F_b Y_a,  face: Fhat Y_a Y_b;
   // the NPART adjacent lanes then sum their partial moments by a fixed
-  // butterfly, so every lane of the group holds the same bits.
-  {
-    constexpr int NPART = DgMomentParts<G>();
-    const int grp = tid / NPART, part = tid - (tid / NPART) * NPART;
-    const int gc = grp / 5, k = grp - (grp / 5) * 5;
-    double mo[10] = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
-    if (gc < nc) {
-      const double *vb = s_vol + gc * NQ * kSlot;
-      for (int q = part; q < NQ; q += NPART) {
-        const double *r = vb + q * kSlot;
-        const double f0 = r[k], f1 = r[5 + k], f2 = r[10 + k];
-        const double y0 = r[kSlotY], y1 = r[kSlotY + 1], y2 = r[kSlotY + 2];
-        mo[1] += f0;
-        mo[2] += f1;
-        mo[3] += f2;
-        if constexpr (N == 10) {
-          mo[4] = __fma_rn(f0, y0, __fma_rn(f0, y0, mo[4]));
-          mo[5] = __fma_rn(f1, y0, __fma_rn(f0, y1, mo[5]));
-          mo[6] = __fma_rn(f2, y0, __fma_rn(f0, y2, mo[6]));
-          mo[7] = __fma_rn(f1, y1, __fma_rn(f1, y1, mo[7]));
-          mo[8] = __fma_rn(f2, y1, __fma_rn(f1, y2, mo[8]));
-          mo[9] = __fma_rn(f2, y2, __fma_rn(f2, y2, mo[9]));
-        }
-      }
-      const double *fb = s_face + gc * NF * NFP * kFaceSlot;
-      for (int q = (part + NPART - NQ % NPART) % NPART; q < NF * NFP; q += NPART) {
-        const double *r = fb + q * kFaceSlot;
-        const double ff = r[k], y0 = r[5], y1 = r[6], y2 = r[7];
-        mo[0] += ff;
-        mo[1] = __fma_rn(ff, y0, mo[1]);
-        mo[2] = __fma_rn(ff, y1, mo[2]);
-        mo[3] = __fma_rn(ff, y2, mo[3]);
-        if constexpr (N == 10) {
-          mo[4] = __fma_rn(ff, y0 * y0, mo[4]);
-          mo[5] = __fma_rn(ff, y0 * y1, mo[5]);
-          mo[6] = __fma_rn(ff, y0 * y2, mo[6]);
-          mo[7] = __fma_rn(ff, y1 * y1, mo[7]);
-          mo[8] = __fma_rn(ff, y1 * y2, mo[8]);
-          mo[9] = __fma_rn(ff, y2 * y2, mo[9]);
-        }
-      }
+  // butterfly, so every lane of the group holds the same bits, and each does
+  // the rows part, part + NPART, ... of what follows.
+  constexpr int NPART = G * 40 <= 64 ? 8 : (G * 20 <= 64 ? 4 : (G * 10 <= 64 ? 2 : 1));
+  constexpr int kRows = (N + NPART - 1) / NPART;
+  static_assert(G * N <= 64 && G * 5 <= 64, "one wavefront finishes the cells");
+  const int grp = tid / NPART, part = tid - grp * NPART;
+  const int gc = grp / 5, k = grp - gc * 5;
+  const bool on = gc < nc;
+  const int gs = on ? gc : 0;
+  const int64_t at = (c0 + gs) * CT + 5 * part + k;  // row part of this lane's column
+  double us[kRows], u0[kRows];
+#pragma unroll
+  for (int t = 0; t < kRows; ++t) us[t] = u0[t] = 0.0;
+  if (tid < 64 && a.stage >= 1) {  // in flight across the barrier
+#pragma unroll
+    for (int t = 0; t < kRows; ++t)
+      if (NPART * t + part < N) us[t] = a.us[at + 5 * NPART * t];
+    if (a.stage >= 2) {
+#pragma unroll
+      for (int t = 0; t < kRows; ++t)
+        if (NPART * t + part < N) u0[t] = a.u0[at + 5 * NPART * t];
     }
-#pragma unroll
-    for (int j = 0; j < N; ++j) mo[j] = GroupSum<NPART>(mo[j]);
-    if (gc < nc) {
-#pragma unroll
-      for (int j = 0; j < N; ++j)
-        if (j % NPART == part) s_rt[gc * 5 * N + 5 * j + k] = mo[j];
-    }
-  }
-#pragma unroll
-  for (int it = 0; it < kSIter; ++it) {
-    const int w = tid + 256 * it;
-    if (w < nc * PK) s_s[w] = s_pf[it];
   }
   __syncthreads();
-
-  // ---- phase 3: R = Rt S^T, RK stage, store
-#pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const int w = tid + 256 * it;
-    if (w >= nc * 5 * N) break;
-    const int gc = w / (5 * N), rem = w - gc * 5 * N, i = rem / 5, k = rem - (rem / 5) * 5;
-    const double *srow = s_s + gc * PK + i * (i + 1) / 2;
-    const double *rt = s_rt + gc * 5 * N;
-    double res = 0.0;
-    for (int j = 0; j <= i; ++j) res = __fma_rn(rt[5 * j + k], srow[j], res);
-    const int64_t idx = c0 * 5 * N + w;
-    double out;
-    if (a.stage == 0) {
-      out = res;
-    } else {
-      const double next = AddRn(us_pf[it], MulRn(res, a.dt));
-      if (a.stage == 1) {
-        out = next;
-      } else if (a.stage == 2) {
-        out = AddRn(MulRn(u0_pf[it], 3.0), next) / 4.0;
-      } else {
-        out = AddRn(MulRn(next, 2.0), u0_pf[it]) / 3.0;
-      }
+  if (tid >= 64) return;
+  double mo[10] = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+  const double *vb = s_vol + gs * NQ * kSlot;
+#pragma unroll 2
+  for (int q0 = 0; q0 < NQ; q0 += NPART) {
+    if (NQ % NPART != 0 && q0 + part >= NQ) break;
+    const double *v = vb + (q0 + part) * kSlot;
+    const double f0 = v[k], f1 = v[5 + k], f2 = v[10 + k];
+    const double y0 = v[kSlotY], y1 = v[kSlotY + 1], y2 = v[kSlotY + 2];
+    mo[1] += f0;
+    mo[2] += f1;
+    mo[3] += f2;
+    if constexpr (N == 10) {
+      mo[4] = __fma_rn(f0, y0 + y0, mo[4]);
+      mo[5] = __fma_rn(f1, y0, __fma_rn(f0, y1, mo[5]));
+      mo[6] = __fma_rn(f2, y0, __fma_rn(f0, y2, mo[6]));
+      mo[7] = __fma_rn(f1, y1 + y1, mo[7]);
+      mo[8] = __fma_rn(f2, y1, __fma_rn(f1, y2, mo[8]));
+      mo[9] = __fma_rn(f2, y2 + y2, mo[9]);
     }
-    a.out[idx] = out;
-    s_new[w] = out;
+  }
+  const double *fb = s_face + gs * NF * NFP * kFaceSlot;
+#pragma unroll 2
+  for (int q0 = 0; q0 < NF * NFP; q0 += NPART) {
+    if (NF * NFP % NPART != 0 && q0 + part >= NF * NFP) break;
+    const double *v = fb + (q0 + part) * kFaceSlot;
+    const double ff = v[k], y0 = v[5], y1 = v[6], y2 = v[7];
+    mo[0] += ff;
+    const double g0 = ff * y0, g1 = ff * y1, g2 = ff * y2;
+    mo[1] += g0;
+    mo[2] += g1;
+    mo[3] += g2;
+    if constexpr (N == 10) {
+      mo[4] = __fma_rn(g0, y0, mo[4]);
+      mo[5] = __fma_rn(g0, y1, mo[5]);
+      mo[6] = __fma_rn(g0, y2, mo[6]);
+      mo[7] = __fma_rn(g1, y1, mo[7]);
+      mo[8] = __fma_rn(g1, y2, mo[8]);
+      mo[9] = __fma_rn(g2, y2, mo[9]);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) mo[j] = GroupSum<NPART>(mo[j]);
+
+  // ---- R = Rt S^T, RK stage, store
+  const double *sc = s_s + gs * PK;
+  // the new state replaces the cell's own Taylor coefficients, then its Taylor
+  // coefficients the new state: one wavefront's LDS operations are in order
+  double *sn = s_ct + gs * CT + k;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int t = 0; t < kRows; ++t) {
+    const int i = NPART * t + part;
+    const int row = i < N ? i : N - 1;
+    const double *srow = sc + row * (row + 1) / 2;
+    double res = 0.0;
+#pragma unroll
+    for (int j = 0; j < N && j < NPART * (t + 1); ++j) {
+      const double next = __fma_rn(mo[j], srow[j <= NPART * t ? j : (j <= row ? j : row)], res);
+      res = j <= NPART * t || j <= row ? next : res;
+    }
+    double out = res;
+    if (a.stage >= 1) {
+      const double next = AddRn(us[t], MulRn(res, a.dt));
+      out = a.stage == 1 ? next : (a.stage == 2 ? AddRn(MulRn(u0[t], 3.0), next) * 0.25
+                                                : ThirdOf(AddRn(MulRn(next, 2.0), u0[t])));
+    }
+    if (on && i < N) {
+      a.out[at + 5 * NPART * t] = out;
+      sn[5 * i] = out;
+    }
   }
   if (!a.ct_out) return;
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  double fresh[kRows];
 
-  // ---- phase 4: Taylor coefficients of the new state for the next pass
-  for (int w = tid; w < nc * 5 * N; w += 256) {
-    const int gc = w / (5 * N), rem = w - gc * 5 * N, j = rem / 5, k = rem - (rem / 5) * 5;
-    const double *sn = s_new + gc * 5 * N;
-    const double *sc = s_s + gc * PK;
+  // ---- Taylor coefficients of the new state for the next pass
+#pragma unroll
+  for (int t = 0; t < kRows; ++t) {
+    const int j = NPART * t + part;
     double acc = 0.0;
-    for (int i = j; i < N; ++i) acc = __fma_rn(sn[5 * i + k], sc[i * (i + 1) / 2 + j], acc);
-    a.ct_out[c0 * 5 * N + w] = acc;
-    s_rt[w] = acc;  // for the fused time step
-    if (a.flag_rec) FlagRecordItem(a.flag_rec + (c0 + gc) * kDgFlagRecord, j, k, acc, sn[k], sc[0]);
+#pragma unroll
+    for (int i = NPART * t; i < N; ++i) {
+      const double next = __fma_rn(sn[5 * i], sc[i * (i + 1) / 2 + (j <= i ? j : i)], acc);
+      acc = i >= NPART * (t + 1) - 1 || i >= j ? next : acc;
+    }
+    fresh[t] = acc;
+    if (on && j < N) {
+      a.ct_out[at + 5 * NPART * t] = acc;
+      if (a.flag_rec) FlagRecordItem(a.flag_rec + (c0 + gs) * kDgFlagRecord, j, k, acc, sn[0], sc[0]);
+    }
   }
   if (!a.dt_min_bits) return;
 
-  // ---- phase 5: fem.hpp:412-435 on the new state, as DgTimeStepKernel: min
-  // over cells of length / max(1e-5, max over the first N points of |u| + c)
-  __syncthreads();
-  double *s_speed = s_vol, *s_cell = s_vol + G * N;
-  for (int w = tid; w < nc * N; w += 256) {
-    const int gc = w / N, q = w - gc * N;
+  // ---- fem.hpp:412-435 on the new state, as DgTimeStepKernel: min over cells of
+  // length / max(1e-5, max over the first N points of |u| + c), which is the min
+  // over those points of length / max(1e-5, |u| + c)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int t = 0; t < kRows; ++t)
+    if (on && NPART * t + part < N) sn[5 * (NPART * t + part)] = fresh[t];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  double local = 1e300;
+  const int cell = tid / N, point = tid - cell * N;
+  if (cell < nc) {
+    const double *geo = s_geo + cell * GS;
     double y[3];
-    Offset(a.geo + (c0 + gc) * GS, tb->vol_eta[q], y);
-    s_speed[w] = MaxSpeed(EvalTaylor<P>(s_rt + gc * 5 * N, y));
+    Offset(geo, tb->vol_eta[point], y);
+    local = geo[10] / fmax(1e-5, MaxSpeed(EvalTaylor<P>(s_ct + cell * CT, y)));
   }
-  __syncthreads();
-  if (tid < nc) {
-    double vmax = 1e-5;
-    for (int q = 0; q < N; ++q) vmax = fmax(vmax, s_speed[tid * N + q]);
-    s_cell[tid] = a.geo[(c0 + tid) * GS + 10] / vmax;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    double local = 1e300;
-    for (int c = 0; c < nc; ++c) local = fmin(local, s_cell[c]);
-    atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(local));
-  }
+#pragma unroll
+  for (int o = 32; o >= 1; o /= 2) local = fmin(local, __shfl_xor(local, o));
+  if (tid == 0) atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(local));
 }
 
-// w Fhat at every face quadrature point, once per face (dg/general.hpp:51-55,
-// 70-89 and the boundary fluxes :92-202): one thread per (face, point).  The
-// point is located in the holder through its canonical order and in the
-// sharer through the corner-permutation code, and each trace is evaluated
-// from the cell's Taylor coefficients.  The exact solver's iteration needs
-// more registers than 4 waves per SIMD allow; the default bound leaves the
-// compiler room for it without spills.
-template <bool kHex, int P, int kRiemann>
+// The exact solver's w Fhat at every face quadrature point, once per face
+// (dg/general.hpp:51-55, 70-89 and the boundary fluxes :92-202): one thread per
+// (face, point).  The point is located in the holder through its canonical order
+// and in the sharer through the corner-permutation code, and each trace is
+// evaluated from the cell's Taylor coefficients.  A serial chain (the iteration's
+// pow) bounds it; the default register bound leaves room for it without spills.
+// 3840 tetrahedra of the Sod tube, face and cell pass: 41 -> 29 us with the fluxes
+// of the face normal alone.
+template <bool kHex, int P>
 __global__ __launch_bounds__(256) void DgFaceFluxKernel(DgModalArgs a) {
   constexpr int N = P == 1 ? 4 : 10, NFP = DgShape<kHex, P>::kNFP, GS = kDgGeoStride;
   const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -385,48 +470,39 @@ __global__ __launch_bounds__(256) void DgFaceFluxKernel(DgModalArgs a) {
   const int32_t holder = a.face_cells[f * 3], sharer = a.face_cells[f * 3 + 1], pk = a.face_cells[f * 3 + 2];
   const int hf = pk & 7, sf = (pk >> 3) & 7, orient = (pk >> 6) & 15;
   const double *fc = a.faces + f * kDgFaceStride;
-  FaceFrame frame;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) { frame.n[d] = fc[d]; frame.t[d] = fc[3 + d]; }
-  frame.b[0] = frame.n[1] * frame.t[2] - frame.n[2] * frame.t[1];
-  frame.b[1] = frame.n[2] * frame.t[0] - frame.n[0] * frame.t[2];
-  frame.b[2] = frame.n[0] * frame.t[1] - frame.n[1] * frame.t[0];
+  const double n[3] = { fc[0], fc[1], fc[2] };
   const double wq = MulRn(tb->face_w[q], fc[6]);
-  double y[3];
-  Offset(a.geo + (int64_t)holder * GS, tb->face_eta[hf][0][q], y);
-  const State own = EvalTaylor<P>(a.ct + (int64_t)holder * 5 * N, y);
-  State flux;
-  // the exact solver's state of this face point (ExactFlux), kept across calls
-  bool star = kRiemann == kExact ? a.exact_star[w] != 0 : false;
+  // the trace in a cell, its J in 16-byte loads
+  auto trace = [&](int32_t cell, const double *eta) {
+    double j[10], y[3];
+#pragma unroll
+    for (int i = 0; i < 10; i += 2) {
+      const double2 v = *reinterpret_cast<const double2 *>(a.geo + (int64_t)cell * GS + i);
+      j[i] = v.x;
+      j[i + 1] = v.y;
+    }
+    Offset(j, eta, y);
+    return TraceAt<P>(a.ct + (int64_t)cell * 5 * N, y);
+  };
+  const State own = trace(holder, tb->face_eta[hf][0][q]);
+  State given;
+  bool star = a.exact_star[w] != 0;  // this face point's state (ExactFlux), kept across calls
+  int kind = kBcSmart;
   if (sharer >= 0) {
-    double ys[3];
-    Offset(a.geo + (int64_t)sharer * GS, tb->face_eta[sf][orient][q], ys);
-    const State other = EvalTaylor<P>(a.ct + (int64_t)sharer * 5 * N, ys);
-    flux = UpwindFlux<kRiemann>(frame, own, other, star);
+    given = trace(sharer, tb->face_eta[sf][orient][q]);
   } else {
     const int tag = -sharer - 1;
-    const int kind = a.bc_kind[tag];
+    kind = a.bc_kind[tag];
     // the tag's constant state, or this point's value of the tag's boundary
     // function at the stage time
     const double *gs = a.bc_point_state ? a.bc_point_state + (w - a.n_interior * NFP) * 5 : a.bc_state + tag * 5;
-    State given;
 #pragma unroll
     for (int k = 0; k < 5; ++k) given.v[k] = gs[k];
-    if (kind == kBcInviscidWall) {
-      flux = WallFlux(frame, own);
-    } else if (kind == kBcSupersonicOutlet) {
-      flux = StateFlux(frame, own);
-    } else if (kind == kBcSupersonicInlet) {
-      flux = StateFlux(frame, given);
-    } else if (kind == kBcSubsonicInlet) {
-      flux = SubsonicInletFlux(frame, own, given);
-    } else if (kind == kBcSubsonicOutlet) {
-      flux = SubsonicOutletFlux(frame, own, given);
-    } else {
-      flux = UpwindFlux<kRiemann>(frame, own, given, star);
-    }
   }
-  if constexpr (kRiemann == kExact) a.exact_star[w] = star ? 1 : 0;
+  State flux;
+  if (kind == kBcSmart) flux = FaceFlux<kExact>(n, own, given, star);
+  else flux = BoundaryFlux(kind, true, n, own, given);
+  a.exact_star[w] = star ? 1 : 0;
 #pragma unroll
   for (int k = 0; k < 5; ++k) a.fhat[w * 5 + k] = flux.v[k] * wq;
 }
@@ -997,12 +1073,13 @@ hipError_t LaunchStage(const DgModalArgs &a, hipStream_t stream) {
   const int64_t blocks = (a.n_cells + G - 1) / G;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
   constexpr int NFP = DgShape<kHex, P>::kNFP;
-  const int64_t fblocks = (a.n_faces * NFP + 255) / 256;
-  if (fblocks > 0x7fffffff || !a.fhat || !a.face_cells) return hipErrorInvalidValue;
-  // face fluxes once per face point, then the cell pass
-  if (fblocks > 0)
-    hipLaunchKernelGGL((DgFaceFluxKernel<kHex, P, R>), dim3((unsigned)fblocks), dim3(256), 0, stream, a);
-  hipLaunchKernelGGL((DgModalStageKernel<kHex, P>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  if constexpr (R == kExact) {
+    const int64_t fblocks = (a.n_faces * NFP + 255) / 256;
+    if (fblocks > 0x7fffffff || !a.fhat || !a.face_cells || !a.exact_star) return hipErrorInvalidValue;
+    if (fblocks > 0)
+      hipLaunchKernelGGL((DgFaceFluxKernel<kHex, P>), dim3((unsigned)fblocks), dim3(256), 0, stream, a);
+  }
+  hipLaunchKernelGGL((DgModalStageKernel<kHex, P, R>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

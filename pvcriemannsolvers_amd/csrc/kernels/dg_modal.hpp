@@ -55,7 +55,9 @@ struct DgModalArgs {
   double *ct_out;         // Taylor coefficients of `out`, or null
   const double *basis;    // [cell][N(N+1)/2] S, packed lower triangle by rows
   const double *geo;      // [cell][kDgGeoStride]
-  const int32_t *finfo;   // [cell][6]: face id << 8 | holder << 7 | orient << 3 | neighbour's local face
+  // [cell][6]: face id << 8 | holder << 7 | orient << 3 | neighbour's local face;
+  // the neighbour or -(1 + boundary tag)
+  const int2 *finfo;
   const double *faces;    // [face][kDgFaceStride]
   const int32_t *bc_kind; // [tag]: BcKind (euler.hpp)
   const double *bc_state; // [tag][5] given state (conservative, or the subsonic parameters)
@@ -71,8 +73,8 @@ struct DgModalArgs {
   // state this pass writes is folded into *dt_min_bits (same arithmetic).
   unsigned long long *dt_min_bits;
   double *flag_rec;       // [cell][kDgFlagRecord] for the WENO detector, or null (no limiter)
-  // The pass runs as two launches: w Fhat once per face point into fhat
-  // [face][point][5], then the cells read it.  face_cells [face][3]: holder,
+  // exact solver only: w Fhat once per face point into fhat [face][point][5],
+  // then the cells read it.  face_cells [face][3]: holder,
   // sharer or -(1 + boundary tag), holder face | sharer face << 3 |
   // orientation << 6.
   double *fhat;

@@ -1,0 +1,43 @@
+"""DG stage kernel at the edges of its workgroups (6 tetrahedra; 8 or 3
+hexahedra of degree 1 or 2): single cells, one cell short of a workgroup, one
+over; every boundary family, all solvers, the step and the time step folded into
+it.  Tolerances as in tests/test_dg_gpu.py: the same FP64 formulas summed in
+another order, 1e-12 relative; the exact solver's stopping rule 1e-7.
+"""
+import numpy as np
+import pytest
+
+from pvcriemannsolvers_amd import meshgen
+from test_dg_gpu import MIXED_BCS, TOL, make_pair, rel, smooth_state
+
+pytestmark = pytest.mark.gpu
+
+
+def first_tets(n):
+    """The first n tetrahedra of a box, their free faces tagged in turn."""
+    mesh = meshgen.box_tet(3, 1, 1, hi=(0.75, 0.25, 0.25))
+    cells = mesh["cells"][:n]
+    faces = np.concatenate([cells[:, [0, 1, 2]], cells[:, [0, 1, 3]], cells[:, [0, 2, 3]], cells[:, [1, 2, 3]]])
+    _, first, counts = np.unique(np.sort(faces, axis=1), axis=0, return_index=True, return_counts=True)
+    bfaces = faces[np.sort(first[counts == 1])]
+    return dict(mesh, cells=np.ascontiguousarray(cells), bface_nodes=np.ascontiguousarray(bfaces),
+                bface_tags=(np.arange(len(bfaces)) % 6).astype(np.int32))
+
+
+@pytest.mark.parametrize("kind,cells", [("tet", 1), ("tet", 5), ("tet", 7), ("tet", 13),
+                                        ("hex", 1), ("hex", 2), ("hex", 4), ("hex", 7), ("hex", 9)])
+@pytest.mark.parametrize("degree", [1, 2])
+@pytest.mark.parametrize("riemann", ["roe", "hllc", "exact"])
+def test_workgroup_edges(kind, cells, degree, riemann):
+    mesh = first_tets(cells) if kind == "tet" else meshgen.box_hex(cells, 1, 1, hi=(0.25 * cells, 0.25, 0.25))
+    o, g = make_pair(mesh, degree, riemann, MIXED_BCS)
+    u = o.approximate(smooth_state(o.cells()["xyz"]))
+    g.set_solution_column(u)
+    assert rel(g.get_residual_column(), o.residual(u)) <= TOL[riemann]
+    dt = g.get_time_step(0.05)
+    g.rk3_update(0.0, dt)
+    ref = o.rk3(u, dt, 1)
+    assert rel(g.get_solution_column(), ref) <= TOL[riemann]
+    expect = o.time_step(ref, 0.05)
+    assert abs(g.get_time_step(0.05) - expect) <= TOL[riemann] * expect
+    g.close()
