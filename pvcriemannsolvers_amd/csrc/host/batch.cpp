@@ -29,6 +29,7 @@ struct CaseRef {
 struct mcfd_batch {
   int32_t n_cases = 0;
   hipStream_t stream = nullptr;
+  mcfd::ColumnCopy copy;                                   // columns of one case
   std::vector<std::unique_ptr<mcfd::FrHexGroup>> groups;  // one per degree
   std::vector<int32_t> tiles;                              // tile variant per group
   std::vector<CaseRef> cases;
@@ -209,6 +210,10 @@ int mcfd_batch_create(int32_t n_cases, const mcfd_mesh_desc *meshes, const int32
     b->dt.assign(n_cases, 0.0);
     b->case_dt.Upload(b->dt, b->stream);
     b->scratch.Allocate(n_cases);
+    size_t most = 0;
+    for (auto const &ref : b->cases)
+      most = std::max(most, size_t(ref.n_cells) * b->groups[ref.group]->np * 5 * sizeof(double));
+    b->copy.Reserve(most);
     Check(hipStreamSynchronize(b->stream), "create sync");
     b->Capture();
   });
@@ -248,7 +253,8 @@ int mcfd_batch_set_solution_column(mcfd_batch *b, int32_t c, const double *colum
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
     const auto &ref = b->cases[c];
-    b->groups[ref.group]->SetColumn(column, ref.first_cell, ref.n_cells, b->stream);
+    std::lock_guard<std::mutex> lock(b->copy.mutex);
+    b->groups[ref.group]->SetColumn(column, ref.first_cell, ref.n_cells, &b->copy, b->stream);
     Check(hipStreamSynchronize(b->stream), "sync");
   });
 }
@@ -258,8 +264,8 @@ int mcfd_batch_get_solution_column(mcfd_batch *b, int32_t c, double *column) {
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
     const auto &ref = b->cases[c];
-    b->groups[ref.group]->GetColumn(column, ref.first_cell, ref.n_cells, b->stream);
-    Check(hipStreamSynchronize(b->stream), "sync");
+    std::lock_guard<std::mutex> lock(b->copy.mutex);
+    b->groups[ref.group]->GetColumn(column, ref.first_cell, ref.n_cells, &b->copy, b->stream);
   });
 }
 

@@ -389,16 +389,17 @@ void FrHexGroup::BuildTileOrder(int tile_cells) {
   for (int64_t t = 0; t < n_tiles; ++t) h_tile_order[t] = key[t].second;
 }
 
-void FrHexGroup::SetColumn(const double *column, int64_t first_cell, int64_t count, hipStream_t stream) {
+void FrHexGroup::SetColumn(const double *column, int64_t first_cell, int64_t count, ColumnCopy *copy,
+                           hipStream_t stream) {
   const size_t at = size_t(first_cell) * np * 5, n = size_t(count) * np * 5;
-  Check(hipMemcpyAsync(res.ptr + at, column, n * sizeof(double), hipMemcpyHostToDevice, stream), "set solution");
+  copy->ToDevice(res.ptr + at, column, n * sizeof(double), stream);
   Check(LaunchFrLayout(true, res.ptr + at, u0.ptr + at, np, count, stream), "set solution layout");
 }
 
-void FrHexGroup::GetColumn(double *column, int64_t first_cell, int64_t count, hipStream_t stream) {
+void FrHexGroup::GetColumn(double *column, int64_t first_cell, int64_t count, ColumnCopy *copy, hipStream_t stream) {
   const size_t at = size_t(first_cell) * np * 5, n = size_t(count) * np * 5;
   Check(LaunchFrLayout(false, u0.ptr + at, res.ptr + at, np, count, stream), "get solution layout");
-  Check(hipMemcpyAsync(column, res.ptr + at, n * sizeof(double), hipMemcpyDeviceToHost, stream), "get solution");
+  copy->ToHost(column, res.ptr + at, n * sizeof(double), stream);
 }
 
 FrHexArgs FrHexGroup::Args(int stage, double dt) const {

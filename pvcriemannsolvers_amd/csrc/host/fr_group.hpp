@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../kernels/fr_hex.hpp"
+#include "column_copy.hpp"
 #include "common.hpp"
 #include "hex_connectivity.hpp"
 
@@ -61,8 +62,9 @@ struct FrHexGroup {
   size_t ColumnSize() const { return size_t(n_cells) * np * 5; }
   // The solution u0 of `count` cells from or to a host column (staged in `res`;
   // not synchronised).
-  void SetColumn(const double *column, int64_t first_cell, int64_t count, hipStream_t stream);
-  void GetColumn(double *column, int64_t first_cell, int64_t count, hipStream_t stream);
+  void SetColumn(const double *column, int64_t first_cell, int64_t count, ColumnCopy *copy,
+                 hipStream_t stream);
+  void GetColumn(double *column, int64_t first_cell, int64_t count, ColumnCopy *copy, hipStream_t stream);
   // Kernel arguments of one pass: stage 0 residual, 1..3 SSP-RK3 stages.
   FrHexArgs Args(int stage, double dt) const;
   void SamplePoints(double *xyz) const;

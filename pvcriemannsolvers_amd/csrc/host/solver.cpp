@@ -34,6 +34,7 @@ struct mcfd_solver {
   hipStream_t stream = nullptr;
   mcfd::FrHexGroup group;
   mcfd::DgGroup modal;
+  mcfd::ColumnCopy copy;
   mcfd::DeviceArray<unsigned long long> scratch;  // time-step reduction
   mcfd::BoundaryTable bct;                         // boundary values that vary in space and time
   // The time step (fem.hpp:412-435) of the state an RK step ends with can be
@@ -67,16 +68,17 @@ struct mcfd_solver {
     }
     if (fuse_dt) dt_fresh = dt_pending = true;
   }
-  // The solution from or to a host column (not synchronised).
+  // The solution from or to a host column.  FR columns pass through the residual's
+  // buffer: the copy's lock keeps its users apart (the caller of SetColumn holds it
+  // until the stream is drained).
   void SetColumn(const double *column) {
-    if (dg) Check(hipMemcpyAsync(modal.u0.ptr, column, ColumnSize() * sizeof(double), hipMemcpyHostToDevice, stream),
-                  "set solution");
-    else group.SetColumn(column, 0, group.n_cells, stream);
+    if (dg) copy.ToDevice(modal.u0.ptr, column, ColumnSize() * sizeof(double), stream);
+    else group.SetColumn(column, 0, group.n_cells, &copy, stream);
   }
   void GetColumn(double *column) {
-    if (dg) Check(hipMemcpyAsync(column, modal.u0.ptr, ColumnSize() * sizeof(double), hipMemcpyDeviceToHost, stream),
-                  "get solution");
-    else group.GetColumn(column, 0, group.n_cells, stream);
+    std::lock_guard<std::mutex> lock(copy.mutex);
+    if (dg) copy.ToHost(column, modal.u0.ptr, ColumnSize() * sizeof(double), stream);
+    else group.GetColumn(column, 0, group.n_cells, &copy, stream);
   }
   size_t ColumnSize() const { return dg ? modal.ColumnSize() : group.ColumnSize(); }
   double *Residual() { return dg ? modal.res.ptr : group.res.ptr; }
@@ -139,6 +141,7 @@ int mcfd_create(const mcfd_mesh_desc *mesh, const mcfd_scheme_desc *scheme, cons
       h->group.Upload(h->stream);
     }
     h->scratch.Allocate(1);
+    h->copy.Reserve(h->ColumnSize() * sizeof(double));
     Check(hipStreamSynchronize(h->stream), "create sync");
   });
   if (rc == MCFD_OK) *out = h.release();
@@ -172,6 +175,7 @@ int mcfd_set_solution_column(mcfd_solver *h, const double *column) {
   MCFD_REQUIRE_DEVICE(h);
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
+    std::lock_guard<std::mutex> lock(h->copy.mutex);
     h->dt_fresh = false;
     h->SetColumn(column);
     if (h->dg) h->modal.SolutionChanged(h->stream);
@@ -183,6 +187,7 @@ int mcfd_restore_solution_column(mcfd_solver *h, const double *column) {
   MCFD_REQUIRE_DEVICE(h);
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
+    std::lock_guard<std::mutex> lock(h->copy.mutex);
     h->dt_fresh = false;
     h->SetColumn(column);
     if (h->dg) h->modal.SolutionChanged(h->stream, /*limit=*/false);
@@ -195,7 +200,6 @@ int mcfd_get_solution_column(mcfd_solver *h, double *column) {
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
     h->GetColumn(column);
-    Check(hipStreamSynchronize(h->stream), "get solution sync");
   });
 }
 
@@ -203,10 +207,9 @@ int mcfd_get_residual_column(mcfd_solver *h, double *column) {
   MCFD_REQUIRE_DEVICE(h);
   if (!column) return Fail(MCFD_EINVAL, "null column");
   return Guard([&] {
+    std::lock_guard<std::mutex> lock(h->copy.mutex);
     h->Stage(0, 0.0);
-    Check(hipMemcpyAsync(column, h->Residual(), h->ColumnSize() * sizeof(double),
-                         hipMemcpyDeviceToHost, h->stream), "get residual");
-    Check(hipStreamSynchronize(h->stream), "get residual sync");
+    h->copy.ToHost(column, h->Residual(), h->ColumnSize() * sizeof(double), h->stream);
   });
 }
 
@@ -276,7 +279,6 @@ int mcfd_evaluate(mcfd_solver *h, const double *column, int32_t n_local, const d
     if (values && !column) {
       own.resize(h->ColumnSize());
       h->GetColumn(own.data());
-      Check(hipStreamSynchronize(h->stream), "get solution sync");
       column = own.data();
     }
     if (h->dg) h->modal.Evaluate(column, n_local, local, xyz, values);
