@@ -395,10 +395,12 @@ void DgGroup::Upload(hipStream_t stream) {
   geo.Upload(h_geo, stream);
   face_rec.Upload(h_faces, stream);
   if (riemann == MCFD_RIEMANN_EXACT) {
-    face_cells.Upload(h_face_cells, stream);
-    fhat.Allocate(faces.size() * nfp * 5);
-    exact_star.Allocate(faces.size() * nfp);
-    Check(hipMemsetAsync(exact_star.ptr, 0, faces.size() * nfp, stream), "memset");
+    if (DgFacePass(riemann, n_cells)) {
+      face_cells.Upload(h_face_cells, stream);
+      fhat.Allocate(faces.size() * nfp * 5);
+    }
+    exact_star.Allocate(faces.size() * 2 * nfp);
+    Check(hipMemsetAsync(exact_star.ptr, 0, faces.size() * 2 * nfp, stream), "memset");
   }
   bc_state.Upload(h_bc_state, stream);
   h_face_info.resize(h_finfo.size());
@@ -463,12 +465,12 @@ void DgGroup::Stage(int stage, double dt, hipStream_t stream, unsigned long long
   a.n_cells = n_cells; a.dt = dt; a.stage = stage;
   a.dt_min_bits = stage > 0 && !limiter ? dt_min_bits : nullptr;
   a.fhat = fhat.ptr;
+  a.face_cells = face_cells.ptr;
+  a.n_faces = (int64_t)faces.size();
   a.exact_star = exact_star.ptr;
   a.bc_point_state = bc_point_state;
   a.n_interior = n_interior;
   a.flag_rec = limiter && stage > 0 ? flag_rec.ptr : nullptr;
-  a.face_cells = face_cells.ptr;
-  a.n_faces = (int64_t)faces.size();
   Check(LaunchDgModalStage(cell_type, degree, riemann, a, stream), "DG stage launch");
   if (stage > 0) Limit(a.out, a.ct_out, stream);  // spatial/with_limiter.hpp:56-59 after each SetSolutionColumn
 }

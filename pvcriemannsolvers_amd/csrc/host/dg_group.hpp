@@ -36,11 +36,11 @@ struct DgGroup {
   std::vector<int2> h_face_info;
   DeviceArray<int2> finfo;
   DeviceArray<int32_t> bc_kind;
-  // exact solver's face pass: w Fhat once per face point, then the cell pass
+  // exact solver's face pass on large meshes: w Fhat once per face point, then the cell pass
   std::vector<int32_t> h_face_cells;  // [face][3]: holder, sharer or -(1 + tag), faces and orientation
   DeviceArray<int32_t> face_cells;
   DeviceArray<double> fhat;           // [face][point][5]
-  DeviceArray<uint8_t> exact_star;    // exact solver: [face][point] sign of the last star velocity
+  DeviceArray<uint8_t> exact_star;    // exact solver: [face][side][point] sign of the last star velocity
   DeviceArray<DgTables> tables_d;
   // WENO limiter (MCFD_LIMITER_*), applied to every state that is set
   int limiter = 0;

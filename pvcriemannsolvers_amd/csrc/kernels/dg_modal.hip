@@ -1,6 +1,6 @@
 // Modal DG stage kernels for affine hexahedra and tetrahedra (gfx950).
 //
-// One stage pass is one launch of DgModalStageKernel (for the exact solver two):
+// One stage pass is one launch of DgModalStageKernel:
 // a workgroup of 256 threads owns G cells; each cell has T = NQ + NF * NFP point
 // tasks (its volume quadrature points and the quadrature points of its faces),
 // one thread per task, volume tasks of all G cells first.
@@ -18,9 +18,9 @@
 // Both cells of a face solve it, from the same two traces formed by the same
 // operations, so the scheme stays conservative without atomics.  That costs the
 // flux twice, and saves writing it once and reading it twice (1.4 KB of a P = 2
-// tetrahedron's 3.4 KB per pass) and a launch.  The exact solver, an iteration
-// of many times an approximate flux, is evaluated once per face point instead, by
-// DgFaceFluxKernel into fhat [face][point][5].
+// tetrahedron's 3.4 KB per pass) and a launch.  The exact solver, which costs many
+// times an approximate flux, is evaluated once per face point on large meshes
+// (DgFacePass), by DgFaceFluxKernel into fhat [face][point][5].
 //
 // What bounds it: no unit is full (P = 2 tetrahedra: FP64 issue 45 %, vector memory
 // 59 %, LDS 37 %, HBM at 56 % of its copy rate); each workgroup passes through three
@@ -31,7 +31,8 @@
 // 146k P = 2 tetrahedra (Roe) 256 -> 195, the four-quadrant problem's 221k (HLLC,
 // with the limiter) 507 -> 417, 750 tetrahedra 15.5 -> 10.2, 64k P = 2 hexahedra
 // 208 -> 157, 83k P = 1 tetrahedra 83 -> 68; the same cell pass after a face
-// pass: 227, 467, 13.6, 179 and 78.  Measured and no better: the neighbours'
+// pass: 227, 467, 13.6, 179 and 78.  With the exact solver, the Sod tube's 3840
+// tetrahedra 41 -> 14, 24.6k 106 -> 52 (most of it the solver itself).  Measured and no better: the neighbours'
 // coefficients loaded once per face and handed round through LDS (a third of the
 // vector memory work, 200), 5 wavefronts per SIMD (200), moments on two
 // wavefronts (212), 3 cells per workgroup (215).
@@ -158,7 +159,8 @@ __device__ __forceinline__ double GroupSum(double v) {
   return v;
 }
 
-template <bool kHex, int P, int kRiemann>
+// kFacePass (exact solver): the faces' w Fhat are read from fhat.
+template <bool kHex, int P, int kRiemann, bool kFacePass>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void DgModalStageKernel(DgModalArgs a) {
   using S = DgShape<kHex, P>;
   constexpr int N = S::kN, NQ = S::kNQ, NF = S::kNF, NFP = S::kNFP, T = S::kT, G = S::kG, PK = S::kPacked;
@@ -211,7 +213,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void D
       const int orient = (info.x >> 3) & 15;
 #pragma unroll
       for (int d = 0; d < 3; ++d) eta[d] = tb->face_eta[lf][holder ? 0 : orient][q][d];
-      if constexpr (kRiemann == kExact) {
+      if constexpr (kFacePass) {
         const double *src = a.fhat + ((int64_t)(info.x >> 8) * NFP + q) * 5;
 #pragma unroll
         for (int k = 0; k < 5; ++k) fw[k] = src[k];
@@ -221,21 +223,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void D
         for (int d = 0; d < 3; ++d) n[d] = fc[d];
         area = fc[6];
         wl = tb->face_w[q];
-        if (info.y >= 0) {
-          const double *eta_n = tb->face_eta[info.x & 7][holder ? orient : 0][q];
-          const double *jn = a.geo + (int64_t)info.y * GS;
-          double j[10], y[3];
+      }
+      if (!kFacePass && info.y >= 0) {
+        const double *eta_n = tb->face_eta[info.x & 7][holder ? orient : 0][q];
+        const double *jn = a.geo + (int64_t)info.y * GS;
+        double j[10], y[3];
 #pragma unroll
-          for (int i = 0; i < 10; i += 2) {
-            const double2 v = *reinterpret_cast<const double2 *>(jn + i);
-            j[i] = v.x;
-            j[i + 1] = v.y;
-          }
-          Offset(j, eta_n, y);
-          const State other = TraceAt<P>(a.ct + (int64_t)info.y * CT, y);
-#pragma unroll
-          for (int k = 0; k < 5; ++k) fw[k] = other.v[k];
+        for (int i = 0; i < 10; i += 2) {
+          const double2 v = *reinterpret_cast<const double2 *>(jn + i);
+          j[i] = v.x;
+          j[i + 1] = v.y;
         }
+        Offset(j, eta_n, y);
+        const State other = TraceAt<P>(a.ct + (int64_t)info.y * CT, y);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) fw[k] = other.v[k];
       }
     }
   }
@@ -246,56 +248,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void D
     const double *geo = s_geo + g * GS;
     double y[3];
     Offset(geo, eta, y);
-    if (!is_face || kRiemann != kExact) {
-      const State own = TraceAt<P>(s_ct + g * CT, y);
-      if (!is_face) {
-        double *slot = s_vol + (g * NQ + r) * kSlot;
-        // the flux matrix (types.hpp:322-333), times the global weight
-        const double zero[3] = { 0, 0, 0 };
-        const FaceTrace t = TraceOf(own, zero);
-        const double w = MulRn(wl, geo[9]);
-        const double wp = t.p * w;
+    State own;
+    if (!kFacePass || !is_face) own = TraceAt<P>(s_ct + g * CT, y);
+    if (!is_face) {
+      double *slot = s_vol + (g * NQ + r) * kSlot;
+      // the flux matrix (types.hpp:322-333), times the global weight
+      const double zero[3] = { 0, 0, 0 };
+      const FaceTrace t = TraceOf(own, zero);
+      const double w = MulRn(wl, geo[9]);
+      const double wp = t.p * w;
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const double wv = t.v[d] * w;
-          slot[5 * d] = own.v[1 + d] * w;
+      for (int d = 0; d < 3; ++d) {
+        const double wv = t.v[d] * w;
+        slot[5 * d] = own.v[1 + d] * w;
 #pragma unroll
-          for (int e = 0; e < 3; ++e) slot[5 * d + 1 + e] = e == d ? __fma_rn(own.v[1 + e], wv, wp) : own.v[1 + e] * wv;
-          slot[5 * d + 4] = (own.v[4] + t.p) * wv;
-          slot[kSlotY + d] = y[d];
-        }
-      } else {
-        State flux;
-        bool star = false;
-        int kind = kBcSmart;
-        if (info.y < 0) {
-          const int tag = -info.y - 1;
-          kind = a.bc_kind[tag];
-          // the tag's constant state, or this point's value of the tag's
-          // boundary function at the stage time
-          const double *gs = a.bc_point_state
-              ? a.bc_point_state + (((int64_t)(info.x >> 8) - a.n_interior) * NFP + q) * 5 : a.bc_state + tag * 5;
-#pragma unroll
-          for (int k = 0; k < 5; ++k) fw[k] = gs[k];
-        }
-        if (kind == kBcSmart) {
-          State l, r;
-#pragma unroll
-          for (int k = 0; k < 5; ++k) {
-            l.v[k] = holder ? own.v[k] : fw[k];
-            r.v[k] = holder ? fw[k] : own.v[k];
-          }
-          flux = FaceFlux<kRiemann>(n, l, r, star);
-        } else {
-          State given;
-#pragma unroll
-          for (int k = 0; k < 5; ++k) given.v[k] = fw[k];
-          flux = BoundaryFlux(kind, true, n, own, given);
-        }
-        const double wq = MulRn(wl, area);
-#pragma unroll
-        for (int k = 0; k < 5; ++k) fw[k] = flux.v[k] * wq;
+        for (int e = 0; e < 3; ++e) slot[5 * d + 1 + e] = e == d ? __fma_rn(own.v[1 + e], wv, wp) : own.v[1 + e] * wv;
+        slot[5 * d + 4] = (own.v[4] + t.p) * wv;
+        slot[kSlotY + d] = y[d];
       }
+    } else if constexpr (!kFacePass) {
+      State flux;
+      // the exact solver's state of this face point, one copy per side: both cells
+      // solve the same problem with the same inputs every pass
+      uint8_t *state = a.exact_star + ((int64_t)(info.x >> 8) * 2 + (holder ? 0 : 1)) * NFP + q;
+      bool star = kRiemann == kExact ? *state != 0 : false;
+      int kind = kBcSmart;
+      if (info.y < 0) {
+        const int tag = -info.y - 1;
+        kind = a.bc_kind[tag];
+        // the tag's constant state, or this point's value of the tag's
+        // boundary function at the stage time
+        const double *gs = a.bc_point_state
+            ? a.bc_point_state + (((int64_t)(info.x >> 8) - a.n_interior) * NFP + q) * 5 : a.bc_state + tag * 5;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) fw[k] = gs[k];
+      }
+      if (kind == kBcSmart) {
+        State l, r;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+          l.v[k] = holder ? own.v[k] : fw[k];
+          r.v[k] = holder ? fw[k] : own.v[k];
+        }
+        flux = FaceFlux<kRiemann>(n, l, r, star);
+        if constexpr (kRiemann == kExact) *state = star ? 1 : 0;
+      } else {
+        State given;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) given.v[k] = fw[k];
+        flux = BoundaryFlux(kind, true, n, own, given);
+      }
+      const double wq = MulRn(wl, area);
+#pragma unroll
+      for (int k = 0; k < 5; ++k) fw[k] = flux.v[k] * wq;
     }
     if (is_face) {
       // dg/general.hpp:80-88: -w Fhat into the holder, +w Fhat into the sharer
@@ -455,10 +460,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void D
 // (dg/general.hpp:51-55, 70-89 and the boundary fluxes :92-202): one thread per
 // (face, point).  The point is located in the holder through its canonical order
 // and in the sharer through the corner-permutation code, and each trace is
-// evaluated from the cell's Taylor coefficients.  A serial chain (the iteration's
-// pow) bounds it; the default register bound leaves room for it without spills.
-// 3840 tetrahedra of the Sod tube, face and cell pass: 41 -> 29 us with the fluxes
-// of the face normal alone.
+// evaluated from the cell's Taylor coefficients.  For large meshes only (DgFacePass).
 template <bool kHex, int P>
 __global__ __launch_bounds__(256) void DgFaceFluxKernel(DgModalArgs a) {
   constexpr int N = P == 1 ? 4 : 10, NFP = DgShape<kHex, P>::kNFP, GS = kDgGeoStride;
@@ -486,7 +488,8 @@ __global__ __launch_bounds__(256) void DgFaceFluxKernel(DgModalArgs a) {
   };
   const State own = trace(holder, tb->face_eta[hf][0][q]);
   State given;
-  bool star = a.exact_star[w] != 0;  // this face point's state (ExactFlux), kept across calls
+  uint8_t *state = a.exact_star + (f * 2) * NFP + q;  // the holder's copy
+  bool star = *state != 0;  // this face point's state (ExactFlux), kept across calls
   int kind = kBcSmart;
   if (sharer >= 0) {
     given = trace(sharer, tb->face_eta[sf][orient][q]);
@@ -502,7 +505,7 @@ __global__ __launch_bounds__(256) void DgFaceFluxKernel(DgModalArgs a) {
   State flux;
   if (kind == kBcSmart) flux = FaceFlux<kExact>(n, own, given, star);
   else flux = BoundaryFlux(kind, true, n, own, given);
-  a.exact_star[w] = star ? 1 : 0;
+  *state = star ? 1 : 0;
 #pragma unroll
   for (int k = 0; k < 5; ++k) a.fhat[w * 5 + k] = flux.v[k] * wq;
 }
@@ -1072,14 +1075,18 @@ hipError_t LaunchStage(const DgModalArgs &a, hipStream_t stream) {
   constexpr int G = DgShape<kHex, P>::kG;
   const int64_t blocks = (a.n_cells + G - 1) / G;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  constexpr int NFP = DgShape<kHex, P>::kNFP;
+  if (R == kExact && !a.exact_star) return hipErrorInvalidValue;
   if constexpr (R == kExact) {
-    const int64_t fblocks = (a.n_faces * NFP + 255) / 256;
-    if (fblocks > 0x7fffffff || !a.fhat || !a.face_cells || !a.exact_star) return hipErrorInvalidValue;
-    if (fblocks > 0)
+    if (a.fhat) {
+      constexpr int NFP = DgShape<kHex, P>::kNFP;
+      const int64_t fblocks = (a.n_faces * NFP + 255) / 256;
+      if (fblocks < 1 || fblocks > 0x7fffffff || !a.face_cells) return hipErrorInvalidValue;
       hipLaunchKernelGGL((DgFaceFluxKernel<kHex, P>), dim3((unsigned)fblocks), dim3(256), 0, stream, a);
+      hipLaunchKernelGGL((DgModalStageKernel<kHex, P, R, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+      return hipGetLastError();
+    }
   }
-  hipLaunchKernelGGL((DgModalStageKernel<kHex, P, R>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  hipLaunchKernelGGL((DgModalStageKernel<kHex, P, R, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

@@ -73,17 +73,24 @@ struct DgModalArgs {
   // state this pass writes is folded into *dt_min_bits (same arithmetic).
   unsigned long long *dt_min_bits;
   double *flag_rec;       // [cell][kDgFlagRecord] for the WENO detector, or null (no limiter)
-  // exact solver only: w Fhat once per face point into fhat [face][point][5],
-  // then the cells read it.  face_cells [face][3]: holder,
-  // sharer or -(1 + boundary tag), holder face | sharer face << 3 |
-  // orientation << 6.
+  // exact solver on large meshes, else null: w Fhat once per face point into fhat
+  // [face][point][5], then the cells read it.  face_cells [face][3]: holder, sharer
+  // or -(1 + boundary tag), holder face | sharer face << 3 | orientation << 6.
   double *fhat;
   const int32_t *face_cells;
   int64_t n_faces;
-  // exact solver only: [face][point] sign of each face point's last star
-  // velocity (ExactFlux), zero-initialised at creation, updated every pass
+  // exact solver only: [face][holder, sharer][point] sign of each face point's last
+  // star velocity (ExactFlux), zero-initialised at creation, updated every pass
   uint8_t *exact_star;
 };
+
+// Whether a stage evaluates the faces in a pass of their own: with the exact
+// solver (riemann 0), where solving them twice costs more than the launch and the
+// fluxes' way through memory once the chip is full.  Measured, us per stage, cells
+// solving / face pass: P = 2 tetrahedra 4374 20.5 / 20.0, 6000 22.8 / 24.6, 7986
+// 29.7 / 29.1, 10368 33.5 / 31.3, 48000 109 / 83; P = 2 hexahedra 5832 36.2 / 36.7,
+// 8000 45.5 / 43.5, 17576 81 / 67; P = 1 tetrahedra 6000 18.8 / 20.6, 13182 31.7 / 30.1.
+inline bool DgFacePass(int riemann, int64_t n_cells) { return riemann == 0 && n_cells > 8000; }
 
 // Ct = C S for every cell of `us` into `ct`.
 hipError_t LaunchDgTaylorCoefficients(int degree, const double *us, const double *basis, int64_t n_cells,

@@ -31,7 +31,8 @@
 // tasks per flux point, columns and a derivative through LDS: 64^3 p3 900 -> 595
 // us, 30 x 28 x 26 curved p3 113 -> 73, 35 x 37 x 33 p4 322 -> 246, 47 x 41 x 43
 // p2 180 -> 121, 36^3 p4 mixed 368 -> 297, 64^3 p1 147 -> 116, 24 x 25 x 23 p5
-// 185 -> 157, 8^3 p3 10.6 -> 9.0 (Roe, p2 HLLC).
+// 185 -> 157, 8^3 p3 10.6 -> 9.0 (Roe, p2 HLLC); exact solver 24^3 p3 350 -> 63,
+// 32^3 p2 531 -> 88 (most of it the solver itself, FastExactState).
 #include "fr_hex.hpp"
 
 #include <algorithm>
@@ -464,13 +465,13 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
 // Wavefronts per SIMD to leave room for: what the registers allow without
 // spills (whose traffic has cost more than a wavefront every time).  Q = 4 mixed
 // with 4 and 76 B of spills: 48^3 428 us instead of 322.
-template <int Q, int kRiemann>
+template <int Q>
 constexpr int LineWaves() {
-  return kRiemann == kExact ? 2 : ((Q <= 3 || Q == 6 ? 4 : 3));
+  return Q <= 3 || Q == 6 ? 4 : 3;
 }
 
 template <int Q, int kRiemann, bool kMixed, bool kCurved>
-__global__ __launch_bounds__(Shape<Q>::kThreads) __attribute__((amdgpu_waves_per_eu(LineWaves<Q, kRiemann>())))
+__global__ __launch_bounds__(Shape<Q>::kThreads) __attribute__((amdgpu_waves_per_eu(LineWaves<Q>())))
 void FrHexStageKernel(FrHexArgs a, LineTables lt) {
   __shared__ double lds[Shape<Q>::kLdsDoubles];
   int64_t block = LogicalBlock(a.xcd_remap);
@@ -769,7 +770,7 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
 }
 
 template <int kCells, int kRiemann, bool kCurved>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kRiemann == kExact ? 2 : 4)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 void FrHexCellKernel(FrHexArgs a, LineTables lt) {
   __shared__ __attribute__((aligned(16))) double lds[CellShape<kCells>::kLdsDoubles];
   constexpr int kPerTile = Shape<4>::kCells / kCells;
@@ -797,7 +798,7 @@ __device__ __noinline__ void BatchBody(const FrHexBatchGroup *g, int64_t block, 
 // cells -- stay in one XCD's L2.  LDS is sized at launch for the largest block
 // in use.
 template <int kRiemann, bool kMixed>
-__global__ __launch_bounds__(Shape<4>::kThreads) __attribute__((amdgpu_waves_per_eu(kRiemann == kExact ? 2 : 3))) void FrHexBatchKernel(FrHexBatchArgs b) {
+__global__ __launch_bounds__(Shape<4>::kThreads) __attribute__((amdgpu_waves_per_eu(3))) void FrHexBatchKernel(FrHexBatchArgs b) {
   extern __shared__ double lds[];
   const int64_t w = blockIdx.x, nw = gridDim.x;
   const int64_t begin = w * b.n_items / nw, end = (w + 1) * b.n_items / nw;
@@ -867,8 +868,7 @@ __global__ __launch_bounds__(256) void FrHexTimeStepKernel(const double *u, cons
 // halve the wavefronts, so a mesh that does not fill the chip with one cell per
 // wavefront (256 CUs, 16 wavefronts each) is better served that way.  Measured,
 // one against two cells, us per pass: 12^3 11.1 / 12.6, 16^3 16.4 / 16.7, 18^3
-// 21.5 / 21.0, 20^3 26.9 / 25.5, 32^3 90.5 / 84.5, 64^3 638 / 595.  The exact
-// solver keeps one: two spill (24^3 250 us against 218).
+// 21.5 / 21.0, 20^3 26.9 / 25.5, 32^3 90.5 / 84.5, 64^3 638 / 595.
 constexpr int64_t kPairCells = 4096;
 
 template <int Q, int R>
@@ -880,13 +880,12 @@ hipError_t Launch(const FrHexArgs &args, const LineTables &lt, hipStream_t strea
   if constexpr (Q == 4) {
     if (!args.mixed) {
       if (blocks * C > 0x7fffffff || !args.cell_ops) return hipErrorInvalidValue;
-      const bool pair = R != kExact && args.n_cells > kPairCells;
+      const bool pair = args.n_cells > kPairCells;
       const dim3 cells((unsigned)(blocks * (pair ? C / 2 : C))), wave(64);
-      if constexpr (R != kExact) {
-        if (pair && args.curved) hipLaunchKernelGGL((FrHexCellKernel<2, R, true>), cells, wave, 0, stream, args, lt);
-        else if (pair) hipLaunchKernelGGL((FrHexCellKernel<2, R, false>), cells, wave, 0, stream, args, lt);
-      }
-      if (!pair) {
+      if (pair) {
+        if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<2, R, true>), cells, wave, 0, stream, args, lt);
+        else hipLaunchKernelGGL((FrHexCellKernel<2, R, false>), cells, wave, 0, stream, args, lt);
+      } else {
         if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<1, R, true>), cells, wave, 0, stream, args, lt);
         else hipLaunchKernelGGL((FrHexCellKernel<1, R, false>), cells, wave, 0, stream, args, lt);
       }

@@ -41,3 +41,20 @@ def test_workgroup_edges(kind, cells, degree, riemann):
     expect = o.time_step(ref, 0.05)
     assert abs(g.get_time_step(0.05) - expect) <= TOL[riemann] * expect
     g.close()
+
+
+@pytest.mark.parametrize("mesh,degree", [(lambda: meshgen.box_tet(11, 11, 11, jitter=0.1, seed=3), 2),
+                                         (lambda: meshgen.box_tet(12, 12, 10, jitter=0.1, seed=4), 2),
+                                         (lambda: meshgen.box_tet(12, 12, 10, jitter=0.1, seed=5), 1),
+                                         (lambda: meshgen.box_hex(21, 20, 20, shuffle_seed=6), 1)])
+def test_exact_solver_on_both_sides_of_the_face_pass(mesh, degree):
+    """7986 cells solve their own faces; 8640 and 8400 read a face pass."""
+    mesh = mesh()
+    o, g = make_pair(mesh, degree, "exact", MIXED_BCS)
+    u = o.approximate(smooth_state(o.cells()["xyz"]))
+    g.set_solution_column(u)
+    assert rel(g.get_residual_column(), o.residual(u)) <= TOL["exact"]
+    dt = g.get_time_step(0.05)
+    g.rk3_update(0.0, dt)
+    assert rel(g.get_solution_column(), o.rk3(u, dt, 1)) <= TOL["exact"]
+    g.close()
