@@ -261,8 +261,9 @@ int mcfd_limiter_flags(mcfd_solver *h, uint8_t *flags, int64_t *n_troubled);
  *   kind SUPERSONIC_OUTLET: GetFluxOnSupersonicOutlet (euler.hpp:144-151) of `left`;
  *   kind SUBSONIC_INLET / SUBSONIC_OUTLET: GetFluxOnSubsonicInlet / Outlet
  *     (euler.hpp:181-280) of `left` with the given values in `right`.
- * form FR: the FR stage kernels' evaluation (Roe with one reciprocal of rho per
- * side); form DG: the modal-DG face pass's.  frames[n][9] holds the rows
+ * form FR: the stage kernels' evaluation (FR and DG), on the unit normal alone;
+ * form DG: rotated into the frame, solved there and rotated back, as the
+ * reference does.  frames[n][9] holds the rows
  * (n, t, b) of each point's frame; left, right [n][5] conservative states
  * (right may be null for INVISCID_WALL and SUPERSONIC_OUTLET); flux [n][5] out.  exact_star[n]
  * (in/out, may be null = fresh solvers) is each point's exact-solver state:

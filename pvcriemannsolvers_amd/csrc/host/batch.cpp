@@ -60,12 +60,13 @@ struct mcfd_batch {
       dst.args = grp.Args(stage, 0.0);
       dst.args.case_dt = case_dt.ptr;
       dst.lt = grp.lt;
+      dst.mt = grp.mt;
       dst.q = grp.q;
       dst.tile = only_group >= 0 && tile >= 0 ? tile : tiles[g];
       dst.first_item = items;
-      const int cells = mcfd::FrHexTileCells(grp.q, dst.tile);
+      const int cells = mcfd::FrHexTileCells(grp.q, dst.tile, mixed);
       items += (grp.n_cells + cells - 1) / cells;
-      *max_lds = std::max(*max_lds, mcfd::FrHexTileLdsBytes(grp.q, dst.tile));
+      *max_lds = std::max(*max_lds, mcfd::FrHexTileLdsBytes(grp.q, dst.tile, mixed));
       out.push_back(dst);
     }
     *n_items = items;
@@ -105,7 +106,7 @@ struct mcfd_batch {
       for (auto &g : groups) {
         auto a = g->Args(stage, 0.0);
         a.case_dt = case_dt.ptr;
-        Check(mcfd::LaunchFrHexStage(g->q, riemann, a, g->lt, stream), "group stage launch");
+        Check(mcfd::LaunchFrHexStage(g->q, riemann, a, g->lt, g->mt, stream), "group stage launch");
       }
     }
   }
@@ -281,7 +282,7 @@ int mcfd_batch_get_time_steps(mcfd_batch *b, double cfl, double *dt) {
     for (int c = 0; c < b->n_cases; ++c) {
       const auto &ref = b->cases[c];
       const auto &g = *b->groups[ref.group];
-      Check(mcfd::LaunchFrHexTimeStep(g.q, g.u0.ptr + ref.first_cell * g.np * 5, g.geo_id.ptr + ref.first_cell,
+      Check(mcfd::LaunchFrHexTimeStep(g.q, g.mixed, g.u0.ptr + ref.first_cell * g.np * 5, g.geo_id.ptr + ref.first_cell,
                                       g.geo.ptr, ref.n_cells, b->scratch.ptr + c, b->stream), "time step launch");
     }
     Check(hipMemcpyAsync(bits.data(), b->scratch.ptr, bits.size() * sizeof(bits[0]), hipMemcpyDeviceToHost,

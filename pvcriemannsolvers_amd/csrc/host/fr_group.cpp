@@ -1,5 +1,6 @@
 // FrHexGroup: host construction and device upload of one FR mesh.
 #include "fr_group.hpp"
+#include "../kernels/fr_mixed.hpp"
 
 #include <algorithm>
 #include <climits>
@@ -210,15 +211,12 @@ void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &schem
   double dg[kMaxQ][kMaxQ];
   for (int m = 0; m < q; ++m) {
     lt.end[m] = LagrangeValue(q, x1d.data(), m, -1.0);
-    lt.lend[0][m] = (float)LagrangeValue(q, x1d.data(), m, -1.0);
-    lt.lend[1][m] = (float)LagrangeValue(q, x1d.data(), m, +1.0);
     lt.gp[0][m] = CorrectionLeftDerivative(degree, scheme.c_next, x1d[m]);
     lt.gp[1][m] = CorrectionRightDerivative(degree, scheme.c_next, x1d[m]);
   }
   for (int i = 0; i < q; ++i)
     for (int m = 0; m < q; ++m) {
       const double d = LagrangeDerivative(q, x1d.data(), m, x1d[i]);
-      lt.d[i][m] = (float)d;
       dg[i][m] = d - lt.gp[0][i] * lt.end[m] - lt.gp[1][i] * lt.end[q - 1 - m];
     }
   for (int i = 0; i < q; ++i)
@@ -246,6 +244,10 @@ void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &schem
   if (curved) {
     if (mixed) throw Failure{ MCFD_ENOTSUP, "the mixed-precision form supports affine hexahedra only" };
     BuildCurved(scheme);
+    return;
+  }
+  if (mixed) {
+    BuildMixed(mesh, scheme);
     return;
   }
 
@@ -297,6 +299,86 @@ void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &schem
   });
 }
 
+// The mixed form's tables and records (fr_mixed.hip), affine cells.
+void FrHexGroup::BuildMixed(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &scheme) {
+  const int64_t nc = mesh.n_cells;
+  for (int i = 0; i < q; ++i)
+    for (int m = 0; m < q; ++m) mt.d[i][m] = LagrangeDerivative(q, x1d.data(), m, x1d[i]);
+  for (int m = 0; m < q; ++m) {
+    mt.lend[0][m] = LagrangeValue(q, x1d.data(), m, -1.0);
+    mt.lend[1][m] = LagrangeValue(q, x1d.data(), m, +1.0);
+    mt.gp[0][m] = CorrectionLeftDerivative(degree, scheme.c_next, x1d[m]);
+    mt.gp[1][m] = CorrectionRightDerivative(degree, scheme.c_next, x1d[m]);
+  }
+
+  // geometry records, deduplicated bitwise
+  std::map<std::array<double, kMixedGeoStride>, int32_t> geo_ids;
+  h_geo.clear();
+  h_geo_id.assign(nc, 0);
+  corner0.resize(nc);
+  for (int64_t c = 0; c < nc; ++c) {
+    const auto &j = conn.jac[c];
+    double d = conn.det[c];
+    // J* = det(J) J^{-1} is the adjugate of J
+    std::array<double, kMixedGeoStride> g{};
+    g[0] = j[4] * j[8] - j[5] * j[7]; g[1] = j[2] * j[7] - j[1] * j[8]; g[2] = j[1] * j[5] - j[2] * j[4];
+    g[3] = j[5] * j[6] - j[3] * j[8]; g[4] = j[0] * j[8] - j[2] * j[6]; g[5] = j[2] * j[3] - j[0] * j[5];
+    g[6] = j[3] * j[7] - j[4] * j[6]; g[7] = j[1] * j[6] - j[0] * j[7]; g[8] = j[0] * j[4] - j[1] * j[3];
+    g[9] = 1.0 / d;
+    for (int f = 0; f < 6; ++f) {
+      int dir = kHexFaceNormalDir[f];
+      double n = std::sqrt(g[dir] * g[dir] + g[3 + dir] * g[3 + dir] + g[6 + dir] * g[6 + dir]);
+      g[10 + f] = kHexFaceSide[f] ? n : -n;
+    }
+    g[16] = std::cbrt(8 * d) * 0.5;  // mesh/part.hpp:230, volume = 8 det(J)
+    auto it = geo_ids.find(g);
+    if (it == geo_ids.end()) {
+      it = geo_ids.emplace(g, (int32_t)geo_ids.size()).first;
+      h_geo.insert(h_geo.end(), g.begin(), g.end());
+    }
+    h_geo_id[c] = it->second;
+    int64_t n0 = mesh.cell_nodes[8 * c];
+    corner0[c] = { mesh.coords[3 * n0], mesh.coords[3 * n0 + 1], mesh.coords[3 * n0 + 2] };
+  }
+  diag_metric = true;
+  for (size_t r = 0; r < h_geo.size(); r += kMixedGeoStride)
+    for (int e = 0; e < 9; ++e)
+      if (e % 4 != 0 && h_geo[r + e] != 0.0) diag_metric = false;
+
+  // per-cell face records
+  std::map<std::array<double, kFrameStride>, int32_t> frame_ids;
+  h_frames.clear();
+  h_nbr.assign(6 * nc, INT32_MIN);
+  h_finfo.assign(6 * nc, 0);
+  for (const auto &face : conn.faces) {
+    std::array<double, kFrameStride> fr;
+    std::copy(face.frame, face.frame + 6, fr.begin());
+    auto it = frame_ids.find(fr);
+    if (it == frame_ids.end()) {
+      it = frame_ids.emplace(fr, (int32_t)frame_ids.size()).first;
+      h_frames.insert(h_frames.end(), fr.begin(), fr.end());
+    }
+    int32_t fid = it->second;
+    if (fid >= (1 << 24)) throw Failure{ MCFD_ENOTSUP, "too many distinct face frames" };
+    int64_t hs = face.holder * 6 + face.holder_face;
+    if (face.sharer >= 0) {
+      int64_t ss = face.sharer * 6 + face.sharer_face;
+      h_nbr[hs] = (int32_t)face.sharer;
+      h_finfo[hs] = (fid << 7) | (1 << 6) | (face.orient << 3) | face.sharer_face;
+      h_nbr[ss] = (int32_t)face.holder;
+      h_finfo[ss] = (fid << 7) | (InverseOrient(face.orient) << 3) | face.holder_face;
+    } else {
+      h_nbr[hs] = -(1 + face.tag);
+      h_finfo[hs] = (fid << 7) | (1 << 6);
+    }
+  }
+  for (auto v : h_nbr)
+    if (v == INT32_MIN) throw std::invalid_argument("cell face without a face record");
+  h_bface_of.assign(6 * nc, -1);
+  for (size_t f = conn.n_interior; f < conn.faces.size(); ++f)
+    h_bface_of[conn.faces[f].holder * 6 + conn.faces[f].holder_face] = (int32_t)(f - conn.n_interior);
+}
+
 void FrHexGroup::BoundaryPoints(std::vector<int32_t> *tags, std::vector<double> *xyz) const {
   const int64_t nb = (int64_t)conn.faces.size() - conn.n_interior;
   tags->assign(nb, 0);
@@ -331,6 +413,12 @@ void FrHexGroup::Upload(hipStream_t stream) {
   size_t cs = ColumnSize();
   u0.Allocate(cs); u1.Allocate(cs); u2.Allocate(cs); res.Allocate(cs);
   Check(hipMemsetAsync(u0.ptr, 0, cs * sizeof(double), stream), "memset");
+  if (mixed) {
+    nbr.Upload(h_nbr, stream);
+    finfo.Upload(h_finfo, stream);
+    frames.Upload(h_frames, stream);
+    bface_of.Upload(h_bface_of, stream);
+  }
   faces.Upload(h_faces, stream);
   geo_id.Upload(h_geo_id, stream);
   geo.Upload(h_geo, stream);
@@ -392,14 +480,15 @@ void FrHexGroup::BuildTileOrder(int tile_cells) {
 void FrHexGroup::SetColumn(const double *column, int64_t first_cell, int64_t count, ColumnCopy *copy,
                            hipStream_t stream) {
   const size_t at = size_t(first_cell) * np * 5, n = size_t(count) * np * 5;
-  copy->ToDevice(res.ptr + at, column, n * sizeof(double), stream);
+  copy->ToDevice((mixed ? u0.ptr : res.ptr) + at, column, n * sizeof(double), stream);
+  if (mixed) return;
   Check(LaunchFrLayout(true, res.ptr + at, u0.ptr + at, np, count, stream), "set solution layout");
 }
 
 void FrHexGroup::GetColumn(double *column, int64_t first_cell, int64_t count, ColumnCopy *copy, hipStream_t stream) {
   const size_t at = size_t(first_cell) * np * 5, n = size_t(count) * np * 5;
-  Check(LaunchFrLayout(false, u0.ptr + at, res.ptr + at, np, count, stream), "get solution layout");
-  copy->ToHost(column, res.ptr + at, n * sizeof(double), stream);
+  if (!mixed) Check(LaunchFrLayout(false, u0.ptr + at, res.ptr + at, np, count, stream), "get solution layout");
+  copy->ToHost(column, (mixed ? u0.ptr : res.ptr) + at, n * sizeof(double), stream);
 }
 
 FrHexArgs FrHexGroup::Args(int stage, double dt) const {
@@ -421,6 +510,10 @@ FrHexArgs FrHexGroup::Args(int stage, double dt) const {
   a.bc_point_state = nullptr;  // set by the caller when boundary functions are in use
   a.any_swap = any_swap ? 1 : 0;
   a.mixed = mixed ? 1 : 0;
+  a.nbr = nbr.ptr; a.finfo = finfo.ptr;
+  a.frames = frames.ptr;
+  a.bface_of = bface_of.ptr;
+  a.diag_metric = diag_metric ? 1 : 0;
   a.curved = curved ? 1 : 0;
   a.col_node = col_node.ptr;
   a.inv_det_node = inv_det.ptr;

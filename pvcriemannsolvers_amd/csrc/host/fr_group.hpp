@@ -25,6 +25,7 @@ struct FrHexGroup {
   int64_t n_cells = 0;
   HexConnectivity conn;
   LineTables lt;
+  MixedTables mt{};  // mixed form
   std::vector<double> x1d, w1d;  // 1-D solution points and their quadrature weights
   std::vector<std::array<double, 3>> corner0;  // node 0 of each cell
   // host copies uploaded by Upload()
@@ -36,7 +37,12 @@ struct FrHexGroup {
   // flux-point normals and scales [cell][6][Q * Q][4]
   std::vector<double> h_col_node, h_inv_det, h_face_point;
   DeviceArray<double> col_node, inv_det, face_point;
-  DeviceArray<double> u0, u1, u2;  // states in planes (FrHexArgs)
+  // mixed form (FrHexArgs)
+  std::vector<int32_t> h_nbr, h_finfo, h_bface_of;
+  std::vector<double> h_frames;
+  DeviceArray<int32_t> nbr, finfo, bface_of;
+  DeviceArray<double> frames;
+  DeviceArray<double> u0, u1, u2;  // states in planes (FrHexArgs); mixed form: columns
   DeviceArray<double> res;         // residual column, and staging of columns in and out
   DeviceArray<FrFace> faces;
   DeviceArray<CellOps> ops;
@@ -50,6 +56,7 @@ struct FrHexGroup {
   void Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &scheme,
              const std::vector<int32_t> &bc_kinds, const std::vector<double> &bc_states);
   void BuildCurved(const mcfd_scheme_desc &scheme);
+  void BuildMixed(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &scheme);
   template <class NormalOf> void BuildFaceRecords(NormalOf &&normal_of);
   // Order in which the stage kernel sweeps its tiles of `tile_cells`
   // consecutive cells: Morton order of the tile centres, so that the tiles in

@@ -64,7 +64,8 @@ struct mcfd_solver {
       mcfd::FrHexArgs a = group.Args(stage, dt);
       a.dt_min_bits = fuse_dt ? scratch.ptr : nullptr;
       a.bc_point_state = bc_points;
-      Check(mcfd::LaunchFrHexStage(group.q, group.riemann, a, group.lt, stream), "FR stage launch");
+      Check(mcfd::LaunchFrHexStage(group.q, group.riemann, a, group.lt, group.mt, stream),
+            "FR stage launch");
     }
     if (fuse_dt) dt_fresh = dt_pending = true;
   }
@@ -137,7 +138,7 @@ int mcfd_create(const mcfd_mesh_desc *mesh, const mcfd_scheme_desc *scheme, cons
     if (h->dg) {
       h->modal.Upload(h->stream);
     } else {
-      h->group.BuildTileOrder(mcfd::FrHexStageTileCells(h->group.q));
+      h->group.BuildTileOrder(mcfd::FrHexStageTileCells(h->group.q, h->group.mixed));
       h->group.Upload(h->stream);
     }
     h->scratch.Allocate(1);
@@ -246,7 +247,7 @@ int mcfd_get_time_step(mcfd_solver *h, double cfl, double dt_guess, double *dt) 
       if (h->dg) {
         h->modal.TimeStepBits(h->scratch.ptr, h->stream);
       } else {
-        Check(mcfd::LaunchFrHexTimeStep(h->group.q, h->group.u0.ptr, h->group.geo_id.ptr, h->group.geo.ptr,
+        Check(mcfd::LaunchFrHexTimeStep(h->group.q, h->group.mixed, h->group.u0.ptr, h->group.geo_id.ptr, h->group.geo.ptr,
                                         h->group.n_cells, h->scratch.ptr, h->stream), "time step launch");
       }
       h->dt_fresh = true;
@@ -369,7 +370,7 @@ int mcfd_startup_limiter(mcfd_solver *h, int32_t kind) {
       mcfd::DeviceArray<double> d_wl, d_det;
       d_wl.Upload(wl, h->stream);
       d_det.Upload(g.NodeDeterminants(), h->stream);
-      Check(mcfd::LaunchFrAverage(g.u0.ptr, d_wl.ptr, d_det.ptr, g.n_cells, g.np, h->stream), "average launch");
+      Check(mcfd::LaunchFrAverage(g.u0.ptr, d_wl.ptr, d_det.ptr, g.n_cells, g.np, !g.mixed, h->stream), "average launch");
       Check(hipStreamSynchronize(h->stream), "average sync");
       return;
     }
@@ -377,12 +378,12 @@ int mcfd_startup_limiter(mcfd_solver *h, int32_t kind) {
     mcfd::DeviceArray<int32_t> failed;
     value.Allocate(size_t(g.n_cells) * 5);
     failed.Upload(std::vector<int32_t>{ 0 }, h->stream);
-    Check(mcfd::LaunchFrMajority(g.u0.ptr, value.ptr, failed.ptr, g.n_cells, g.np, h->stream), "majority launch");
+    Check(mcfd::LaunchFrMajority(g.u0.ptr, value.ptr, failed.ptr, g.n_cells, g.np, !g.mixed, h->stream), "majority launch");
     int32_t bad = 0;
     Check(hipMemcpyAsync(&bad, failed.ptr, sizeof(bad), hipMemcpyDeviceToHost, h->stream), "majority flag");
     Check(hipStreamSynchronize(h->stream), "majority sync");
     if (bad) throw mcfd::Failure{ MCFD_EINVAL, "majority limiter: a cell component has no value held by more than half of its nodes" };
-    Check(mcfd::LaunchFrSetNodes(g.u0.ptr, value.ptr, g.n_cells, g.np, h->stream), "majority set");
+    Check(mcfd::LaunchFrSetNodes(g.u0.ptr, value.ptr, g.n_cells, g.np, !g.mixed, h->stream), "majority set");
     Check(hipStreamSynchronize(h->stream), "majority sync");
   });
 }

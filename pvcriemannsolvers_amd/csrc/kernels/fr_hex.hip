@@ -30,16 +30,16 @@
 // costs four lanes one cache line.  Per pass, against one thread per node with
 // tasks per flux point, columns and a derivative through LDS: 64^3 p3 900 -> 595
 // us, 30 x 28 x 26 curved p3 113 -> 73, 35 x 37 x 33 p4 322 -> 246, 47 x 41 x 43
-// p2 180 -> 121, 36^3 p4 mixed 368 -> 297, 64^3 p1 147 -> 116, 24 x 25 x 23 p5
+// p2 180 -> 121, 64^3 p1 147 -> 116, 24 x 25 x 23 p5
 // 185 -> 157, 8^3 p3 10.6 -> 9.0 (Roe, p2 HLLC); exact solver 24^3 p3 350 -> 63,
 // 32^3 p2 531 -> 88 (most of it the solver itself, FastExactState).
 #include "fr_hex.hpp"
 
 #include <algorithm>
-#include <type_traits>
 
 #include "euler.hpp"
 #include "fr_common.hpp"
+#include "fr_mixed.hpp"
 
 namespace mcfd {
 
@@ -102,16 +102,9 @@ __device__ __forceinline__ void Pin(T *v) {
   for (int k = 0; k < 5; ++k) asm volatile("" : "+v"(v[k]));
 }
 
-// kMixed: the F~ lines are contracted as FP32 deviations from the value at the
-// cell's first solution point, with FP32 FMAs (each row of the derivative
-// matrix sums to zero, so the FP64 reference value drops out of the
-// divergence); each line's FP32 partial is accumulated in FP64.  States,
-// pressure recovery, traces, the Riemann solve, the flux gaps and the RK
-// combination stay FP64.
-//
 // kCurved (trilinear cells): J* and 1/det(J) are read per solution point, the
 // normal and the scale per cell flux point instead of per cell and per face.
-template <int Q, int kRiemann, bool kMixed, bool kCurved>
+template <int Q, int kRiemann, bool kCurved>
 __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables &lt, int64_t block, double *lds) {
   using S = Shape<Q>;
   constexpr int NP = S::kPoints, NL = S::kLines, C = S::kCells, PAD = S::kPad, DL = S::kDirLanes;
@@ -315,33 +308,18 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
 
   // ---- F~_r along the line, contracted node by node, so that only the Q x 5
   // sums stay in registers; then the fluxes lifted
-  typedef typename std::conditional<kMixed, float, double>::type Sum;
-  Sum d[S::kRows][5];
-  Sum gap_end[2][5];  // mixed: F~_r's deviation at the line's ends
-  // Nodes are taken upwards, and inwards from the lane's end of a split line:
-  // the tables' symmetry leaves the sums there with the opposite sign.  FP32
-  // sums keep one order for all rows, and the upper lane its own table rows.
-  const bool inwards = S::kSplit && !kMixed && half == 1;
+  double d[S::kRows][5];
+  // Nodes are taken upwards, and mirror from the lane's end of a split line:
+  // the tables' symmetry leaves the sums there with the opposite sign.
   const bool mirror = S::kSplit && half == 1;
-  const int first_pos = pos0 + (inwards ? (Q - 1) * pos_step : 0), node_step = inwards ? -pos_step : pos_step;
-  double ref[5];      // mixed: F~_r of the cell's first solution point, formed by every line alike
+  const int first_pos = pos0 + (mirror ? (Q - 1) * pos_step : 0), node_step = mirror ? -pos_step : pos_step;
   if (active) {
-    const double *col_src = kCurved ? a.col_node + ((c * 3 + dir) * NP + node0 + (inwards ? (Q - 1) * stride : 0)) * 3 : nullptr;
-    const int col_step = inwards ? -3 * stride : 3 * stride;
+    const double *col_src = kCurved ? a.col_node + ((c * 3 + dir) * NP + node0 + (mirror ? (Q - 1) * stride : 0)) * 3 : nullptr;
+    const int col_step = mirror ? -3 * stride : 3 * stride;
     double col[3], next[3] = { dir_col[0], dir_col[1], dir_col[2] };
     if constexpr (kCurved) {
 #pragma unroll
       for (int e = 0; e < 3; ++e) next[e] = col_src[e];
-    }
-    if constexpr (kMixed) {
-      State first;
-#pragma unroll
-      for (int k = 0; k < 5; ++k) first.v[k] = lds[cell * 5 * PAD + k * PAD];
-      const FaceTrace t = TraceOf(first, dir_col);
-      ref[0] = first.v[1] * dir_col[0] + first.v[2] * dir_col[1] + first.v[3] * dir_col[2];
-#pragma unroll
-      for (int e = 0; e < 3; ++e) ref[1 + e] = first.v[1 + e] * t.un + t.p * dir_col[e];
-      ref[4] = (first.v[4] + t.p) * t.un;
     }
 #pragma unroll
     for (int m = 0; m < Q; ++m) {
@@ -370,26 +348,12 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
 #pragma unroll
       for (int k = 0; k < 5; ++k) {
         const double f = k == 0 ? mom : (k == 4 ? (w[4] + p) * vel : w[k] * vel + p * col[k == 0 ? 0 : k - 1]);
-        if constexpr (kMixed) {
-          const float dev = (float)(f - ref[k]);
-#pragma unroll
-          for (int i = 0; i < S::kRows; ++i)
-            d[i][k] = __fmaf_rn(mirror ? lt.d[Q - 1 - i][m] : lt.d[i][m], dev, m ? d[i][k] : 0.0f);
-#pragma unroll
-          for (int s = 0; s < 2; ++s)
-            gap_end[s][k] = m ? __fmaf_rn(lt.lend[s][m], dev, gap_end[s][k]) : lt.lend[s][0] * dev;
-        } else {
-#pragma unroll
-          for (int i = 0; i < S::kRows; ++i)
-            d[i][k] = m ? __fma_rn(DerivativeEntry<Q>(lt, i, m), f, d[i][k]) : DerivativeEntry<Q>(lt, i, 0) * f;
-        }
+        #pragma unroll
+        for (int i = 0; i < S::kRows; ++i)
+          d[i][k] = m ? __fma_rn(DerivativeEntry<Q>(lt, i, m), f, d[i][k]) : DerivativeEntry<Q>(lt, i, 0) * f;
       }
 #pragma unroll
       for (int i = 0; i < S::kRows; ++i) Pin(d[i]);  // else the sums are put off and all nodes' fluxes stay in registers
-      if constexpr (kMixed) {
-        Pin(gap_end[0]);
-        Pin(gap_end[1]);
-      }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -400,16 +364,9 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
     for (int k = 0; k < 5; ++k) {
       // the lower and the upper end's gap; of a split line the near and the far end's
       double gap[2] = { flux[0][k], S::kSplit ? far_flux[k] : flux[S::kEnds - 1][k] };
-      if constexpr (kMixed) {
-#pragma unroll
-        for (int s = 0; s < 2; ++s)  // less F~_r at the ends
-          gap[s] -= ref[k] + (double)(mirror ? gap_end[1 - s][k] : gap_end[s][k]);
-      }
 #pragma unroll
       for (int i = 0; i < S::kRows; ++i) {
-        double sum = (double)d[i][k];
-        if (kMixed && mirror) sum = -sum;
-        sum = __fma_rn(lt.gp[0][i], gap[0], sum);
+        double sum = __fma_rn(lt.gp[0][i], gap[0], d[i][k]);
         sum = __fma_rn(-lt.gp[0][Q - 1 - i], gap[1], sum);
         if (mirror) sum = -sum;
         const int at = k * PAD + (mirror ? Q - 1 - i : i) * pos_step;
@@ -463,20 +420,19 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
 }
 
 // Wavefronts per SIMD to leave room for: what the registers allow without
-// spills (whose traffic has cost more than a wavefront every time).  Q = 4 mixed
-// with 4 and 76 B of spills: 48^3 428 us instead of 322.
+// spills (whose traffic has cost more than a wavefront every time).
 template <int Q>
 constexpr int LineWaves() {
   return Q <= 3 || Q == 6 ? 4 : 3;
 }
 
-template <int Q, int kRiemann, bool kMixed, bool kCurved>
+template <int Q, int kRiemann, bool kCurved>
 __global__ __launch_bounds__(Shape<Q>::kThreads) __attribute__((amdgpu_waves_per_eu(LineWaves<Q>())))
 void FrHexStageKernel(FrHexArgs a, LineTables lt) {
   __shared__ double lds[Shape<Q>::kLdsDoubles];
   int64_t block = LogicalBlock(a.xcd_remap);
   if (a.tile_order) block = a.tile_order[block];
-  FrLineBody<Q, kRiemann, kMixed, kCurved>(a, lt, block, lds);
+  FrLineBody<Q, kRiemann, kCurved>(a, lt, block, lds);
 }
 
 // ------------------------------------------------------------ Q = 4, FP64
@@ -787,9 +743,9 @@ constexpr int TileBlocks(int tile) { return 1 << tile; }
 
 // One out-of-line body per Q: each is register-allocated on its own within the
 // kernel's budget, where the inlined bodies would share one allocation.
-template <int Q, int kRiemann, bool kMixed>
+template <int Q, int kRiemann>
 __device__ __noinline__ void BatchBody(const FrHexBatchGroup *g, int64_t block, double *lds) {
-  FrLineBody<Q, kRiemann, kMixed, false>(g->args, g->lt, block, lds);
+  FrLineBody<Q, kRiemann, false>(g->args, g->lt, block, lds);
 }
 
 // Persistent batched pass: workgroup w processes the contiguous item range
@@ -797,7 +753,7 @@ __device__ __noinline__ void BatchBody(const FrHexBatchGroup *g, int64_t block, 
 // degree groups in order), so consecutive blocks -- and their neighbour
 // cells -- stay in one XCD's L2.  LDS is sized at launch for the largest block
 // in use.
-template <int kRiemann, bool kMixed>
+template <int kRiemann>
 __global__ __launch_bounds__(Shape<4>::kThreads) __attribute__((amdgpu_waves_per_eu(3))) void FrHexBatchKernel(FrHexBatchArgs b) {
   extern __shared__ double lds[];
   const int64_t w = blockIdx.x, nw = gridDim.x;
@@ -812,9 +768,9 @@ __global__ __launch_bounds__(Shape<4>::kThreads) __attribute__((amdgpu_waves_per
     for (int v = 0; v < blocks; ++v) {
       const int64_t block = (item - g.first_item) * blocks + v;
       switch (g.q) {
-      case 2: BatchBody<2, kRiemann, kMixed>(&g, block, lds); break;
-      case 3: BatchBody<3, kRiemann, kMixed>(&g, block, lds); break;
-      default: BatchBody<4, kRiemann, kMixed>(&g, block, lds); break;
+      case 2: BatchBody<2, kRiemann>(&g, block, lds); break;
+      case 3: BatchBody<3, kRiemann>(&g, block, lds); break;
+      default: BatchBody<4, kRiemann>(&g, block, lds); break;
       }
       __syncthreads();  // the next block reuses the LDS buffers
     }
@@ -875,29 +831,25 @@ template <int Q, int R>
 hipError_t Launch(const FrHexArgs &args, const LineTables &lt, hipStream_t stream) {
   constexpr int C = Shape<Q>::kCells;
   const int64_t blocks = (args.n_cells + C - 1) / C;
-  if (blocks > 0x7fffffff || (args.curved && args.mixed)) return hipErrorInvalidValue;
+  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks), block(Shape<Q>::kThreads);
   if constexpr (Q == 4) {
-    if (!args.mixed) {
-      if (blocks * C > 0x7fffffff || !args.cell_ops) return hipErrorInvalidValue;
-      const bool pair = args.n_cells > kPairCells;
-      const dim3 cells((unsigned)(blocks * (pair ? C / 2 : C))), wave(64);
-      if (pair) {
-        if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<2, R, true>), cells, wave, 0, stream, args, lt);
-        else hipLaunchKernelGGL((FrHexCellKernel<2, R, false>), cells, wave, 0, stream, args, lt);
-      } else {
-        if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<1, R, true>), cells, wave, 0, stream, args, lt);
-        else hipLaunchKernelGGL((FrHexCellKernel<1, R, false>), cells, wave, 0, stream, args, lt);
-      }
-      return hipGetLastError();
+    if (blocks * C > 0x7fffffff || !args.cell_ops) return hipErrorInvalidValue;
+    const bool pair = args.n_cells > kPairCells;
+    const dim3 cells((unsigned)(blocks * (pair ? C / 2 : C))), wave(64);
+    if (pair) {
+      if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<2, R, true>), cells, wave, 0, stream, args, lt);
+      else hipLaunchKernelGGL((FrHexCellKernel<2, R, false>), cells, wave, 0, stream, args, lt);
+    } else {
+      if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<1, R, true>), cells, wave, 0, stream, args, lt);
+      else hipLaunchKernelGGL((FrHexCellKernel<1, R, false>), cells, wave, 0, stream, args, lt);
     }
+    return hipGetLastError();
   }
   if (args.curved) {
-    hipLaunchKernelGGL((FrHexStageKernel<Q, R, false, true>), grid, block, 0, stream, args, lt);
-  } else if (args.mixed) {
-    hipLaunchKernelGGL((FrHexStageKernel<Q, R, true, false>), grid, block, 0, stream, args, lt);
+    hipLaunchKernelGGL((FrHexStageKernel<Q, R, true>), grid, block, 0, stream, args, lt);
   } else {
-    hipLaunchKernelGGL((FrHexStageKernel<Q, R, false, false>), grid, block, 0, stream, args, lt);
+    hipLaunchKernelGGL((FrHexStageKernel<Q, R, false>), grid, block, 0, stream, args, lt);
   }
   return hipGetLastError();
 }
@@ -914,8 +866,10 @@ hipError_t LaunchQ(int riemann, const FrHexArgs &args, const LineTables &lt, hip
 
 }  // namespace
 
-hipError_t LaunchFrHexStage(int q, int riemann, const FrHexArgs &args, const LineTables &lt,
+hipError_t LaunchFrHexStage(int q, int riemann, const FrHexArgs &args, const LineTables &lt, const MixedTables &mt,
                             hipStream_t stream) {
+  if (args.curved && args.mixed) return hipErrorInvalidValue;
+  if (args.mixed) return LaunchFrMixedStage(q, riemann, args, mt, stream);
   switch (q) {
   case 2: return LaunchQ<2>(riemann, args, lt, stream);
   case 3: return LaunchQ<3>(riemann, args, lt, stream);
@@ -926,7 +880,8 @@ hipError_t LaunchFrHexStage(int q, int riemann, const FrHexArgs &args, const Lin
   }
 }
 
-int FrHexStageTileCells(int q) {
+int FrHexStageTileCells(int q, bool mixed) {
+  if (mixed) return FrMixedStageTileCells(q);
   switch (q) {
   case 2: return Shape<2>::kCells;
   case 3: return Shape<3>::kCells;
@@ -937,29 +892,28 @@ int FrHexStageTileCells(int q) {
   }
 }
 
-int FrHexTileLdsBytes(int q, int tile) {
+int FrHexTileLdsBytes(int q, int tile, bool mixed) {
+  if (mixed) return FrMixedTileLdsBytes(q, tile);
   if (q < 2 || q > 4 || tile < 0 || tile > 2) return 0;
   return (int)sizeof(double) * (q == 2 ? Shape<2>::kLdsDoubles : (q == 3 ? Shape<3>::kLdsDoubles : Shape<4>::kLdsDoubles));
 }
 
-int FrHexTileCells(int q, int tile) {
+int FrHexTileCells(int q, int tile, bool mixed) {
+  if (mixed) return FrMixedTileCells(q, tile);
   if (q < 2 || q > 4 || tile < 0 || tile > 2) return 0;
-  return FrHexStageTileCells(q) * TileBlocks(tile);
+  return FrHexStageTileCells(q, false) * TileBlocks(tile);
 }
 
 hipError_t LaunchFrHexBatch(int riemann, bool mixed, const FrHexBatchArgs &args, int n_workgroups,
                             hipStream_t stream) {
+  if (mixed) return LaunchFrMixedBatch(riemann, args, n_workgroups, stream);
   if (args.n_groups < 1 || args.n_groups > kMaxBatchGroups || n_workgroups < 1) return hipErrorInvalidValue;
   const dim3 grid((unsigned)n_workgroups), block(Shape<4>::kThreads);
   const size_t lds = (size_t)args.max_tile_lds;
   switch (riemann) {
-#define MCFD_BATCH_CASE(R)                                                                        \
-  case R:                                                                                         \
-    if (mixed) hipLaunchKernelGGL((FrHexBatchKernel<R, true>), grid, block, lds, stream, args);   \
-    else hipLaunchKernelGGL((FrHexBatchKernel<R, false>), grid, block, lds, stream, args);        \
-    break;
-  MCFD_BATCH_CASE(kExact) MCFD_BATCH_CASE(kHllc) MCFD_BATCH_CASE(kRoe)
-#undef MCFD_BATCH_CASE
+  case kExact: hipLaunchKernelGGL(FrHexBatchKernel<kExact>, grid, block, lds, stream, args); break;
+  case kHllc: hipLaunchKernelGGL(FrHexBatchKernel<kHllc>, grid, block, lds, stream, args); break;
+  case kRoe: hipLaunchKernelGGL(FrHexBatchKernel<kRoe>, grid, block, lds, stream, args); break;
   default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -968,13 +922,11 @@ hipError_t LaunchFrHexBatch(int riemann, bool mixed, const FrHexBatchArgs &args,
 int FrHexBatchResidentWorkgroups(int riemann, bool mixed, int lds_bytes) {
   int per_cu = 0;
   hipError_t e = hipErrorInvalidValue;
-  switch (riemann * 2 + (mixed ? 1 : 0)) {
-#define MCFD_OCC(R, M) \
-  case R * 2 + M: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<R, M>, Shape<4>::kThreads, lds_bytes); break;
-  MCFD_OCC(kExact, 0) MCFD_OCC(kExact, 1) MCFD_OCC(kHllc, 0) MCFD_OCC(kHllc, 1) MCFD_OCC(kRoe, 0) MCFD_OCC(kRoe, 1)
-#undef MCFD_OCC
-  default: break;
-  }
+  constexpr int kThreads = Shape<4>::kThreads;
+  if (mixed) e = FrMixedBatchResident(riemann, lds_bytes, &per_cu);
+  else if (riemann == kExact) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kExact>, kThreads, lds_bytes);
+  else if (riemann == kHllc) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kHllc>, kThreads, lds_bytes);
+  else if (riemann == kRoe) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kRoe>, kThreads, lds_bytes);
   int dev = 0, cus = 0;
   if (e != hipSuccess || hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -999,8 +951,9 @@ hipError_t LaunchResetTimeStepBits(unsigned long long *bits, hipStream_t stream)
   return hipGetLastError();
 }
 
-hipError_t LaunchFrHexTimeStep(int q, const double *u, const int32_t *geo_id, const double *geo,
+hipError_t LaunchFrHexTimeStep(int q, bool mixed, const double *u, const int32_t *geo_id, const double *geo,
                                int64_t n_cells, unsigned long long *dt_min_bits, hipStream_t stream) {
+  if (mixed) return LaunchFrMixedTimeStep(q, u, geo_id, geo, n_cells, dt_min_bits, stream);
   int64_t blocks = std::min<int64_t>((n_cells + 255) / 256, 4096);
   if (blocks < 1) blocks = 1;
   switch (q) {

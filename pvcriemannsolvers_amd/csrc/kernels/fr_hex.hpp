@@ -18,14 +18,16 @@ constexpr int kMaxBatchGroups = 4;
 //   end[m]    = l_m(-1), the extrapolation to a line end from the node next to it
 //               inwards (the points are symmetric: l_{Q-1-m}(+1) = l_m(-1))
 //   gp[e][i]  = g_L'(x_i), g_R'(x_i) (Vincent correction derivatives)
-// and for the mixed form, which contracts deviations in FP32,
-//   d[i][m]   = l_m'(x_i), lend[e][m] = l_m(-1), l_m(+1).
 struct LineTables {
   double dg[kMaxQ][kMaxQ];
   double end[kMaxQ];
   double gp[2][kMaxQ];
-  float d[kMaxQ][kMaxQ];
-  float lend[2][kMaxQ];
+};
+// The mixed form's tables: d[i][m] = l_m'(x_i), lend[e][m] = l_m(-1), l_m(+1), gp as above.
+struct MixedTables {
+  double d[kMaxQ][kMaxQ];
+  double lend[2][kMaxQ];
+  double gp[2][kMaxQ];
 };
 
 // Per-cell affine geometry record (16 doubles):
@@ -90,12 +92,19 @@ struct FrHexArgs {
   int32_t stage;         // 0 residual, 1..3 SSP-RK3 stage
   int32_t xcd_remap;     // remap block ids so each XCD sweeps a contiguous range
   int32_t any_swap;      // some FrFace has its swap bit set
-  int32_t mixed;         // FP32 flux-column contractions (mixed-precision form)
+  int32_t mixed;         // FP32 flux-column contractions (mixed-precision form, fr_mixed.hip)
   int32_t curved;        // per-node metrics and per-point normals and scales
   const int32_t *tile_order;  // [tile]: tile swept by logical block b (spatial locality), or null
   // If set, the time-step reduction of LaunchFrHexTimeStep over the state this
   // pass writes is folded into *dt_min_bits (same arithmetic, no extra pass).
   unsigned long long *dt_min_bits;
+  // mixed form only, whose states are columns [cell][node][5] and whose geo has
+  // records of kMixedGeoStride:
+  const int32_t *nbr;       // [cell][6]: neighbour cell, or -(1 + boundary tag)
+  const int32_t *finfo;     // [cell][6]: frame id << 7 | holder << 6 | orient << 3 | neighbour face
+  const double *frames;     // [frame][kFrameStride]
+  const int32_t *bface_of;  // [cell][6] boundary face index, -1 elsewhere
+  int32_t diag_metric;      // every J* is diagonal (axis-aligned cells)
   // exact solver only: [cell][local face][point] sign of each flux point's
   // last star velocity (ExactFlux), zero-initialised at creation
   uint8_t *exact_star;
@@ -103,16 +112,17 @@ struct FrHexArgs {
 
 // Launches one residual / RK-stage pass for Q points per direction and the
 // given Riemann solver on `stream`.  Returns hipSuccess or the launch error.
-hipError_t LaunchFrHexStage(int q, int riemann, const FrHexArgs &args, const LineTables &lt,
+hipError_t LaunchFrHexStage(int q, int riemann, const FrHexArgs &args, const LineTables &lt, const MixedTables &mt,
                             hipStream_t stream);
 // Cells per workgroup (one tile) of LaunchFrHexStage for Q points per direction.
-int FrHexStageTileCells(int q);
+int FrHexStageTileCells(int q, bool mixed);
 
 // One degree group of a batched launch: its own arrays, line tables and tile
 // variant (cells per workgroup, see FrHexTileCells).
 struct FrHexBatchGroup {
   FrHexArgs args;
   LineTables lt;
+  MixedTables mt;
   int32_t q;
   int32_t tile;
   int64_t first_item;   // first work item of this group
@@ -126,8 +136,8 @@ struct FrHexBatchArgs {
 
 // Cells per workgroup and LDS bytes of tile variant `tile` (0..2) for q
 // points (2..4); 0 if invalid.
-int FrHexTileCells(int q, int tile);
-int FrHexTileLdsBytes(int q, int tile);
+int FrHexTileCells(int q, int tile, bool mixed);
+int FrHexTileLdsBytes(int q, int tile, bool mixed);
 
 // Persistent batched stage over all groups with n_workgroups workgroups.
 hipError_t LaunchFrHexBatch(int riemann, bool mixed, const FrHexBatchArgs &args, int n_workgroups,
@@ -142,7 +152,7 @@ hipError_t LaunchFrLayout(bool to_planes, const double *in, double *out, int np,
 // (spatial/fem.hpp:417-435), reduced to one double in *dt_min (device).
 // *bits = the ordered bits of 1e300, the start of a time-step reduction.
 hipError_t LaunchResetTimeStepBits(unsigned long long *bits, hipStream_t stream);
-hipError_t LaunchFrHexTimeStep(int q, const double *u, const int32_t *geo_id, const double *geo,
+hipError_t LaunchFrHexTimeStep(int q, bool mixed, const double *u, const int32_t *geo_id, const double *geo,
                                int64_t n_cells, unsigned long long *dt_min_bits, hipStream_t stream);
 
 }  // namespace mcfd

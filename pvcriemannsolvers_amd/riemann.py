@@ -21,8 +21,8 @@ _FORM = {"fr": C.FLUX_FORM_FR, "dg": C.FLUX_FORM_DG}
 
 
 class Rotated:
-    """``riemann``: "exact", "hllc" or "roe"; ``form``: "fr" (the FR stage
-    kernels' evaluation) or "dg" (the modal-DG face pass's)."""
+    """``riemann``: "exact", "hllc" or "roe"; ``form``: "fr" (the stage
+    kernels' evaluation, on the unit normal) or "dg" (rotated into the frame and back)."""
 
     def __init__(self, riemann: str, n_points: int, form: str = "fr"):
         self.riemann = _KIND[riemann]
