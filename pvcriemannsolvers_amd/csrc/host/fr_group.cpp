@@ -228,11 +228,8 @@ void FrHexGroup::Build(const mcfd_mesh_desc &mesh, const mcfd_scheme_desc &schem
     for (int lane = 0; lane < 64; ++lane) {
       const int h = lane >> 4, l = lane & 3;
       o.dg[lane] = lt.dg[l][h];
-      const double end = (l & 1) ? lt.end[3 - h] : lt.end[h], gp = lt.gp[h & 1][l];
-      o.end01[lane] = l < 2 ? end : 0.0;
-      o.end23[lane] = l < 2 ? 0.0 : end;
-      o.gp01[lane] = h < 2 ? gp : 0.0;
-      o.gp23[lane] = h < 2 ? 0.0 : gp;
+      o.end[lane] = (l & 1) ? lt.end[3 - h] : lt.end[h];
+      o.gp[lane] = lt.gp[h & 1][l];
     }
     h_ops.push_back(o);
   }

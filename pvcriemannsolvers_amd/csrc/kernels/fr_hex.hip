@@ -547,16 +547,24 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
 #pragma unroll
     for (int k = 0; k < 5; ++k) lds[g * S::kState + k * 79 + at_x] = u[g][k];
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  double end01 = ops->end01[lane], end23 = ops->end23[lane];
+  const double end = ops->end[lane];
   // the cell's own traces at its ends
   auto own_trace = [&](int s) {
     State own;
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       const double *const su = lds + (s == Z ? 0 : s) * S::kState + k * 79;
-      if (s < Z) own.v[k] = Mfma(end23, su[at_y], Mfma(end01, su[at_x], 0.0));
-      else if (kCells == 1) own.v[k] = Mfma(end01 + end23, su[at_z], 0.0);
-      else own.v[k] = Mfma(end23, su[S::kState + at_z], Mfma(end01, su[at_z], 0.0));
+      // selected, not added to the other half's zeros: 0 times a NaN or an infinity
+      // there, of another line or even of the other cell, is a NaN
+      if (s < Z) {
+        const double x = Mfma(end, su[at_x], 0.0), y = Mfma(end, su[at_y], 0.0);
+        own.v[k] = h < 2 ? x : y;
+      } else if (kCells == 1) {
+        own.v[k] = Mfma(end, su[at_z], 0.0);
+      } else {
+        const double first = Mfma(end, su[at_z], 0.0), second = Mfma(end, su[S::kState + at_z], 0.0);
+        own.v[k] = h < 2 ? first : second;
+      }
     }
     return own;
   };
@@ -633,7 +641,7 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
 
   // ---- F~_r = F J*.col(r) at the nodes, contracted: x and z into div in the
   // node order, y into divy with j in h; and the fluxes lifted
-    const double dg = ops->dg[lane], gp01 = ops->gp01[lane], gp23 = ops->gp23[lane];
+    const double dg = ops->dg[lane], gp = ops->gp[lane];
     const int g = s;
     const int64_t c = g ? c1 : c0;
     double *const su = lds + g * S::kState;
@@ -677,9 +685,10 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
 #pragma unroll
       for (int k = 0; k < 5; ++k) {
         const double fk = k == 0 ? mom : (k == 4 ? (v[4] + p) * vel : v[k] * vel + p * col[r][k == 0 ? 0 : k - 1]);
-        if (r == 0) div[k] = Mfma(gp01, flux[k], Mfma(dg, fk, 0.0));
-        else if (r == 1) divy[k] = Mfma(gp23, flux[k], Mfma(dg, fk, 0.0));
-        else div[k] = Mfma(flux_z[k], g ? gp23 : gp01, Mfma(fk, dg, div[k]));
+        // the fluxes of this direction, or in z of this cell: see own_trace
+        if (r == 0) div[k] = Mfma(gp, h < 2 ? flux[k] : 0.0, Mfma(dg, fk, 0.0));
+        else if (r == 1) divy[k] = Mfma(gp, h < 2 ? 0.0 : flux[k], Mfma(dg, fk, 0.0));
+        else div[k] = Mfma((h < 2) == (g == 0) ? flux_z[k] : 0.0, gp, Mfma(fk, dg, div[k]));
       }
     }
 

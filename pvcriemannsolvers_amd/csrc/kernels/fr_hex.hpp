@@ -54,11 +54,9 @@ struct alignas(16) FrFace {
 
 // Lane operators of the one-wavefront-per-cell kernel (Q = 4), lane = 16 h + 4 m + l:
 struct CellOps {
-  double dg[64];     // dg[l][h]
-  double end01[64];  // extrapolation to the lower (l = 0) and upper (l = 1) line end from node h, 0 for l = 2, 3
-  double end23[64];  // the same for l = 2, 3
-  double gp01[64];   // g_L'(x_l) (h = 0) and g_R'(x_l) (h = 1), 0 for h = 2, 3
-  double gp23[64];   // the same for h = 2, 3
+  double dg[64];   // dg[l][h]
+  double end[64];  // extrapolation to the lower (l even) and upper (l odd) line end from node h
+  double gp[64];   // g_L'(x_l) (h even) and g_R'(x_l) (h odd)
 };
 
 // States live in planes, [cell][5][node]: a wavefront's lines are then read

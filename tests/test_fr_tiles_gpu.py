@@ -63,3 +63,30 @@ def test_two_cells_per_wavefront(riemann, jitter):
     expect = o.time_step(ref, 0.1)
     assert abs(g.get_time_step(0.1) - expect) <= (1e-12 if riemann != "exact" else 1e-7) * expect
     g.close()
+
+
+@pytest.mark.parametrize("degree,size", [(3, (17, 17, 15)), (3, (6, 5, 4)), (1, (6, 5, 4)), (2, (6, 5, 4)),
+                                         (4, (6, 5, 4)), (5, (6, 5, 4))])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_bad_values_reach_face_neighbours_only(degree, size, value):
+    """A NaN or an infinity in one cell leaves the cells that share its wavefront
+    or workgroup, but no face, as they are."""
+    mesh = meshgen.box_hex(*size, periodic=(True,) * 3, shuffle_seed=3)
+    g = spatial.FiniteElement(mesh, degree=degree, riemann="roe")
+    n = len(mesh["cells"])
+    u = density_wave(g.sample_points(), seed=2).reshape(n, -1)
+    g.set_solution_column(u.reshape(-1))
+    want = g.get_residual_column().reshape(n, -1)
+    faces = g.faces()
+    for cell in (0, n // 2, n // 2 + 1, n - 1):
+        bad = u.copy()
+        bad[cell, 0] = value
+        g.set_solution_column(bad.reshape(-1))
+        got = g.get_residual_column().reshape(n, -1)
+        near = {cell}
+        for a, b in zip(faces["holder"], faces["sharer"]):
+            if a == cell or b == cell:
+                near |= {int(a), int(b)}
+        far = np.setdiff1d(np.arange(n), sorted(near))
+        np.testing.assert_array_equal(got[far], want[far])
+    g.close()
