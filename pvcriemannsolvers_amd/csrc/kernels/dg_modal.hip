@@ -453,7 +453,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void D
   }
 #pragma unroll
   for (int o = 32; o >= 1; o /= 2) local = fmin(local, __shfl_xor(local, o));
-  if (tid == 0) atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(local));
+  if (tid == 0) FoldMin(a.dt_min_bits, local);
 }
 
 // The exact solver's w Fhat at every face quadrature point, once per face

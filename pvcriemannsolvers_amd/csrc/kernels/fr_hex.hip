@@ -415,7 +415,7 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
     }
 #pragma unroll
     for (int o = 32; o >= 1; o /= 2) local = fmin(local, __shfl_xor(local, o));
-    if ((tid & 63) == 0) atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(local));
+    if ((tid & 63) == 0) FoldMin(a.dt_min_bits, local);
   }
 }
 
@@ -721,8 +721,7 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
       double v = fmax(1e-5, MaxSpeed(out));
 #pragma unroll
       for (int o = 32; o >= 1; o /= 2) v = fmax(v, __shfl_xor(v, o));
-      if (lane == 0)
-        atomicMin(a.dt_min_bits, (unsigned long long)__double_as_longlong(geo[g][kGeoLength] / v));
+      if (lane == 0) FoldMin(a.dt_min_bits, geo[g][kGeoLength] / v);
     }
     if (turn < Z) {
       asm volatile("" ::: "memory");
@@ -803,30 +802,27 @@ __global__ void ResetTimeStepBitsKernel(unsigned long long *bits) {
   *bits = (unsigned long long)__double_as_longlong(1e300);
 }
 
+// fem.hpp:412-435: min over cells of length / max(1e-5, max over nodes of |u| + c),
+// which is the min over nodes of length / max(1e-5, |u| + c).  Bound by the read of
+// the states: consecutive lanes take consecutive nodes of the planes (a cell per
+// lane, as for columns, reads lines 5 Q^3 doubles apart: 64^3 p3 1480 us, traced).  The
+// call, us: 64^3 p3 180, 32^3 p4 100, 8^3 p3 27.
 template <int Q>
 __global__ __launch_bounds__(256) void FrHexTimeStepKernel(const double *u, const int32_t *geo_id,
     const double *geo, int64_t n_cells, unsigned long long *dt_min_bits) {
   constexpr int NP = Q * Q * Q;
-  __shared__ double s_min[256];
   double local = 1e300;
-  for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < n_cells; c += (int64_t)gridDim.x * 256) {
-    double vmax = 1e-5;  // fem.hpp:419, avoids 0 in the divisor
-    const double *uc = u + c * NP * 5;
-    for (int p = 0; p < NP; ++p) {
-      State s;
+  for (int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x; w < n_cells * NP; w += (int64_t)gridDim.x * 256) {
+    const int64_t c = w / NP;
+    const double *uc = u + c * (4 * NP) + w;
+    State s;
 #pragma unroll
-      for (int k = 0; k < 5; ++k) s.v[k] = uc[k * NP + p];
-      vmax = fmax(vmax, MaxSpeed(s));
-    }
-    local = fmin(local, geo[(int64_t)geo_id[c] * kGeoStride + kGeoLength] / vmax);
+    for (int k = 0; k < 5; ++k) s.v[k] = uc[k * NP];
+    local = fmin(local, geo[(int64_t)geo_id[c] * kGeoStride + kGeoLength] / fmax(1e-5, MaxSpeed(s)));
   }
-  s_min[threadIdx.x] = local;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) s_min[threadIdx.x] = fmin(s_min[threadIdx.x], s_min[threadIdx.x + s]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) atomicMin(dt_min_bits, (unsigned long long)__double_as_longlong(s_min[0]));
+#pragma unroll
+  for (int o = 32; o >= 1; o /= 2) local = fmin(local, __shfl_xor(local, o));
+  if ((threadIdx.x & 63) == 0) FoldMin(dt_min_bits, local);
 }
 
 // Q = 4: two cells per wavefront save a quarter of the flux points' lanes but
@@ -963,7 +959,8 @@ hipError_t LaunchResetTimeStepBits(unsigned long long *bits, hipStream_t stream)
 hipError_t LaunchFrHexTimeStep(int q, bool mixed, const double *u, const int32_t *geo_id, const double *geo,
                                int64_t n_cells, unsigned long long *dt_min_bits, hipStream_t stream) {
   if (mixed) return LaunchFrMixedTimeStep(q, u, geo_id, geo, n_cells, dt_min_bits, stream);
-  int64_t blocks = std::min<int64_t>((n_cells + 255) / 256, 4096);
+  // four nodes per thread, up to two rounds of wavefronts
+  int64_t blocks = std::min<int64_t>((n_cells * q * q * q + 1023) / 1024, 4096);
   if (blocks < 1) blocks = 1;
   switch (q) {
 #define MCFD_TS_CASE(QQ) \

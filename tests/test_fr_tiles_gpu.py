@@ -65,6 +65,32 @@ def test_two_cells_per_wavefront(riemann, jitter):
     g.close()
 
 
+@pytest.mark.parametrize("degree", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("size", [(1, 1, 1), (7, 5, 3), (17, 16, 16)])
+@pytest.mark.parametrize("jitter", [0.0, 0.2])
+def test_time_step_of_any_node(degree, size, jitter):
+    """The smallest length / (|u| + c), wherever the fastest node lies: read of a
+    state and folded into a step's last stage."""
+    mesh = meshgen.box_hex(*size, jitter=jitter, seed=9, shuffle_seed=2)
+    o, g = make_pair(mesh, degree, "roe", [("smart", LEFT)] * 6)
+    u = density_wave(o.node_coords(), seed=3).reshape(len(mesh["cells"]), -1, 5)
+    rng = np.random.default_rng(degree)
+    places = [(0, 0), (-1, -1)] + [(rng.integers(u.shape[0]), rng.integers(u.shape[1])) for _ in range(4)]
+    for cell, node in places:
+        v = u.copy()
+        v[cell, node, 4] *= 9
+        g.set_solution_column(v.reshape(-1))
+        expect = o.time_step(v.reshape(-1), 0.1)
+        assert abs(g.get_time_step(0.1) - expect) <= 1e-12 * expect
+        g.rk3_update(0.0, 0.01 * expect)
+        state = g.get_solution_column()
+        fused, expect = g.get_time_step(0.1), o.time_step(state, 0.1)
+        assert abs(fused - expect) <= 1e-12 * expect
+        g.set_solution_column(state)
+        assert g.get_time_step(0.1) == fused
+    g.close()
+
+
 @pytest.mark.parametrize("degree,size", [(3, (17, 17, 15)), (3, (6, 5, 4)), (1, (6, 5, 4)), (2, (6, 5, 4)),
                                          (4, (6, 5, 4)), (5, (6, 5, 4))])
 @pytest.mark.parametrize("value", [np.nan, np.inf])
