@@ -786,16 +786,17 @@ __global__ __launch_bounds__(Shape<4>::kThreads) __attribute__((amdgpu_waves_per
 }
 
 // Column layout [cell][node][5] <-> the kernels' planes [cell][5][node], one
-// thread per value of the planes.
+// thread per value of the planes (several above 2^30 values: a launch holds 2^32
+// threads at most).
 template <bool kToPlanes>
 __global__ __launch_bounds__(256) void FrLayoutKernel(const double *in, double *out, int np, int64_t n) {
-  const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (w >= n) return;
-  const int64_t c = w / (5 * np);
-  const int r = (int)(w - c * (5 * np)), k = r / np, node = r - k * np;
-  const int64_t col = (c * np + node) * 5 + k;
-  if constexpr (kToPlanes) out[w] = in[col];
-  else out[col] = in[w];
+  for (int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x; w < n; w += (int64_t)gridDim.x * 256) {
+    const int64_t c = w / (5 * np);
+    const int r = (int)(w - c * (5 * np)), k = r / np, node = r - k * np;
+    const int64_t col = (c * np + node) * 5 + k;
+    if constexpr (kToPlanes) out[w] = in[col];
+    else out[col] = in[w];
+  }
 }
 
 __global__ void ResetTimeStepBitsKernel(unsigned long long *bits) {
@@ -940,9 +941,8 @@ int FrHexBatchResidentWorkgroups(int riemann, bool mixed, int lds_bytes) {
 }
 
 hipError_t LaunchFrLayout(bool to_planes, const double *in, double *out, int np, int64_t n_cells, hipStream_t stream) {
-  const int64_t n = n_cells * np * 5, blocks = (n + 255) / 256;
+  const int64_t n = n_cells * np * 5, blocks = std::min<int64_t>((n + 255) / 256, int64_t(1) << 22);
   if (blocks < 1) return hipSuccess;
-  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
   if (to_planes) {
     hipLaunchKernelGGL(FrLayoutKernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream, in, out, np, n);
   } else {
