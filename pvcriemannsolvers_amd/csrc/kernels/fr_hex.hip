@@ -706,7 +706,10 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
       const double sum = div[k] + su[k * 79 + at_x];
       out.v[k] = fr::RkOutput(a.stage, -sum * inv_det, uc[k], u0[k], dt[g]);
     }
-    if (g == 0 || c1 != c0) {
+    // An odd last cell's second turn is worth nothing: stage 3 has written over its
+    // U0.  (Left out by a branch ahead of it, the solvers' other kernels spill.)
+    const bool real = g == 0 || c1 != c0;
+    if (real) {
       // the residual is handed out as a column, states stay in planes; streamed,
       // so that the states which neighbours still gather keep the L2
       const int64_t to = a.stage == 0 ? (c * NP + lane) * 5 : c * (5 * NP) + lane;
@@ -714,7 +717,7 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
 #pragma unroll
       for (int k = 0; k < 5; ++k) __builtin_nontemporal_store(out.v[k], a.out + to + k * step);
     }
-    if (a.dt_min_bits) {
+    if (a.dt_min_bits && real) {
       // fem.hpp:412-435 on the state just written, as FrHexTimeStepKernel: min
       // over cells of length / max(1e-5, max over nodes of |u| + c); the bits of
       // positive doubles order as the doubles do

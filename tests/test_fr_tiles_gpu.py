@@ -116,3 +116,26 @@ def test_bad_values_reach_face_neighbours_only(degree, size, value):
         far = np.setdiff1d(np.arange(n), sorted(near))
         np.testing.assert_array_equal(got[far], want[far])
     g.close()
+
+
+@pytest.mark.parametrize("cell", [0, 2166, 4333, 4334])
+def test_folded_time_step_of_an_odd_last_cell(cell):
+    """4335 cells of degree 3, two to a wavefront, the last one with its
+    wavefront to itself: with a cell whose fastest node gains speed in the step, the
+    minimum folded into stage 3, which writes over the state it reads, is that of the
+    state it wrote."""
+    mesh = meshgen.box_hex(17, 17, 15, shuffle_seed=2)
+    o, g = make_pair(mesh, 3, "roe", [("smart", LEFT)] * 6)
+    u = density_wave(o.node_coords(), seed=3).reshape(len(mesh["cells"]), -1, 5)
+    u[cell, :, 4] *= np.random.default_rng(0).uniform(5, 9, 64)
+    g.set_solution_column(u.reshape(-1))
+    dt = g.get_time_step(0.1)
+    g.rk3_update(0.0, dt)
+    fused = g.get_time_step(0.1)
+    assert fused < 0.99 * dt
+    state = g.get_solution_column()
+    g.set_solution_column(state)
+    assert fused == g.get_time_step(0.1)
+    expect = o.time_step(state, 0.1)
+    assert abs(fused - expect) <= 1e-12 * expect
+    g.close()
