@@ -47,11 +47,12 @@ __device__ __forceinline__ double FastSqrt(double x) {
 }
 
 // x / 3, correctly rounded: the quotient by the rounded reciprocal is at most
-// one unit off, and the fused remainder puts it right (Markstein's division
-// for a constant divisor), in 3 instructions instead of the divide's 10.
+// one unit off, and the fused remainder, exact also below the normal range, puts
+// it right (Markstein's division for a constant divisor); the fixup returns
+// infinities and signed zeros as the divide does.  4 instructions instead of 10.
 __device__ __forceinline__ double ThirdOf(double x) {
   const double q = x * (1.0 / 3.0);
-  return __fma_rn(__fma_rn(-3.0, q, x), 1.0 / 3.0, q);
+  return __builtin_amdgcn_div_fixup(__fma_rn(__fma_rn(-3.0, q, x), 1.0 / 3.0, q), 3.0, x);
 }
 
 // One trace of a face with what the fluxes need of it: density and its
