@@ -15,14 +15,19 @@ namespace mcfd {
 // v_rcp_f64 refined by two Newton steps: within 1 ulp of 1/x for normal x.
 // Used by the throughput kernels in place of IEEE division (a ~10
 // instruction sequence on CDNA); both cells of a face run the same code, so
-// the face flux stays bit-identical on the two sides.
-__device__ __forceinline__ double FastRcp(double x) {
+// the face flux stays bit-identical on the two sides.  NaN for zeros and
+// infinities, of which the steps know nothing.
+__device__ __forceinline__ double FiniteRcp(double x) {
   double r = __builtin_amdgcn_rcp(x);
   double e = __fma_rn(-x, r, 1.0);
   r = __fma_rn(r, e, r);
   e = __fma_rn(-x, r, 1.0);
   return __fma_rn(r, e, r);
 }
+// The same with zeros and infinities as the divide has them, one instruction more
+// (in the nodes' fluxes too it would cost 0.3 % of a pass, and change nothing: they
+// replace what a zero density gives).
+__device__ __forceinline__ double FastRcp(double x) { return __builtin_amdgcn_div_fixup(FiniteRcp(x), x, 1.0); }
 
 // The smallest of the positive `value`s in *bits (the bits of positive doubles
 // order as the doubles do).  Atomics on one address pass at about 11 ns each, 3 ms
@@ -33,9 +38,10 @@ __device__ __forceinline__ void FoldMin(unsigned long long *bits, double value) 
   if (own < __hip_atomic_load(bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(bits, own);
 }
 
-// sqrt by v_rsq_f64 and two fused corrections: within 1 ulp for normal x,
-// 0 for 0, NaN for x < 0.  The compiler's correctly rounded sqrt adds range
+// sqrt by v_rsq_f64 and two fused corrections: within 1 ulp for normal x, x for
+// zeros and infinity, NaN for x < 0.  The compiler's correctly rounded sqrt adds range
 // scaling and class checks, about twice the instructions.
+constexpr int kZerosAndInfinity = 0x20 | 0x40 | 0x200;  // v_cmp_class: -0, +0, +inf
 __device__ __forceinline__ double FastSqrt(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
@@ -43,7 +49,7 @@ __device__ __forceinline__ double FastSqrt(double x) {
   g = __fma_rn(g, r, g);
   h = __fma_rn(h, r, h);
   g = __fma_rn(__fma_rn(-g, g, x), h, g);
-  return x == 0 ? 0.0 : g;
+  return __builtin_amdgcn_class(x, kZerosAndInfinity) ? x : g;
 }
 
 // x / 3, correctly rounded: the quotient by the rounded reciprocal is at most

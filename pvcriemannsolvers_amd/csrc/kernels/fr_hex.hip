@@ -334,7 +334,7 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
       }
       // contravariant momentum and velocity, and pressure; the zeroing rule of
       // types.hpp:195-202,289-301 only where some lane of the wavefront needs it
-      const double inv = FastRcp(w[0]);
+      const double inv = FiniteRcp(w[0]);
       const double mom = w[1] * col[0] + w[2] * col[1] + w[3] * col[2];
       double vel = mom * inv;
       double p = (w[4] - 0.5 * (w[1] * w[1] + w[2] * w[2] + w[3] * w[3]) * inv) * kGm1;
@@ -671,7 +671,7 @@ __device__ __forceinline__ void FrCellBody(const FrHexArgs &a, const LineTables 
 #pragma unroll
       for (int k = 0; k < 5; ++k) v[k] = su[k * 79 + (r == 0 ? at_x : (r == 1 ? at_y : at_z))];
       // contravariant momentum and velocity, and pressure
-      const double inv = FastRcp(v[0]);
+      const double inv = FiniteRcp(v[0]);
       const double mom = v[1] * col[r][0] + v[2] * col[r][1] + v[3] * col[r][2];
       double vel = mom * inv;
       double p = (v[4] - 0.5 * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]) * inv) * kGm1;

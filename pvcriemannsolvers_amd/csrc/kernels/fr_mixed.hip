@@ -130,10 +130,10 @@ __device__ __forceinline__ double LiftedGaps(const double *g, const MixedTables 
 // arithmetic is done first; the rule only selects among its results, so
 // a wavefront where no lane needs the rule (rho > 0, E >= 0, p >= 0 on every
 // lane) skips the selects and gets bitwise the same values as one that
-// applies them.  *inv_rho receives FastRcp of the returned density.
+// applies them.  *inv_rho receives FiniteRcp of the returned density.
 __device__ __forceinline__ State FastPrimitive(State const &c, double *inv_rho) {
   const double rho = c.v[0];
-  const double inv = FastRcp(rho);
+  const double inv = FiniteRcp(rho);
   State p;
   p.v[0] = rho;
   p.v[1] = c.v[1] * inv;
@@ -151,7 +151,7 @@ __device__ __forceinline__ State FastPrimitive(State const &c, double *inv_rho) 
 #pragma unroll
   for (int k = 1; k < 5; ++k) p.v[k] = zero ? 0.0 : (vacuum ? c.v[k] : p.v[k]);
   p.v[0] = zero ? 0.0 : rho;  // a vacuum keeps its signed zero
-  if (zero || vacuum) *inv_rho = FastRcp(p.v[0]);
+  if (zero || vacuum) *inv_rho = FiniteRcp(p.v[0]);
   return p;
 }
 __device__ __forceinline__ State FastPrimitive(State const &c) {
@@ -160,7 +160,7 @@ __device__ __forceinline__ State FastPrimitive(State const &c) {
 }
 
 // Roe flux of normal-frame primitives (same waves as RoeFlux) with
-// reciprocals instead of divisions; inv_l, inv_r = FastRcp of the densities.
+// reciprocals instead of divisions; inv_l, inv_r = FiniteRcp of the densities.
 __device__ __forceinline__ State FastRoeFlux(State const &l, State const &r, double inv_l, double inv_r) {
   constexpr double kGoGm1 = kGamma / kGm1;
   double kel = 0.5 * (l.v[1] * l.v[1] + l.v[2] * l.v[2] + l.v[3] * l.v[3]);
@@ -174,7 +174,7 @@ __device__ __forceinline__ State FastRoeFlux(State const &l, State const &r, dou
   flux.v[3] = 0.5 * ((l.v[0] * l.v[3]) * l.v[1] + (r.v[0] * r.v[3]) * r.v[1]);
   flux.v[4] = 0.5 * ((el + l.v[4]) * l.v[1] + (er + r.v[4]) * r.v[1]);
   double sl = sqrt(l.v[0]), sr = sqrt(r.v[0]);
-  double inv = FastRcp(sl + sr);
+  double inv = FiniteRcp(sl + sr);
   double h0l = l.v[4] * inv_l * kGoGm1 + kel;
   double h0r = r.v[4] * inv_r * kGoGm1 + ker;
   double rho = sl * sr;
@@ -184,7 +184,7 @@ __device__ __forceinline__ State FastRoeFlux(State const &l, State const &r, dou
   double h = (sl * h0l + sr * h0r) * inv;
   double ke = (u * u + v * v + w * w) * 0.5;
   double aa = kGm1 * (h - ke);
-  double a = sqrt(aa), ua = u * a, inv_aa = FastRcp(aa);
+  double a = sqrt(aa), ua = u * a, inv_aa = FiniteRcp(aa);
   double dp = r.v[4] - l.v[4], du = r.v[1] - l.v[1];
   double s1 = 0.25 * (dp - rho * a * du) * inv_aa * fabs(u - a);
   double s2 = 0.5 * ((r.v[0] - l.v[0]) - dp * inv_aa) * fabs(u);

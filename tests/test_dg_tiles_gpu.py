@@ -58,3 +58,32 @@ def test_exact_solver_on_both_sides_of_the_face_pass(mesh, degree):
     g.rk3_update(0.0, dt)
     assert rel(g.get_solution_column(), o.rk3(u, dt, 1)) <= TOL["exact"]
     g.close()
+
+
+@pytest.mark.parametrize("kind", ["tet", "hex"])
+@pytest.mark.parametrize("degree", [1, 2])
+@pytest.mark.parametrize("riemann", ["roe", "hllc", "exact"])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_bad_values_reach_face_neighbours_only(kind, degree, riemann, value):
+    """A NaN or an infinity in one cell leaves the cells that share its workgroup,
+    but no face, as they are."""
+    mesh = meshgen.box_tet(3, 3, 3, jitter=0.1, seed=3) if kind == "tet" else meshgen.box_hex(6, 4, 4, shuffle_seed=3)
+    o, g = make_pair(mesh, degree, riemann, MIXED_BCS)
+    n = len(mesh["cells"])
+    u = o.approximate(smooth_state(o.cells()["xyz"])).reshape(n, -1)
+    g.set_solution_column(u.reshape(-1))
+    want = g.get_residual_column().reshape(n, -1)
+    faces = g.faces()
+    for cell in (0, n // 2, n // 2 + 1, n - 1):
+        bad = u.copy()
+        bad[cell, 0] = value
+        g.set_solution_column(bad.reshape(-1))
+        got = g.get_residual_column().reshape(n, -1)
+        near = {cell}
+        for a, b in zip(faces["holder"], faces["sharer"]):
+            if a == cell or b == cell:
+                near |= {int(a), int(b)}
+        far = np.setdiff1d(np.arange(n), sorted(near))
+        np.testing.assert_array_equal(got[far], want[far])
+        assert not np.isfinite(got[cell]).all()
+    g.close()
