@@ -153,14 +153,16 @@ __device__ __forceinline__ State FastRoe(FaceTrace const &l, FaceTrace const &r,
 }
 
 // HLLC flux (hllc.hpp:30-109): wave speeds u -+ a q from one square root each
-// (a q = sqrt(a^2 + c (p* - p) / rho) needs no division by p), the star state
-// formed once, for the side the contact selects.
+// (a q = sqrt(a^2 + c (p* - p) / rho) needs no division by p; a side without
+// density but with pressure has a = 0 and a finite q, so a q is 0 there, not the
+// formula's infinity), the star state formed once, for the side the contact selects.
 __device__ __forceinline__ State FastHllc(FaceTrace const &l, FaceTrace const &r, const double *n) {
   const double al = l.rho > 0 && l.p > 0 ? FastSqrt(kGamma * l.p * l.inv) : 0.0;
   const double ar = r.rho > 0 && r.p > 0 ? FastSqrt(kGamma * r.p * r.inv) : 0.0;
   const double p_est = fmax(0.0, 0.5 * (l.p + r.p - (r.un - l.un) * (0.25 * (l.rho + r.rho) * (al + ar))));
-  const double aql = p_est > l.p ? FastSqrt((kGamma * l.p + (kGp1 / 2) * (p_est - l.p)) * l.inv) : al;
-  const double aqr = p_est > r.p ? FastSqrt((kGamma * r.p + (kGp1 / 2) * (p_est - r.p)) * r.inv) : ar;
+  const bool still_l = p_est <= l.p || (l.p > 0 && !(l.rho > 0)), still_r = p_est <= r.p || (r.p > 0 && !(r.rho > 0));
+  const double aql = still_l ? al : FastSqrt((kGamma * l.p + (kGp1 / 2) * (p_est - l.p)) * l.inv);
+  const double aqr = still_r ? ar : FastSqrt((kGamma * r.p + (kGp1 / 2) * (p_est - r.p)) * r.inv);
   const double wl = l.un - aql, wr = r.un + aqr;
   const double ml = l.rho * (wl - l.un), mr = r.rho * (wr - r.un);
   const double ws = (r.p - l.p + ml * l.un - mr * r.un) * FastRcp(ml - mr);
