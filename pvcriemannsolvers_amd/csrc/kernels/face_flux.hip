@@ -1,9 +1,10 @@
-// Face fluxes at independent points, evaluated by the same device code as
-// the stage kernels: the upwind flux of rotated::Euler
+// Face fluxes at independent points: the upwind flux of rotated::Euler
 // (riemann/rotated/euler.hpp:153-159) and the boundary fluxes of an inviscid
 // wall (:160-174), a supersonic outlet (:144-151) and the subsonic inlet and
-// outlet (:181-280).  It lets the device
-// solvers be checked on the reference's known answers pair by pair.
+// outlet (:181-280).  Form FR is the stage kernels' device code, on the unit
+// normal; form DG rotates into the frame and back, as the reference and the
+// mixed form do.  It lets the device solvers be checked on the reference's known
+// answers pair by pair.
 #include "face_flux.hpp"
 
 #include <mutex>
@@ -32,7 +33,11 @@ __global__ __launch_bounds__(64) void FaceFluxPointsKernel(int kind, int64_t n, 
 #pragma unroll
   for (int k = 0; k < 5; ++k) { l.v[k] = left[i * 5 + k]; r.v[k] = right[i * 5 + k]; }
   bool star = star_state ? star_state[i] != 0 : false;
-  if (kind == kFluxInviscidWall) {
+  if constexpr (kForm == 0) {  // as the stage kernels: on the unit normal, which points out of `left`
+    constexpr int kBoundary[] = { kBcSmart, kBcInviscidWall, kBcSupersonicOutlet, kBcSubsonicInlet, kBcSubsonicOutlet };
+    if (kind == kFluxUpwind) out = FaceFlux<kRiemann>(f.n, l, r, star);
+    else out = BoundaryFlux(kBoundary[kind], true, f.n, l, r);
+  } else if (kind == kFluxInviscidWall) {
     out = WallFlux(f, l);
   } else if (kind == kFluxSupersonicOutlet) {
     out = StateFlux(f, l);
@@ -40,8 +45,6 @@ __global__ __launch_bounds__(64) void FaceFluxPointsKernel(int kind, int64_t n, 
     out = SubsonicInletFlux(f, l, r);
   } else if (kind == kFluxSubsonicOutlet) {
     out = SubsonicOutletFlux(f, l, r);
-  } else if constexpr (kForm == 0) {
-    out = FaceFlux<kRiemann>(f.n, l, r, star);
   } else {
     out = UpwindFlux<kRiemann>(f, l, r, star);
   }

@@ -17,8 +17,8 @@ constexpr int kFluxSubsonicOutlet = 4;  // right[4] = the back pressure
 
 // flux[i] of point i (device arrays): frames [n][9] rows (n, t, b), left and
 // right [n][5] conservative, star_state [n] the exact solver's per-point state
-// (in/out, or null for fresh solvers).  form 0: the FR stage kernels' code;
-// form 1: the modal-DG face pass's code.  kind: kFlux*.
+// (in/out, or null for fresh solvers).  form 0: the stage kernels' code, on the
+// unit normal alone; form 1: rotated into the frame and back.  kind: kFlux*.
 hipError_t LaunchFaceFluxPoints(int riemann, int form, int kind, int64_t n, const double *frames,
                                 const double *left, const double *right, uint8_t *star_state, double *flux,
                                 hipStream_t stream);

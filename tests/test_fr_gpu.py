@@ -248,6 +248,36 @@ def test_batched_forms_match_single_case_oracle(precision, mode, tile):
     batch.close()
 
 
+@pytest.mark.parametrize("riemann", ["exact", "hllc", "roe"])
+@pytest.mark.parametrize("lengths", [(33, 50, 18), (150, 290, 1100)])
+def test_batched_forms_give_the_same_bits(riemann, lengths):
+    """The autotuner picks a launch form by its time, so the forms agree bit for
+    bit: per degree group and persistent with every tile, on few cells and on
+    more than 4096 of degree 3, an odd number."""
+    cases, refs = [], []
+    for i, n in enumerate(lengths):
+        mesh, degree, bcs, left, right = _tube_case(n, i + 1, 1.0, 0.2, 2.0, 0.4, -0.1, 0.5)
+        if degree == 3:  # a single cell more
+            cases.append((meshgen.box_hex(1, 1, 1), degree, [("smart", left)] * 6))
+            refs.append((left, left, 1))
+        cases.append((mesh, degree, bcs))
+        refs.append((left, right, n))
+    results = []
+    for mode, tile in [(0, 0), (1, 0), (1, 1), (1, 2)]:
+        batch = spatial.Batch(cases, riemann=riemann)
+        for i, (left, right, n) in enumerate(refs):
+            w = 0.5 * (1 + np.tanh((batch.sample_points(i)[..., 0] - 0.5) * n / 2.0))
+            batch.set_solution_column(i, ((1 - w)[..., None] * left + w[..., None] * right).reshape(-1))
+        batch.set_time_steps(batch.get_time_steps(0.1))
+        batch.set_mode(mode, [tile] * 3)
+        batch.rk3_steps(3)
+        results.append([batch.get_solution_column(i) for i in range(len(cases))])
+        batch.close()
+    for got in results[1:]:
+        for a, b in zip(got, results[0]):
+            np.testing.assert_array_equal(a, b)
+
+
 def test_batched_autotune_keeps_results():
     """The autotuner's choice (whatever it is on this device) gives the same
     states as the oracle; its trial launches leave no trace in the state."""

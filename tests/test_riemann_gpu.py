@@ -251,3 +251,29 @@ def test_states_without_density_or_pressure_match_oracle(riemann, form):
     scale = np.maximum(np.abs(want[finite]).max(axis=1), 1.0)
     assert np.isfinite(got[finite]).all()
     assert (np.abs(got[finite] - want[finite]).max(axis=1) / scale).max() < 1e-12
+
+
+@pytest.mark.parametrize("kind", ["wall", "supersonic_outlet", "subsonic_inlet", "subsonic_outlet"])
+def test_boundary_fluxes_of_the_stage_kernels(kind):
+    """The "fr" form is the stage kernels' evaluation, which knows the unit normal
+    only: tangents that are not a number change nothing."""
+    rng = np.random.default_rng(31)
+    n, frames = 512, random_frames(512, 131)
+    d = -frames[:, 0] + 0.3 * frames[:, 1]  # air, flowing in subsonically
+    d /= np.linalg.norm(d, axis=1)[:, None]
+    rho, vel, p = 1.2 + 0.1 * rng.random(n), 50 * d + 5 * rng.standard_normal((n, 3)), 1e5 * (1 + 0.05 * rng.random(n))
+    left = np.column_stack([rho, rho[:, None] * vel, p / (GAMMA - 1) + 0.5 * rho * (vel ** 2).sum(axis=1)])
+    given = np.column_stack([1.03e5 * (1 + 0.01 * rng.random(n)), d, 300 + rng.random(n)])
+    if kind == "subsonic_outlet":
+        given = np.column_stack([np.zeros((n, 4)), np.full(n, 0.97e5)])
+    code = {"wall": 1, "supersonic_outlet": 2, "subsonic_inlet": 3, "subsonic_outlet": 4}[kind]
+    s, blind = rm.Rotated("hllc", 512), frames.copy()
+    blind[:, 1:] = np.nan
+    call = {"wall": s.get_flux_on_inviscid_wall, "supersonic_outlet": s.get_flux_on_supersonic_outlet,
+            "subsonic_inlet": s.get_flux_on_subsonic_inlet, "subsonic_outlet": s.get_flux_on_subsonic_outlet}[kind]
+    args = (left, given) if code > 2 else (left,)
+    got = call(blind, *args)
+    want = ol.face_fluxes(HLLC, code, frames, *args)
+    assert np.isfinite(want).all()
+    assert per_point_rel(got, want) < (1e-12 if kind == "subsonic_inlet" else 1e-13)  # the inlet takes roots of both
+    np.testing.assert_array_equal(got, call(frames, *args))
