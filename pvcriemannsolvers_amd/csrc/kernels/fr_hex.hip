@@ -6,7 +6,7 @@
 //
 // Two kernels.  FP64 at Q = 4 points: one wavefront per cell or per two cells
 // on v_mfma_f64_4x4x4 (below).  All else: lanes that own a line of solution
-// points.  A workgroup owns C cells (16, 7, 4, 3, 1 for Q = 2..6), and each lane
+// points.  A workgroup owns C cells (16, 7, 3, 1 for Q = 2, 3, 5, 6), and each lane
 //   1. gathers, for the flux points at its line's ends, the neighbours' lines
 //      behind them (through L1 and L2); the cells' own states go to LDS once;
 //   2. extrapolates both traces of each end and solves the upwind flux there;
@@ -17,9 +17,9 @@
 // Then the threads, one per value, sum the three directions' parts and do the
 // RK stage in the reference's operation order.  Each interior face is solved by
 // both of its cells with bit-identical inputs, so the scheme stays conservative
-// without atomics or a separate face pass.  The line body serves the
-// single-mesh launch and the persistent batched launch that walks a work list
-// spanning several polynomial degrees.
+// without atomics or a separate face pass.  The bodies serve the single-mesh
+// launch and the persistent batched launch that walks a work list spanning several
+// polynomial degrees.
 //
 // What bounds both: a pass must move U, U0 and the new U, 120 B per node (HBM at
 // about half its copy rate), and issues its FP64 instructions in about half the
@@ -70,11 +70,9 @@ struct Shape {
   static constexpr int kSI = Q * kSJ;
   static constexpr int kPad = kSkew ? ((Q - 1) * (kSI + kSJ + 1) + 1) | 1 : Q * Q * Q;  // of a component
   // the cells' states, later the z direction's part of the divergence; the x
-  // direction's; and the y direction's, or (kAddY) no third share, which would
-  // cost resident workgroups: there y adds to x's part, behind one more barrier
+  // direction's; and the y direction's
   static constexpr int kShare = kCells * 5 * kPad;
-  static constexpr bool kAddY = Q == 4;
-  static constexpr int kCellData = (kAddY ? 2 : 3) * kShare;  // per cell: 1 / det(J), time step
+  static constexpr int kCellData = 3 * kShare;  // per cell: 1 / det(J), time step
   static constexpr int kFlux = kCellData + 2 * kCells;  // kSplit: the fluxes, for the line's other lane
   static constexpr int kLdsDoubles = kFlux + (kSplit ? 3 * kDirLanes * 5 : 0);
   static constexpr int kValues = kCells * 5 * kPoints, kLoads = (kValues + kThreads - 1) / kThreads;
@@ -358,8 +356,8 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
     }
   }
   __syncthreads();  // from here on the z lines' parts replace the states
-  double *const part = lds + (dir == 2 ? 0 : (dir == 1 && !S::kAddY ? 2 : 1) * S::kShare) + pos0;
-  auto lift = [&](bool add) {
+  double *const part = lds + (dir == 2 ? 0 : (dir == 1 ? 2 : 1) * S::kShare) + pos0;
+  if (active) {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       // the lower and the upper end's gap; of a split line the near and the far end's
@@ -370,17 +368,11 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
         sum = __fma_rn(-lt.gp[0][Q - 1 - i], gap[1], sum);
         if (mirror) sum = -sum;
         const int at = k * PAD + (mirror ? Q - 1 - i : i) * pos_step;
-        if (add) sum = part[at] + sum;
         part[at] = sum;
       }
     }
-  };
-  if (active && !(S::kAddY && dir == 1)) lift(false);
-  __syncthreads();
-  if constexpr (S::kAddY) {
-    if (active && dir == 1) lift(true);
-    __syncthreads();
   }
+  __syncthreads();
 
   // ---- per value: the three directions' sum, 1/det(J), RK stage, store
 #pragma unroll
@@ -389,9 +381,7 @@ __device__ __forceinline__ void FrLineBody(const FrHexArgs &a, const LineTables 
     if (e >= values) continue;
     const int at = S::At(e), cl = C == 1 ? 0 : e / (5 * NP), k = (e - cl * (5 * NP)) / NP, node = e - (cl * 5 + k) * NP;
     const double inv_det = kCurved ? a.inv_det_node[(c0 + cl) * NP + node] : lds[S::kCellData + cl];
-    double sum = lds[S::kShare + at];
-    if constexpr (!S::kAddY) sum += lds[2 * S::kShare + at];
-    sum += lds[at];
+    const double sum = lds[S::kShare + at] + lds[2 * S::kShare + at] + lds[at];
     const double out = fr::RkOutput(a.stage, -sum * inv_det, v[it], u0[it], lds[S::kCellData + C + cl]);
     // the residual is handed out as a column, states stay in planes; streamed,
     // so that the states which neighbours still gather keep the L2
@@ -447,7 +437,8 @@ __device__ __forceinline__ double Mfma(double a, double b, double c) {
   return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
 }
 
-// LDS of the kernel below, in doubles: the cells' states (skewed as Shape<4>)
+constexpr int kCellTile = 4;  // cells of one tile of tile_order
+// LDS of the kernel below, in doubles: the cells' states (skewed as Shape<Q>'s)
 // and the records of the flux points to come.
 template <int kCells>
 struct CellShape {
@@ -740,23 +731,36 @@ template <int kCells, int kRiemann, bool kCurved>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 void FrHexCellKernel(FrHexArgs a, LineTables lt) {
   __shared__ __attribute__((aligned(16))) double lds[CellShape<kCells>::kLdsDoubles];
-  constexpr int kPerTile = Shape<4>::kCells / kCells;
+  constexpr int kPerTile = kCellTile / kCells;
   const int64_t block = LogicalBlock(a.xcd_remap);
   const int64_t tile = a.tile_order ? a.tile_order[block / kPerTile] : block / kPerTile;
-  const int64_t c = tile * Shape<4>::kCells + block % kPerTile * kCells;
+  const int64_t c = tile * kCellTile + block % kPerTile * kCells;
   if (c >= a.n_cells) return;
   FrCellBody<kCells, kRiemann, kCurved>(a, lt, c, lds);
 }
 
 // Tile variants of the persistent batched launch: a work item is 1, 2 or 4
-// consecutive blocks of Shape<Q>::kCells cells.
+// consecutive blocks of BatchCells(q) cells.
 constexpr int TileBlocks(int tile) { return 1 << tile; }
+constexpr int kBatchThreads = Shape<3>::kThreads, kBatchWaves = kBatchThreads / 64;
+static_assert(Shape<2>::kThreads == kBatchThreads, "one workgroup size for all degrees");
+constexpr int BatchCells(int q) { return q == 2 ? Shape<2>::kCells : (q == 3 ? Shape<3>::kCells : kBatchWaves); }
 
 // One out-of-line body per Q: each is register-allocated on its own within the
-// kernel's budget, where the inlined bodies would share one allocation.
+// kernel's budget, where the inlined bodies would share one allocation.  The same
+// bodies as in the launches per degree group, so that both forms give the same
+// bits: at Q = 4 a cell to each wavefront.  256 tubes, ms per step: 11.2 (11.5 with
+// lines at Q = 4 too), 3.9 per degree group, as calls spill their callee's registers.
 template <int Q, int kRiemann>
 __device__ __noinline__ void BatchBody(const FrHexBatchGroup *g, int64_t block, double *lds) {
-  FrLineBody<Q, kRiemann, false>(g->args, g->lt, block, lds);
+  if constexpr (Q == 4) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t c = block * kBatchWaves + wave;
+    if (c < g->args.n_cells)
+      FrCellBody<1, kRiemann, false>(g->args, g->lt, c, lds + wave * CellShape<1>::kLdsDoubles);
+  } else {
+    FrLineBody<Q, kRiemann, false>(g->args, g->lt, block, lds);
+  }
 }
 
 // Persistent batched pass: workgroup w processes the contiguous item range
@@ -765,8 +769,8 @@ __device__ __noinline__ void BatchBody(const FrHexBatchGroup *g, int64_t block, 
 // cells -- stay in one XCD's L2.  LDS is sized at launch for the largest block
 // in use.
 template <int kRiemann>
-__global__ __launch_bounds__(Shape<4>::kThreads) __attribute__((amdgpu_waves_per_eu(3))) void FrHexBatchKernel(FrHexBatchArgs b) {
-  extern __shared__ double lds[];
+__global__ __launch_bounds__(kBatchThreads) __attribute__((amdgpu_waves_per_eu(3))) void FrHexBatchKernel(FrHexBatchArgs b) {
+  extern __shared__ __attribute__((aligned(16))) double lds[];
   const int64_t w = blockIdx.x, nw = gridDim.x;
   const int64_t begin = w * b.n_items / nw, end = (w + 1) * b.n_items / nw;
   int gi = 0;
@@ -838,10 +842,9 @@ constexpr int64_t kPairCells = 4096;
 
 template <int Q, int R>
 hipError_t Launch(const FrHexArgs &args, const LineTables &lt, hipStream_t stream) {
-  constexpr int C = Shape<Q>::kCells;
+  constexpr int C = Q == 4 ? kCellTile : Shape<Q>::kCells;
   const int64_t blocks = (args.n_cells + C - 1) / C;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)blocks), block(Shape<Q>::kThreads);
   if constexpr (Q == 4) {
     if (blocks * C > 0x7fffffff || !args.cell_ops) return hipErrorInvalidValue;
     const bool pair = args.n_cells > kPairCells;
@@ -853,12 +856,10 @@ hipError_t Launch(const FrHexArgs &args, const LineTables &lt, hipStream_t strea
       if (args.curved) hipLaunchKernelGGL((FrHexCellKernel<1, R, true>), cells, wave, 0, stream, args, lt);
       else hipLaunchKernelGGL((FrHexCellKernel<1, R, false>), cells, wave, 0, stream, args, lt);
     }
-    return hipGetLastError();
-  }
-  if (args.curved) {
-    hipLaunchKernelGGL((FrHexStageKernel<Q, R, true>), grid, block, 0, stream, args, lt);
   } else {
-    hipLaunchKernelGGL((FrHexStageKernel<Q, R, false>), grid, block, 0, stream, args, lt);
+    const dim3 grid((unsigned)blocks), block(Shape<Q>::kThreads);
+    if (args.curved) hipLaunchKernelGGL((FrHexStageKernel<Q, R, true>), grid, block, 0, stream, args, lt);
+    else hipLaunchKernelGGL((FrHexStageKernel<Q, R, false>), grid, block, 0, stream, args, lt);
   }
   return hipGetLastError();
 }
@@ -894,7 +895,7 @@ int FrHexStageTileCells(int q, bool mixed) {
   switch (q) {
   case 2: return Shape<2>::kCells;
   case 3: return Shape<3>::kCells;
-  case 4: return Shape<4>::kCells;
+  case 4: return kCellTile;
   case 5: return Shape<5>::kCells;
   case 6: return Shape<6>::kCells;
   default: return 0;
@@ -904,20 +905,21 @@ int FrHexStageTileCells(int q, bool mixed) {
 int FrHexTileLdsBytes(int q, int tile, bool mixed) {
   if (mixed) return FrMixedTileLdsBytes(q, tile);
   if (q < 2 || q > 4 || tile < 0 || tile > 2) return 0;
-  return (int)sizeof(double) * (q == 2 ? Shape<2>::kLdsDoubles : (q == 3 ? Shape<3>::kLdsDoubles : Shape<4>::kLdsDoubles));
+  return (int)sizeof(double) * (q == 2 ? Shape<2>::kLdsDoubles
+                                       : (q == 3 ? Shape<3>::kLdsDoubles : kBatchWaves * CellShape<1>::kLdsDoubles));
 }
 
 int FrHexTileCells(int q, int tile, bool mixed) {
   if (mixed) return FrMixedTileCells(q, tile);
   if (q < 2 || q > 4 || tile < 0 || tile > 2) return 0;
-  return FrHexStageTileCells(q, false) * TileBlocks(tile);
+  return BatchCells(q) * TileBlocks(tile);
 }
 
 hipError_t LaunchFrHexBatch(int riemann, bool mixed, const FrHexBatchArgs &args, int n_workgroups,
                             hipStream_t stream) {
   if (mixed) return LaunchFrMixedBatch(riemann, args, n_workgroups, stream);
   if (args.n_groups < 1 || args.n_groups > kMaxBatchGroups || n_workgroups < 1) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)n_workgroups), block(Shape<4>::kThreads);
+  const dim3 grid((unsigned)n_workgroups), block(kBatchThreads);
   const size_t lds = (size_t)args.max_tile_lds;
   switch (riemann) {
   case kExact: hipLaunchKernelGGL(FrHexBatchKernel<kExact>, grid, block, lds, stream, args); break;
@@ -931,11 +933,10 @@ hipError_t LaunchFrHexBatch(int riemann, bool mixed, const FrHexBatchArgs &args,
 int FrHexBatchResidentWorkgroups(int riemann, bool mixed, int lds_bytes) {
   int per_cu = 0;
   hipError_t e = hipErrorInvalidValue;
-  constexpr int kThreads = Shape<4>::kThreads;
   if (mixed) e = FrMixedBatchResident(riemann, lds_bytes, &per_cu);
-  else if (riemann == kExact) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kExact>, kThreads, lds_bytes);
-  else if (riemann == kHllc) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kHllc>, kThreads, lds_bytes);
-  else if (riemann == kRoe) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kRoe>, kThreads, lds_bytes);
+  else if (riemann == kExact) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kExact>, kBatchThreads, lds_bytes);
+  else if (riemann == kHllc) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kHllc>, kBatchThreads, lds_bytes);
+  else if (riemann == kRoe) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, FrHexBatchKernel<kRoe>, kBatchThreads, lds_bytes);
   int dev = 0, cus = 0;
   if (e != hipSuccess || hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
