@@ -4,7 +4,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -28,10 +28,10 @@ class Crew {
  public:
   template <class Work>
   Crew(int n, Work const &work) {
-    threads_.reserve(n);
     try {
+      threads_.reserve(n);
       for (int i = 0; i < n; ++i) threads_.emplace_back(work);
-    } catch (std::system_error const &) {  // fewer threads than wished for
+    } catch (std::exception const &) {  // no threads or no memory left: fewer than wished for
     }
   }
   ~Crew() {

@@ -1,0 +1,117 @@
+// host/column_copy.cpp on the stand-in runtime (stand_in/hip/hip_runtime.h): what is
+// put in comes out at the sizes where the copy changes form, and failures of the
+// host leave the caller with a copy or an error, never with an abort.
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <new>
+#include <vector>
+
+#include "../../pvcriemannsolvers_amd/csrc/host/column_copy.hpp"
+
+// operator new of this program fails once after `allocations_left` more calls
+static std::atomic<long> allocations_left{ -1 };
+void *operator new(size_t n) {
+  if (allocations_left.load() >= 0 && allocations_left.fetch_sub(1) == 0) throw std::bad_alloc();
+  if (void *p = std::malloc(n)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
+namespace mcfd {
+std::string &LastError() {
+  thread_local std::string e;
+  return e;
+}
+}  // namespace mcfd
+
+namespace {
+
+constexpr size_t kMiB = size_t(1) << 20;
+
+std::vector<char> Pattern(size_t n, unsigned seed) {
+  std::vector<char> v(n);
+  for (size_t i = 0; i < n; ++i) v[i] = (char)((i * 2654435761u + seed) >> 13);
+  return v;
+}
+
+struct Handle {
+  mcfd::ColumnCopy copy;
+  StandInStream stream;
+  std::vector<char> device;
+  explicit Handle(size_t n) : device(n) { copy.Reserve(n); }
+  ~Handle() { (void)hipStreamSynchronize(&stream); }
+  bool In(const std::vector<char> &host) {
+    std::lock_guard<std::mutex> lock(copy.mutex);
+    copy.ToDevice(device.data(), host.data(), host.size(), &stream);
+    (void)hipStreamSynchronize(&stream);
+    return std::memcmp(device.data(), host.data(), host.size()) == 0;
+  }
+  bool Out() {
+    std::vector<char> host(device.size(), 0);
+    std::lock_guard<std::mutex> lock(copy.mutex);
+    copy.ToHost(host.data(), device.data(), host.size(), &stream);
+    return host == device;
+  }
+};
+
+const size_t kSizes[] = { 8, 2 * kMiB - 8, 2 * kMiB, 2 * kMiB + 8, 5 * kMiB + 24, 16 * kMiB, 17 * kMiB + 40,
+                          32 * kMiB - 8, 32 * kMiB, 32 * kMiB + 8, 67 * kMiB + 16 };
+
+bool RoundTrips() {
+  for (size_t n : kSizes) {
+    Handle h(n);
+    for (unsigned seed = 0; seed < 2; ++seed)
+      if (!h.In(Pattern(n, seed)) || !h.Out()) return false;
+  }
+  return true;
+}
+
+// Memory runs out while the copy's threads are started, at every allocation of it.
+bool NoMemoryForThreads() {
+  for (size_t n : { 5 * kMiB, 40 * kMiB }) {
+    Handle h(n);
+    const std::vector<char> host = Pattern(n, 3);
+    std::vector<char> back(n);
+    for (long k = 0; k < 12; ++k) {
+      std::lock_guard<std::mutex> lock(h.copy.mutex);
+      bool in = false, out = false;
+      allocations_left = k;
+      try {
+        h.copy.ToDevice(h.device.data(), host.data(), n, &h.stream);
+        in = true;
+      } catch (std::bad_alloc const &) {
+      }
+      allocations_left = -1;
+      (void)hipStreamSynchronize(&h.stream);
+      if (in && h.device != host) return false;
+      h.device = host;
+      allocations_left = k;
+      try {
+        h.copy.ToHost(back.data(), h.device.data(), n, &h.stream);
+        out = true;
+      } catch (std::bad_alloc const &) {
+      }
+      allocations_left = -1;
+      if (out && back != host) return false;
+      back.assign(n, 0);
+    }
+  }
+  return true;
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const struct { const char *name; bool (*run)(); } tests[] = { { "round_trips", RoundTrips },
+                                                                { "no_memory_for_threads", NoMemoryForThreads } };
+  for (auto const &t : tests) {
+    if (argc > 1 && std::strcmp(argv[1], t.name) != 0) continue;
+    const bool ok = t.run();
+    std::printf("%s %s\n", ok ? "PASS" : "FAIL", t.name);
+    if (!ok) return 1;
+  }
+  return 0;
+}
