@@ -84,12 +84,20 @@ ColumnCopy::~ColumnCopy() {
     if (e) (void)hipEventDestroy(e);
 }
 
+void ColumnCopy::Settle() {
+  if (!busy_) return;
+  Check(hipStreamSynchronize(busy_), "column copy sync");
+  busy_ = nullptr;
+}
+
 void ColumnCopy::ToHost(void *host, const void *device, size_t bytes, hipStream_t stream) {
   if (!Ring(bytes, kLeastToHost)) {
     Check(hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, stream), "column to host");
     Check(hipStreamSynchronize(stream), "column to host sync");
     return;
   }
+  Settle();
+  busy_ = stream;
   const size_t chunk = Chunk(bytes);
   const int64_t n = (int64_t)((bytes + chunk - 1) / chunk);
   auto size = [&](int64_t c) { return std::min(chunk, bytes - size_t(c) * chunk); };
@@ -139,6 +147,7 @@ void ColumnCopy::ToHost(void *host, const void *device, size_t bytes, hipStream_
       Check(hipStreamSynchronize(stream), "column to host sync");
     }
   }
+  busy_ = nullptr;
 }
 
 void ColumnCopy::ToDevice(void *device, const void *host, size_t bytes, hipStream_t stream) {
@@ -146,6 +155,8 @@ void ColumnCopy::ToDevice(void *device, const void *host, size_t bytes, hipStrea
     Check(hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, stream), "column to device");
     return;
   }
+  Settle();
+  busy_ = stream;
   const size_t chunk = Chunk(bytes);
   const int64_t n = (int64_t)((bytes + chunk - 1) / chunk);
   auto size = [&](int64_t c) { return std::min(chunk, bytes - size_t(c) * chunk); };

@@ -37,10 +37,14 @@ class ColumnCopy {
   static constexpr int kThreads = 4;
   bool Ring(size_t bytes, size_t least) const;
   static size_t Chunk(size_t bytes);
+  // Waits for what may still read or fill the slots: a call that failed leaves its
+  // copies in flight, and a copy to the device those that its caller waits for.
+  void Settle();
   char *pinned_ = nullptr;
   size_t slot_ = 0;  // bytes of one
   size_t most_ = 0;  // chunks of a column: the slots where the ring is not full, else any number
   hipEvent_t events_[kSlots] = {};
+  hipStream_t busy_ = nullptr;  // of those copies
 };
 
 }  // namespace mcfd

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../pvcriemannsolvers_amd/csrc/host/column_copy.hpp"
+#include "../../pvcriemannsolvers_amd/csrc/host/common.hpp"
 
 // operator new of this program fails once after `allocations_left` more calls
 static std::atomic<long> allocations_left{ -1 };
@@ -102,11 +103,38 @@ bool NoMemoryForThreads() {
   return true;
 }
 
+// A copy that fails on its way leaves copies to and from the slots in flight; what
+// follows it on the same handle is whole all the same.
+bool CopiesAfterAFailure() {
+  for (size_t n : { 7 * kMiB, 40 * kMiB, 70 * kMiB }) {
+    Handle h(n);
+    for (long k : { 0, 1, 3, 9, 20 }) {
+      for (bool in : { false, true }) {
+        std::vector<char> host = Pattern(n, (unsigned)k), other = Pattern(n, (unsigned)k + 1);
+        Runtime().copies_until_failure = k;
+        bool failed = false;
+        try {
+          std::lock_guard<std::mutex> lock(h.copy.mutex);
+          if (in) h.copy.ToDevice(h.device.data(), other.data(), n, &h.stream);
+          else h.copy.ToHost(other.data(), h.device.data(), n, &h.stream);
+        } catch (mcfd::Failure const &) {
+          failed = true;
+        }
+        if (failed != (Runtime().copies_until_failure == -1)) return false;
+        Runtime().copies_until_failure = -1;
+        if (!h.In(host) || !h.Out()) return false;
+      }
+    }
+  }
+  return true;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
   const struct { const char *name; bool (*run)(); } tests[] = { { "round_trips", RoundTrips },
-                                                                { "no_memory_for_threads", NoMemoryForThreads } };
+                                                                { "no_memory_for_threads", NoMemoryForThreads },
+                                                                { "copies_after_a_failure", CopiesAfterAFailure } };
   for (auto const &t : tests) {
     if (argc > 1 && std::strcmp(argv[1], t.name) != 0) continue;
     const bool ok = t.run();
