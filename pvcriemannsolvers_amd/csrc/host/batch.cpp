@@ -256,7 +256,7 @@ int mcfd_batch_set_solution_column(mcfd_batch *b, int32_t c, const double *colum
     const auto &ref = b->cases[c];
     std::lock_guard<std::mutex> lock(b->copy.mutex);
     b->groups[ref.group]->SetColumn(column, ref.first_cell, ref.n_cells, &b->copy, b->stream);
-    Check(hipStreamSynchronize(b->stream), "sync");
+    b->copy.Wait(b->stream);
   });
 }
 

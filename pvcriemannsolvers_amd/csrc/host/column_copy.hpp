@@ -5,7 +5,11 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <cstdint>
+#include <memory>
 #include <mutex>
+#include <thread>
+#include <vector>
 
 namespace mcfd {
 
@@ -13,38 +17,63 @@ namespace mcfd {
 // drain the slots while several host threads copy between them and the caller's
 // memory.  The caller's side bounds a direct copy: pages that numpy.empty has
 // just handed out are zeroed as the copy touches them, by one thread.  The
-// threads live for one call, so nothing runs between calls; more than four gain
-// nothing.  One copy at a time: callers hold `mutex` over it, over the launches
-// that fill or read the same device buffer, and until the stream is drained.
+// threads live for one call and more than four gain nothing.  The caller waits
+// for none that has not begun: where the processors are busy (another library's
+// threads spinning) that takes milliseconds, and it copies in their place.  One
+// copy at a time: callers hold `mutex` over it, over the launches that fill or
+// read the same device buffer, and until the stream is drained.
+//
+// The rings belong to the process, as many as there are users, up to four, so that
+// pinned memory is bounded and a new handle beside others finds pages that are
+// mapped already: a ring's own cost its first copy 0.4 ms per MiB and thread.  The
+// last user gives them back.  A new handle's first 4.4 MB to the host, us, with a
+// ring per handle / the process's, on processors that another library's threads keep
+// busy: 1800 to 4600 / 210 to 240 (direct 290; the first handle's 1100).
 class ColumnCopy {
  public:
   ColumnCopy() = default;
   ColumnCopy(const ColumnCopy &) = delete;
   ColumnCopy &operator=(const ColumnCopy &) = delete;
   ~ColumnCopy();
-  // Prepares the ring for columns of up to `bytes`; without it (or where
-  // the memory cannot be had) copies are direct.
+  // Prepares for columns of up to `bytes`; without it (or where the memory
+  // cannot be had, or all rings are lent) copies are direct.
   void Reserve(size_t bytes);
   // Returns when the column is in `host`.
   void ToHost(void *host, const void *device, size_t bytes, hipStream_t stream);
-  // The caller synchronises the stream.
+  // The caller waits with Wait().
   void ToDevice(void *device, const void *host, size_t bytes, hipStream_t stream);
+  // Waits for the stream.
+  void Wait(hipStream_t stream);
 
   std::mutex mutex;
 
- private:
+  struct Ring {  // of kSlots slots at most
+    char *pinned;
+    size_t bytes;
+  };
   static constexpr int kSlots = 16;
+
+ private:
   static constexpr int kThreads = 4;
-  bool Ring(size_t bytes, size_t least) const;
-  static size_t Chunk(size_t bytes);
+  struct Job;
+  struct Late {  // a thread that had not begun when its call returned
+    std::thread thread;
+    std::shared_ptr<Job> job;
+    int index;
+  };
+  // A ring for a column of `bytes`, or false for a direct copy.
+  bool Take(size_t bytes, size_t least, hipStream_t stream);
+  void GiveBack();
   // Waits for what may still read or fill the slots: a call that failed leaves its
   // copies in flight, and a copy to the device those that its caller waits for.
   void Settle();
-  char *pinned_ = nullptr;
-  size_t slot_ = 0;  // bytes of one
-  size_t most_ = 0;  // chunks of a column: the slots where the ring is not full, else any number
+  class Crew;
+
+  bool user_ = false;  // of the rings
+  Ring *ring_ = nullptr;
   hipEvent_t events_[kSlots] = {};
-  hipStream_t busy_ = nullptr;  // of those copies
+  hipStream_t busy_ = nullptr;  // of the copies in flight
+  std::vector<Late> late_;
 };
 
 }  // namespace mcfd

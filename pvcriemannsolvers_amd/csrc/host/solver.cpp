@@ -180,7 +180,7 @@ int mcfd_set_solution_column(mcfd_solver *h, const double *column) {
     h->dt_fresh = false;
     h->SetColumn(column);
     if (h->dg) h->modal.SolutionChanged(h->stream);
-    Check(hipStreamSynchronize(h->stream), "set solution sync");
+    h->copy.Wait(h->stream);
   });
 }
 
@@ -192,7 +192,7 @@ int mcfd_restore_solution_column(mcfd_solver *h, const double *column) {
     h->dt_fresh = false;
     h->SetColumn(column);
     if (h->dg) h->modal.SolutionChanged(h->stream, /*limit=*/false);
-    Check(hipStreamSynchronize(h->stream), "restore solution sync");
+    h->copy.Wait(h->stream);
   });
 }
 
