@@ -53,3 +53,27 @@ def test_batch_columns_of_different_sizes():
     for i, u in enumerate(columns):
         np.testing.assert_array_equal(batch.get_solution_column(i), u)
     batch.close()
+
+
+def test_reads_from_two_threads_complete():
+    """Solution and residual, which pass through one buffer, read over and over by
+    two threads: every read returns, and returns its own column."""
+    g = spatial.FiniteElement(meshgen.box_hex(19, 19, 19), degree=3, riemann="hllc", bcs=[("inviscid_wall", None)] * 6)
+    rng = np.random.default_rng(7)
+    u = 1 + 1e-2 * rng.random((g.column_size // 5, 5))
+    u[:, 4] += 9
+    g.set_solution_column(u.reshape(-1))
+    want = {g.get_solution_column: u.reshape(-1), g.get_residual_column: g.get_residual_column()}
+    seen = {get: [] for get in want}
+
+    def read(get):
+        for _ in range(8):
+            seen[get].append(np.array_equal(get(), want[get]))
+
+    threads = [threading.Thread(target=read, args=(get,)) for get in want]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(seen[get] == [True] * 8 for get in want)
+    g.close()
