@@ -268,10 +268,7 @@ MCFD_HD State NearVacuum(State const &l, State const &r) {  // exact.hpp:293-320
 // passive tangential velocities take the side given by its sign
 // (exact.hpp:49-57), also in the vacuum branches, which do not update it.
 // `star_positive` carries that sign in and out; a fresh solver holds 0.
-//
-// ExactState is the state on the face (density, normal velocity, pressure;
-// the passive velocities are left at 0), ExactFlux its flux.
-MCFD_HD State ExactState(State const &l, State const &r, bool &star_positive) {
+MCFD_HD State ExactFlux(State const &l, State const &r, bool &star_positive) {
   bool sp = star_positive;
   State res;
   for (int i = 0; i < 5; ++i) res.v[i] = 0;
@@ -326,13 +323,9 @@ MCFD_HD State ExactState(State const &l, State const &r, bool &star_positive) {
       res = NearVacuum(l, r);
     }
   }
+  res.v[2] = sp ? l.v[2] : r.v[2];
+  res.v[3] = sp ? l.v[3] : r.v[3];
   star_positive = sp;
-  return res;
-}
-MCFD_HD State ExactFlux(State const &l, State const &r, bool &star_positive) {
-  State res = ExactState(l, r, star_positive);
-  res.v[2] = star_positive ? l.v[2] : r.v[2];
-  res.v[3] = star_positive ? l.v[3] : r.v[3];
   return NormalFlux(res);
 }
 

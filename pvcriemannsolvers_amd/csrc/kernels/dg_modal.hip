@@ -46,9 +46,9 @@
 namespace mcfd {
 namespace {
 
-// LDS record of one volume task: the weighted flux matrix as F[d][k] (15),
-// a pad, then the point's offset y (3) from kSlotY.  A face task: the
-// weighted flux (5), then y (3).
+// LDS record of one volume task: the weighted flux matrix as F[d][k] (15), then
+// the point's offset y (3) from kSlotY.  A face task: the weighted flux (5), then y
+// (3).  One double more makes either odd, against bank conflicts.
 constexpr int kSlot = 19;
 constexpr int kSlotY = 15;
 constexpr int kFaceSlot = 9;
@@ -144,18 +144,16 @@ __device__ __forceinline__ double DppMove(double v) {
   return __hiloint2double(hi, lo);
 }
 
-// Sum over each aligned group of NPART lanes (NPART = 1, 2, 4, 8 or 16), by
-// a butterfly: lane ^ 1 (quad_perm 1,0,3,2), lane ^ 2 (quad_perm 2,3,0,1),
-// the other quad of the half row (row_half_mirror), the other half of the
-// row (row_ror 8).  Every lane of a group ends with the same bits, since each
-// step adds two values whose order does not matter.  All lanes of the
-// wavefront must execute it.
+// Sum over each aligned group of NPART lanes (NPART = 1, 2, 4 or 8), by a
+// butterfly: lane ^ 1 (quad_perm 1,0,3,2), lane ^ 2 (quad_perm 2,3,0,1), the
+// other quad of the half row (row_half_mirror).  Every lane of a group ends with
+// the same bits, since each step adds two values whose order does not matter.  All
+// lanes of the wavefront must execute it.
 template <int NPART>
 __device__ __forceinline__ double GroupSum(double v) {
   if constexpr (NPART >= 2) v += DppMove<0xB1>(v);
   if constexpr (NPART >= 4) v += DppMove<0x4E>(v);
   if constexpr (NPART >= 8) v += DppMove<0x141>(v);
-  if constexpr (NPART >= 16) v += DppMove<0x128>(v);
   return v;
 }
 

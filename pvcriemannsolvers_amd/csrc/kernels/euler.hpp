@@ -237,8 +237,9 @@ __device__ __forceinline__ State FastInsideFan(double rho0, double a0, double gr
   s.v[4] = a2 * s.v[0] * (1 / kGamma);
   return s;
 }
-// ExactState of euler_core.hpp (the same branches, starting point, iteration
-// and stopping rule) on the functions above.
+// The state on the face (density, normal velocity, pressure; passive velocities 0),
+// by ExactFlux's branches, starting point, iteration and stopping rule
+// (euler_core.hpp) on the functions above.
 __device__ __forceinline__ State FastExactState(State const &l, State const &r, bool &star_positive) {
   State res;
 #pragma unroll
