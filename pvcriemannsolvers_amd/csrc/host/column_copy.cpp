@@ -251,8 +251,9 @@ void ColumnCopy::ToHost(void *host, const void *device, size_t bytes, hipStream_
   issue();  // the first copies run while the threads start
   {
     Crew crew(job, &late_);
+    const int64_t first = std::min<int64_t>(job->n, kSlots);  // till these are filled, threads may still begin
     while (job->copied.load(std::memory_order_acquire) < job->n) {
-      if (filled < issued && !(crew.Short() && job->Step())) {
+      if (filled < issued && !(filled >= first && crew.Short() && job->Step())) {
         Check(hipEventSynchronize(events_[filled % kSlots]), "column to host sync");
         job->limit.store(++filled, std::memory_order_release);
       } else if (filled == issued) {  // all slots wait to be emptied, or it is the column's end

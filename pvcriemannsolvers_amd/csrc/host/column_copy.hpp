@@ -19,7 +19,9 @@ namespace mcfd {
 // just handed out are zeroed as the copy touches them, by one thread.  The
 // threads live for one call and more than four gain nothing.  The caller waits
 // for none that has not begun: where the processors are busy (another library's
-// threads spinning) that takes milliseconds, and it copies in their place.  One
+// threads spinning) that takes milliseconds.  It copies in their place, but only from
+// the first ring's end on: till then its own part, the next transfers, comes first
+// (48 columns of 0.5 to 10 MB 1 ms a pass slower else).  One
 // copy at a time: callers hold `mutex` over it, over the launches that fill or
 // read the same device buffer, and until the stream is drained.
 //
@@ -27,8 +29,9 @@ namespace mcfd {
 // pinned memory is bounded and a new handle beside others finds pages that are
 // mapped already: a ring's own cost its first copy 0.4 ms per MiB and thread.  The
 // last user gives them back.  A new handle's first 4.4 MB to the host, us, with a
-// ring per handle / the process's, on processors that another library's threads keep
-// busy: 1800 to 4600 / 210 to 240 (direct 290; the first handle's 1100).
+// ring per handle / the process's: 770 to 960 / 240 to 280, and on processors that
+// another library's threads keep busy 1060 to 6000 / 200 to 330, 1 of 8 at 4000,
+// where a thread was stopped at its work (direct 290; a process's first handle 870).
 class ColumnCopy {
  public:
   ColumnCopy() = default;
