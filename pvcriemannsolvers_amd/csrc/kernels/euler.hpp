@@ -16,7 +16,8 @@ namespace mcfd {
 // Used by the throughput kernels in place of IEEE division (a ~10
 // instruction sequence on CDNA); both cells of a face run the same code, so
 // the face flux stays bit-identical on the two sides.  NaN for zeros and
-// infinities, of which the steps know nothing.
+// infinities, of which the steps know nothing: for arguments that are neither, or
+// where a NaN, or the zeroing rule's values, come of it either way.
 __device__ __forceinline__ double FiniteRcp(double x) {
   double r = __builtin_amdgcn_rcp(x);
   double e = __fma_rn(-x, r, 1.0);
@@ -25,8 +26,7 @@ __device__ __forceinline__ double FiniteRcp(double x) {
   return __fma_rn(r, e, r);
 }
 // The same with zeros and infinities as the divide has them, one instruction more
-// (in the nodes' fluxes too it would cost 0.3 % of a pass, and change nothing: they
-// replace what a zero density gives).
+// (everywhere, 0.3 to 0.6 % of a pass of 64^3 p3, 1 to 2 % of a small one's chain).
 __device__ __forceinline__ double FastRcp(double x) { return __builtin_amdgcn_div_fixup(FiniteRcp(x), x, 1.0); }
 
 // The smallest of the positive `value`s in *bits (the bits of positive doubles
@@ -75,7 +75,7 @@ struct FaceTrace { double rho, inv, v[3], p, e, un; };
 __device__ __forceinline__ FaceTrace PlainTrace(State const &c, const double *n, bool *plain) {
   FaceTrace t;
   t.rho = c.v[0];
-  t.inv = FastRcp(t.rho);
+  t.inv = FiniteRcp(t.rho);
 #pragma unroll
   for (int d = 0; d < 3; ++d) t.v[d] = c.v[1 + d] * t.inv;
   t.e = c.v[4];
@@ -86,7 +86,10 @@ __device__ __forceinline__ FaceTrace PlainTrace(State const &c, const double *n,
   return t;
 }
 // types.hpp:195-202: all zero where rho < 0, E < 0 or p < 0; momenta and E kept
-// as velocity and pressure where rho == 0.
+// as velocity and pressure where rho == 0.  kStill (HLLC): such a state with pressure
+// takes 1 / rho = 0, which gives it the wave speed u of a side whose a is 0 and whose
+// q is finite.
+template <bool kStill = false>
 __device__ __forceinline__ void ApplyZeroRule(State const &c, const double *n, FaceTrace *t) {
   const bool bad = c.v[0] < 0 || c.v[4] < 0;
   const bool vacuum = !bad && c.v[0] == 0;
@@ -96,7 +99,7 @@ __device__ __forceinline__ void ApplyZeroRule(State const &c, const double *n, F
   t->p = zero ? 0.0 : (vacuum ? c.v[4] : t->p);
   t->e = zero ? 0.0 : (vacuum ? c.v[4] * (1 / kGm1) : t->e);
   t->rho = zero ? 0.0 : t->rho;
-  if (zero || vacuum) t->inv = FastRcp(t->rho);
+  if (zero || vacuum) t->inv = kStill && t->p > 0 ? 0.0 : FastRcp(t->rho);
   t->un = t->v[0] * n[0] + t->v[1] * n[1] + t->v[2] * n[2];
 }
 __device__ __forceinline__ FaceTrace TraceOf(State const &c, const double *n) {
@@ -122,7 +125,7 @@ __device__ __forceinline__ State TraceFlux(FaceTrace const &t, const double *n) 
 __device__ __forceinline__ State FastRoe(FaceTrace const &l, FaceTrace const &r, const double *n) {
   const double hl = (l.e + l.p), hr = (r.e + r.p);  // rho times total enthalpy
   const double ratio = FastSqrt(r.rho * l.inv);
-  const double wr = ratio * FastRcp(1.0 + ratio);
+  const double wr = ratio * FiniteRcp(1.0 + ratio);
   const double rho = l.rho * ratio;
   double dv[3], v[3];
 #pragma unroll
@@ -134,7 +137,7 @@ __device__ __forceinline__ State FastRoe(FaceTrace const &l, FaceTrace const &r,
   const double h0l = hl * l.inv, h = h0l + wr * (hr * r.inv - h0l);
   const double ke = 0.5 * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
   const double aa = kGm1 * (h - ke);
-  const double a = FastSqrt(aa), inv_aa = FastRcp(aa);
+  const double a = FastSqrt(aa), inv_aa = FiniteRcp(aa);
   const double rad = rho * a * dun;
   const double s1 = 0.25 * (dp - rad) * inv_aa * fabs(un - a);
   const double s5 = 0.25 * (dp + rad) * inv_aa * fabs(un + a);
@@ -153,19 +156,18 @@ __device__ __forceinline__ State FastRoe(FaceTrace const &l, FaceTrace const &r,
 }
 
 // HLLC flux (hllc.hpp:30-109): wave speeds u -+ a q from one square root each
-// (a q = sqrt(a^2 + c (p* - p) / rho) needs no division by p; a side without
-// density but with pressure has a = 0 and a finite q, so a q is 0 there, not the
-// formula's infinity), the star state formed once, for the side the contact selects.
+// (a q = sqrt(a^2 + c (p* - p) / rho) needs no division by p; kStill of the zeroing
+// rule sees to a side without density), the star state formed once, for the side the
+// contact selects.
 __device__ __forceinline__ State FastHllc(FaceTrace const &l, FaceTrace const &r, const double *n) {
   const double al = l.rho > 0 && l.p > 0 ? FastSqrt(kGamma * l.p * l.inv) : 0.0;
   const double ar = r.rho > 0 && r.p > 0 ? FastSqrt(kGamma * r.p * r.inv) : 0.0;
   const double p_est = fmax(0.0, 0.5 * (l.p + r.p - (r.un - l.un) * (0.25 * (l.rho + r.rho) * (al + ar))));
-  const bool still_l = p_est <= l.p || (l.p > 0 && !(l.rho > 0)), still_r = p_est <= r.p || (r.p > 0 && !(r.rho > 0));
-  const double aql = still_l ? al : FastSqrt((kGamma * l.p + (kGp1 / 2) * (p_est - l.p)) * l.inv);
-  const double aqr = still_r ? ar : FastSqrt((kGamma * r.p + (kGp1 / 2) * (p_est - r.p)) * r.inv);
+  const double aql = p_est > l.p ? FastSqrt((kGamma * l.p + (kGp1 / 2) * (p_est - l.p)) * l.inv) : al;
+  const double aqr = p_est > r.p ? FastSqrt((kGamma * r.p + (kGp1 / 2) * (p_est - r.p)) * r.inv) : ar;
   const double wl = l.un - aql, wr = r.un + aqr;
   const double ml = l.rho * (wl - l.un), mr = r.rho * (wr - r.un);
-  const double ws = (r.p - l.p + ml * l.un - mr * r.un) * FastRcp(ml - mr);
+  const double ws = (r.p - l.p + ml * l.un - mr * r.un) * FiniteRcp(ml - mr);
   const bool super_l = 0.0 <= wl, super_r = !super_l && wr <= 0.0;
   const bool left = super_l || (!super_r && 0.0 <= ws);
   FaceTrace k;
@@ -197,7 +199,7 @@ __device__ __forceinline__ double SeventhRoot(double x) {
   const double m = __builtin_amdgcn_ldexp(__builtin_amdgcn_frexp_mant(x), e - 7 * q);  // in [1/2, 64)
   const double y = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)m) * (1.0f / 7));
   const double y2 = y * y, y3 = y2 * y, y7 = y3 * y3 * y;
-  const double root = __fma_rn(y * (m - y7), FastRcp(__fma_rn(4.0, y7, 3.0 * m)), y);
+  const double root = __fma_rn(y * (m - y7), FiniteRcp(__fma_rn(4.0, y7, 3.0 * m)), y);
   return __builtin_amdgcn_ldexp(root, q);
 }
 
@@ -330,8 +332,8 @@ __device__ __forceinline__ State FaceFlux(const double *n, State const &cl, Stat
   bool plain = true;
   FaceTrace l = PlainTrace(cl, n, &plain), r = PlainTrace(cr, n, &plain);
   if (!__all(plain)) {
-    ApplyZeroRule(cl, n, &l);
-    ApplyZeroRule(cr, n, &r);
+    ApplyZeroRule<kRiemann == kHllc>(cl, n, &l);
+    ApplyZeroRule<kRiemann == kHllc>(cr, n, &r);
   }
   return TraceUpwind<kRiemann>(l, r, n, star);
 }
