@@ -156,7 +156,7 @@ void FrHexGroup::BuildCurved(const mcfd_scheme_desc &) {
     corner0[c] = { xv[0], xv[1], xv[2] };
   }
   if ((int64_t)conn.faces.size() >= (int64_t(1) << 24))
-    throw Failure{ MCFD_ENOTSUP, "too many faces for the per-point normals of a trilinear mesh" };
+    throw Failure{ MCFD_ENOTSUP, "a trilinear mesh of 2^24 faces or more" };
   BuildFaceRecords([&](size_t fi, double sign) {
     const auto &face = conn.faces[fi];
     for (int i = 0; i < q; ++i)

@@ -1,10 +1,10 @@
 // One mesh discretised by nodal FR on hexahedra: host connectivity, line
-// tables, geometry/frame records and the device arrays the stage kernel
+// tables, geometry and face records and the device arrays the stage kernel
 // reads.  A solver handle owns one group; a batch owns one per degree.
-// Meshes of affine cells keep one deduplicated geometry record per cell and
-// one frame per face; a mesh with a trilinear cell ("curved") keeps the
-// metric of every solution point, the signed scale of every cell flux point
-// and the frame of every face flux point.
+// Meshes of affine cells keep one deduplicated geometry record per cell and one
+// deduplicated unit normal per face (the mixed form: a frame); a mesh with a
+// trilinear cell ("curved") keeps the metric of every solution point, and the unit
+// normal and scale of every cell flux point.
 #ifndef MINICFD_HOST_FR_GROUP_HPP_
 #define MINICFD_HOST_FR_GROUP_HPP_
 

@@ -22,8 +22,8 @@
 // times an approximate flux, is evaluated once per face point on large meshes
 // (DgFacePass), by DgFaceFluxKernel into fhat [face][point][5].
 //
-// What bounds it: no unit is full (P = 2 tetrahedra: FP64 issue 45 %, vector memory
-// 59 %, LDS 37 %, HBM at 56 % of its copy rate); each workgroup passes through three
+// What bounds it: no unit is full (P = 2 tetrahedra: vector issue 43 %, vector memory
+// 47 %, LDS 35 %, 2.8 of the 4.9 TB/s of a copy); each workgroup passes through three
 // dependent phases, and 4 to 5 of them fit in a CU's LDS.  Moments by one
 // wavefront with 60 lanes in use take 600 instructions where eight lanes per
 // (cell, component) in all four took 4 x 430.  us per pass, against one launch
@@ -31,11 +31,12 @@
 // 146k P = 2 tetrahedra (Roe) 256 -> 195, the four-quadrant problem's 221k (HLLC,
 // with the limiter) 507 -> 417, 750 tetrahedra 15.5 -> 10.2, 64k P = 2 hexahedra
 // 208 -> 157, 83k P = 1 tetrahedra 83 -> 68; the same cell pass after a face
-// pass: 227, 467, 13.6, 179 and 78.  With the exact solver, the Sod tube's 3840
-// tetrahedra 41 -> 14, 24.6k 106 -> 52 (most of it the solver itself).  Measured and no better: the neighbours'
-// coefficients loaded once per face and handed round through LDS (a third of the
-// vector memory work, 200), 5 wavefronts per SIMD (200), moments on two
-// wavefronts (212), 3 cells per workgroup (215).
+// pass: 227, 467, 13.6, 179 and 78.  With the exact solver, the Sod tube's 640
+// hexahedra 41 -> 14, 3840 tetrahedra 33 -> 19, 24.6k 102 -> 49 (most of it the
+// solver itself).  Measured and no better: the neighbours' coefficients loaded once
+// per face and handed round through LDS (a third of the vector memory work, 200),
+// 5 wavefronts per SIMD (200), moments on two wavefronts (212), 3 cells per
+// workgroup (215).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -208,7 +208,7 @@ __device__ __forceinline__ double SeventhRoot(double x) {
 // gamma = 1.4 the rarefaction's powers are z - 1 and z^-6 of the one seventh root z
 // of pa / p, function and slope come from one evaluation, and the state inside a
 // fan from rho (a / a0)^5.  us per stage: FR 24^3 p3 217 -> 63, 32^3 p2 330 -> 88; DG
-// on the 3840 tetrahedra of a Sod tube 29 -> 14 (face and cell pass -> one).
+// on the 640 hexahedra of a Sod tube 41 -> 14 (face and cell pass -> one, too).
 //
 // One side's pressure function (exact.hpp:153-200) and its derivative at pa.
 struct FastWave {
