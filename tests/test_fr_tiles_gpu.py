@@ -139,3 +139,26 @@ def test_folded_time_step_of_an_odd_last_cell(cell):
     expect = o.time_step(state, 0.1)
     assert abs(fused - expect) <= 1e-12 * expect
     g.close()
+
+
+@pytest.mark.parametrize("riemann", ["hllc", "exact"])
+@pytest.mark.parametrize("degree,size", [(3, (17, 17, 15)), (3, (6, 5, 4)), (2, (6, 5, 4))])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_bad_values_stay_local_with_every_solver(riemann, degree, size, value):
+    """As test_bad_values_reach_face_neighbours_only, whose solver is Roe's."""
+    mesh = meshgen.box_hex(*size, periodic=(True,) * 3, shuffle_seed=3)
+    g = spatial.FiniteElement(mesh, degree=degree, riemann=riemann)
+    n = len(mesh["cells"])
+    u = density_wave(g.sample_points(), seed=2).reshape(n, -1)
+    g.set_solution_column(u.reshape(-1))
+    want = g.get_residual_column().reshape(n, -1)
+    faces = g.faces()
+    cell = n - 1
+    u[cell, 0] = value
+    g.set_solution_column(u.reshape(-1))
+    got = g.get_residual_column().reshape(n, -1)
+    near = {cell} | {int(a + b - cell) for a, b in zip(faces["holder"], faces["sharer"]) if cell in (a, b)}
+    far = np.setdiff1d(np.arange(n), sorted(near))
+    np.testing.assert_array_equal(got[far], want[far])
+    assert not np.isfinite(got[cell]).all()
+    g.close()
